@@ -278,7 +278,8 @@ static dim3 cell_grid(int n) { return dim3((n + 63) / 64, (n + 3) / 4); }
 // for the source src read as f = -src.  Returns the sweeps taken.
 // With warm start the solve starts from psi[0] as the caller left it, else from 0.
 static int solve_rel(cnv_adjoint* a, cnv_ctx* c, const double* src, double rtol, int* kpred, int* sweeps) {
-    ALAUNCH_OF(a, poisson_init_launch(c->psi[0], c->ctl, nullptr, c->n, c->ld, 0.0, c->p.itmax, c->stream, !a->warm));
+    ALAUNCH_OF(a, poisson_init_launch(c->psi[0], c->ctl, nullptr, c->n, c->ld, 0.0, c->p.itmax, c->stream, !a->warm,
+                                      resident_reset_of(c)));
     hipLaunchKernelGGL(adj_slots_kernel, dim3(1), dim3(64), 0, c->stream, c->ctl, 1e-300, rtol, c->p.itmax);
     ALAUNCH(a);
     SorArgs<double> sa = sor_args64(c, src, 1);

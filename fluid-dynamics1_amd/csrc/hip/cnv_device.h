@@ -117,6 +117,40 @@ struct SorArgs {
                          // tests every sweep (0)
 };
 
+// A resident solve (sor_resident.h): its exchange planes, decision words and place on the XCDs.
+constexpr unsigned long long kMark64 = 0x7ff4c0de0badc0deull;  // signalling NaNs: not an arithmetic result
+constexpr unsigned kMark32 = 0x7fa5c0deu;
+constexpr int kResidentRows = 16;  // doubles per tile and epoch of partial sums (128 bytes)
+constexpr int kClaimStride = 32;   // ints between two XCDs' counters (128 bytes)
+struct SorResident {
+    void* exch;                // three planes of nr rows, pitch ldx, marked where nothing was given yet
+    long long xplane;          // elements of one plane
+    double* part;              // [4][ntiles][kResidentRows], marked
+    unsigned long long* dec;   // [ntiles][8]: each tile's decision word
+    double* snap;              // FP64 tiles too large for LDS: two copies of each extended tile
+    int* abort;                // set by a wave that gave up waiting
+    int ldx, ntiles;
+    int blocks;                // workgroups of a launch
+    int epochs, launch0;       // epochs at most; index of the first one within the solve
+    int stop;                  // > 0: run to exactly this many sweeps of the solve, without tests
+    int src, dst;              // planes of the input and of the result
+    int rslot, wslot;          // state slots read and written
+    int* claim;                // [9][kClaimStride]: tiles taken on each XCD; the deciding workgroup
+};
+constexpr int kBands = 8;      // XCDs of an MI355X, each with a band of tile rows
+__host__ __device__ inline int band_start(int band, int tiles_i) { return band * tiles_i / kBands; }
+constexpr int kNotStored = -1;  // SorCtl::rb_n: the solve has ended, its iterate is not in plane `parity` yet
+// FP64 tiles whose two copies fit in LDS
+constexpr bool resident_snap_lds(int nw, int rb) { return nw * rb <= 32; }
+// What one reset writes before a resident launch: marks over the exchange planes, marks over the
+// partial sums, zeros over the decision words and tile counters (in that order from base) and in the abort flag.
+struct ResidentReset {
+    unsigned long long* base;    // nullptr: nothing to reset
+    long long exch, part, zero;  // 64-bit words
+    unsigned long long mark;     // of the exchange planes
+    int* abort;
+};
+
 // Batched SOR launch: workgroup -> (solve, tile); inst < 0 marks padding workgroups, tile ==
 // the solve's tile count its deciding workgroup.
 struct SorBlock {
@@ -136,6 +170,10 @@ inline int tile_rows(const TileShape& t) { return t.nw * t.rb - 4 * t.s; }
 
 int sor_fp64_launch(const SorArgs<double>& a, TileShape shape, bool gs, hipStream_t st);
 int sor_fp32_launch(const SorArgs<float>& a, TileShape shape, bool gs, hipStream_t st);
+int sor_fp64_resident(const SorArgs<double>& a, const SorResident& r, TileShape shape, bool gs, hipStream_t st);
+int sor_fp32_resident(const SorArgs<float>& a, const SorResident& r, TileShape shape, bool gs, hipStream_t st);
+bool sor_resident_supported(TileShape shape);
+int resident_reset_launch(const ResidentReset& rr, hipStream_t st);
 bool sor_shape_supported(TileShape shape);
 
 int wall_vorticity_launch(double* w, const double* u, const double* v, int n, int ld,
@@ -148,7 +186,7 @@ int transport_fp32_launch(const double* w_in, double* w_out, const double* u, co
                           double dt, hipStream_t st);
 // zero = 0 keeps psi0 (warm start) and only resets the state slots and the diagnostic
 int poisson_init_launch(double* psi0, SorCtl* ctl, Diag* diag, int n, int ld, double tol,
-                        int itmax, hipStream_t st, int zero = 1);
+                        int itmax, hipStream_t st, int zero = 1, const ResidentReset& rr = ResidentReset{});
 // warm start: psi0 <- psi.p[fin->parity] (the previous solve's final iterate)
 int warm_start_launch(double* psi0, const Planes& psi, const SorCtl* fin, int n, int ld, hipStream_t st);
 int velocity_launch(const Planes& psi, const SorCtl* fin, double* u, double* v, int n, int ld,
@@ -174,7 +212,8 @@ int dc_correct_launch(double* psi, const float* e0, const float* e1, const SorCt
                       int ld, hipStream_t st);
 // budget != nullptr: the inner solve's sweep budget is read from that device counter
 int dc_inner_init_launch(float* e0, SorCtl* ctl, int n, int ld, double rtol, double tol,
-                         int itmax, hipStream_t st, const int* budget = nullptr);
+                         int itmax, hipStream_t st, const int* budget = nullptr,
+                         const ResidentReset& rr = ResidentReset{});
 // the device budget counter: fin == nullptr sets it to itmax, else subtracts fin->k
 int dc_budget_launch(int* budget, int itmax, const SorCtl* fin, hipStream_t st);
 

@@ -281,7 +281,8 @@ void cnv_destroy(cnv_ctx* c) {
     if (c->snap_stream) (void)hipStreamSynchronize(c->snap_stream);
     drop_graphs(c);
     void* dev[] = {c->w[0], c->w[1], c->psi[0], c->psi[1], c->psi[2], c->u, c->v, c->d_start, c->d_tab, c->d_ftab,
-                   c->ctl, c->diag, c->partial, c->e32[0], c->e32[1], c->r32, c->d_budget, c->d_snap};
+                   c->ctl, c->diag, c->partial, c->e32[0], c->e32[1], c->r32, c->d_budget, c->d_snap,
+                   c->d_res, c->d_res_snap};
     for (void* p : dev)
         if (p) (void)hipFree(p);
     if (c->h_ctl) (void)hipHostFree(c->h_ctl);
@@ -298,7 +299,9 @@ void cnv_destroy(cnv_ctx* c) {
     delete c;
 }
 
-int cnv_create(const cnv_params* p, cnv_ctx** out) {
+int cnv_create(const cnv_params* p, cnv_ctx** out) { return cnv_create_ctx(p, out, true); }
+
+int cnv_create_ctx(const cnv_params* p, cnv_ctx** out, bool resident) {
     if (!out) return cnv_fail(nullptr, CNV_ERR_ARG, "null output pointer");
     *out = nullptr;
     if (!p) return cnv_fail(nullptr, CNV_ERR_ARG, "null params");
@@ -355,9 +358,9 @@ int cnv_create(const cnv_params* p, cnv_ctx** out) {
         for (int b = 0; b < 3; ++b) HIPC(c, hipMalloc(&c->psi[b], bytes));
         HIPC(c, hipMalloc(&c->u, bytes));
         HIPC(c, hipMalloc(&c->v, bytes));
-        HIPC(c, hipMalloc(&c->ctl, 2 * sizeof(SorCtl)));
+        HIPC(c, hipMalloc(&c->ctl, 3 * sizeof(SorCtl)));
         HIPC(c, hipMalloc(&c->diag, sizeof(Diag)));
-        HIPC(c, hipMemset(c->ctl, 0, 2 * sizeof(SorCtl)));
+        HIPC(c, hipMemset(c->ctl, 0, 3 * sizeof(SorCtl)));
         HIPC(c, hipMemset(c->diag, 0, sizeof(Diag)));
         HIPC(c, hipMalloc(&c->partial, sizeof(double) * 2 * 2 * kMaxSweepsPerLaunch * (size_t)c->tiles_i * c->tiles_j));
         HIPC(c, hipHostMalloc(&c->h_ctl, sizeof(SorCtl) * kSlots, hipHostMallocDefault));
@@ -371,6 +374,7 @@ int cnv_create(const cnv_params* p, cnv_ctx** out) {
             HIPC(c, hipMalloc(&c->d_budget, sizeof(int)));
         }
         int rc = upload_tables(c);
+        if (!rc && resident) rc = resident_setup(c);
         if (rc) return rc;
         return initial_state(c);
     };
@@ -393,7 +397,7 @@ static int poisson_fp64(cnv_ctx* c, const double* f_src, int negate, SorCtl* fin
     if (c->p.warm_start)
         LAUNCH(c, warm_start_launch(c->psi[0], planes_of(c), c->ctl + c->fin_slot, c->n, c->ld, c->stream));
     LAUNCH(c, poisson_init_launch(c->psi[0], c->ctl, c->diag, c->n, c->ld, c->p.tol, c->p.itmax, c->stream,
-                                  !c->p.warm_start));
+                                  !c->p.warm_start, resident_reset_of(c)));
     SorArgs<double> a = sor_args64(c, f_src, negate);
     int rc = run_sor<double>(c, a, fin);
     if (rc) return rc;
@@ -416,7 +420,7 @@ static int poisson_dc(cnv_ctx* c, const double* w_src, SorCtl* fin, int* outer) 
     for (int o = 0; o < max_outer && total < c->p.itmax; ++o) {
         LAUNCH(c, dc_residual_launch(w_src, c->psi[0], c->r32, c->n, c->ld, c1, c2, c3, B, c->stream));
         LAUNCH(c, dc_inner_init_launch(c->e32[0], c->ctl, c->n, c->ld, c->p.inner_rtol, c->p.tol, c->p.itmax - total,
-                                       c->stream));
+                                       c->stream, nullptr, resident_reset_of(c)));
         SorCtl snap{};
         c->k_prev = o < cnv_ctx::kDcPred ? c->k_dc[o] : 0;  // this outer iteration's last length
         int rc = run_sor<float>(c, a, &snap);
@@ -483,7 +487,7 @@ static int body_pre(cnv_ctx* c, int wc) {
     // warm start: whole chunks end on slot 1, which holds the previous solve's final state
     if (c->p.warm_start) LAUNCH(c, warm_start_launch(c->psi[0], planes_of(c), c->ctl + 1, n, ld, c->stream));
     LAUNCH(c, poisson_init_launch(c->psi[0], c->ctl, c->diag, n, ld, c->p.tol, c->p.itmax, c->stream,
-                                  !c->p.warm_start));
+                                  !c->p.warm_start, resident_reset_of(c)));
     return CNV_OK;
 }
 // m SOR launches, L = 0..m-1: FP64 on the source w[src] (f = -w), or the refined form's FP32
@@ -510,7 +514,7 @@ static int body_resid(cnv_ctx* c, int src) {
     LAUNCH(c, dc_residual_launch(c->w[src], c->psi[0], c->r32, c->n, c->ld, dy * dy, dx * dx,
                                  dx * dx * dy * dy, 2 * (dx * dx + dy * dy), c->stream));
     LAUNCH(c, dc_inner_init_launch(c->e32[0], c->ctl, c->n, c->ld, c->p.inner_rtol, c->p.tol, 0, c->stream,
-                                   c->d_budget));
+                                   c->d_budget, resident_reset_of(c)));
     return CNV_OK;
 }
 // ... and after the inner solve (final slot 1): psi[0] += e, budget -= its sweeps
@@ -531,11 +535,8 @@ static int build_graphs(cnv_ctx* c) {
     // whole chunks end on slot 1 and on the launch index's phase (plane rotation, stopping tests)
     const int u = c->tail_chunk;
     c->launches_per_poll = (c->launches_per_poll + u - 1) / u * u;
-    const int nsrc = is_dc(c) ? 1 : 2;  // the refined form's inner solves always read r32
     for (int wc = 0; wc < 2; ++wc) {
         int rc = capture(c, &c->g_pre[wc], body_pre, wc);
-        if (!rc && wc < nsrc) rc = capture(c, &c->g_chunk[wc], body_chunk, wc);
-        if (!rc && wc < nsrc) rc = capture(c, &c->g_tail[wc], body_tail, wc);
         if (!rc && is_dc(c)) rc = capture(c, &c->g_resid[wc], body_resid, wc);
         if (rc) return rc;
     }
@@ -551,6 +552,21 @@ static int build_graphs(cnv_ctx* c) {
 // tail chunks follow, as many per poll as make up the eager solve's chunk for that prediction
 // (poll_chunk); without one, big chunks one per poll.
 static int replay_solve(cnv_ctx* c, int src, int predicted_sweeps, SorCtl* final_ctl) {
+    bool ran = false;
+    int rc = is_dc(c) ? run_sor_resident<float>(c, sor_args32(c), final_ctl, &ran)
+                      : run_sor_resident<double>(c, sor_args64(c, c->w[src], 1), final_ctl, &ran);
+    if (rc) return rc;
+    if (ran) {  // the captured launches that follow read slot 1
+        if (c->fin_slot != 1)
+            HIPC(c, hipMemcpyAsync(c->ctl + 1, c->ctl, sizeof(SorCtl), hipMemcpyDeviceToDevice, c->stream));
+        c->fin_slot = 1;
+        return CNV_OK;
+    }
+    if (!c->g_tail[src]) {  // captured when a solve first needs them
+        rc = capture(c, &c->g_chunk[src], body_chunk, src);
+        if (!rc) rc = capture(c, &c->g_tail[src], body_tail, src);
+        if (rc) return rc;
+    }
     const int M = c->launches_per_poll, Mt = c->tail_chunk;
     const int S = c->shape.s;
     const int P = predicted_sweeps > 0 ? predicted_sweeps / S : 0;

@@ -29,7 +29,7 @@ struct cnv_ctx {
     float* d_ftab = nullptr;
     cnv::Stencils st{};
     // solver control
-    cnv::SorCtl* ctl = nullptr;  // the Poisson solve's two state slots
+    cnv::SorCtl* ctl = nullptr;  // the Poisson solve's two state slots, then the resident abort flag
     int fin_slot = 0;            // slot written by the last SOR launch of the last solve
     cnv::Diag* diag = nullptr;
     double* partial = nullptr;
@@ -62,6 +62,15 @@ struct cnv_ctx {
     hipGraphExec_t g_resid[2] = {nullptr, nullptr};
     hipGraphExec_t g_correct = nullptr;
     hipGraphExec_t g_post = nullptr;
+    // resident solves (sor_resident.h): usable, their memory and arguments, CUs they need (resident.hip)
+    bool res_on = false;
+    unsigned long long* d_res = nullptr;
+    double* d_res_snap = nullptr;
+    cnv::SorResident res{};
+    cnv::ResidentReset res_reset{};
+    int res_units = 0;
+    cnv::TileShape res_shape{5, 16, 4};
+    int res_tiles_i = 0, res_tiles_j = 0;
     int* d_budget = nullptr;  // refined form, captured: the solve's remaining sweep budget
     // output snapshots (cnv_snapshot_begin/wait): a device copy of (w, psi, u, v) taken in stream
     // order, then transferred to pinned host memory on a stream of its own
@@ -195,7 +204,7 @@ inline int poll_chunk(const cnv_ctx* c, int predicted_launches) {
     return m < 4 ? 4 : (m > 32 ? 32 : m);
 }
 template <typename T>
-inline int run_sor(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* final_ctl) {
+inline int run_sor_launches(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* final_ctl, int launch0 = 0) {
     const bool gs = (c->p.poisson_type == 1);
     const int S = c->shape.s;
     const int P = c->k_prev > 0 ? c->k_prev / S : 0;  // predicted launches
@@ -210,11 +219,11 @@ inline int run_sor(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* final_ctl)
     while (true) {
         const int chunk = queued == 0 ? first : M;
         for (int l = 0; l < chunk; ++l) {
-            if (launch_sor(c, a, (int)(queued + l), gs))
+            if (launch_sor(c, a, launch0 + (int)(queued + l), gs))
                 return cnv_fail(c, CNV_ERR_HIP, "SOR launch failed: %s", hipGetErrorString(hipGetLastError()));
         }
         queued += chunk;
-        c->fin_slot = (int)((queued - 1) & 1);
+        c->fin_slot = (int)((launch0 + queued - 1) & 1);
         HIPC(c, hipMemcpyAsync(&c->h_ctl[slot], c->ctl + c->fin_slot, sizeof(cnv::SorCtl), hipMemcpyDeviceToHost, c->stream));
         HIPC(c, hipEventRecord(c->ev[slot], c->stream));
         pending[npend++] = slot;
@@ -233,3 +242,21 @@ inline int run_sor(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* final_ctl)
         if (queued > cap + first) return cnv_fail(c, CNV_ERR_HIP, "SOR state did not terminate after %lld launches", queued);
     }
 }
+
+// ---- resident solves (resident.hip) -----------------------------------------------------------
+// Sets up the context's resident solves where its grid and the device allow them.
+int resident_setup(cnv_ctx* c);
+// What the init kernels reset for a solve that may run resident.
+inline cnv::ResidentReset resident_reset_of(const cnv_ctx* c) { return c->res_on ? c->res_reset : cnv::ResidentReset{}; }
+// The solve as resident kernels when they can run now (*ran = false: nothing was done).
+template <typename T>
+int run_sor_resident(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* final_ctl, bool* ran);
+
+template <typename T>
+inline int run_sor(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* final_ctl) {
+    bool ran = false;
+    const int rc = run_sor_resident<T>(c, a, final_ctl, &ran);
+    return ran ? rc : run_sor_launches<T>(c, a, final_ctl);
+}
+// cnv_create without (resident = false) the memory of resident solves, which a batch does not use.
+int cnv_create_ctx(const cnv_params* p, cnv_ctx** out, bool resident);

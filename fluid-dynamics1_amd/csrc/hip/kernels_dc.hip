@@ -22,12 +22,17 @@
 
 #include "cnv_device.h"
 #include "sor_rb.h"
+#include "sor_resident.h"
 #include "step_kernels.h"
 
 namespace cnv {
 
 int sor_fp32_launch(const SorArgs<float>& a, TileShape shape, bool gs, hipStream_t st) {
     return sor_dispatch<float>(a, shape, gs, st);
+}
+
+int sor_fp32_resident(const SorArgs<float>& a, const SorResident& r, TileShape shape, bool gs, hipStream_t st) {
+    return sor_resident_dispatch<float>(a, r, shape, gs, st);
 }
 
 // r32 = (float)(f - L psi) on the interior, f = -w; 0 on the edges.
@@ -54,11 +59,12 @@ __global__ void __launch_bounds__(kBlock) dc_correct_kernel(double* __restrict__
 // solver's stopping rule) and the FP32 fold ratio
 __global__ void __launch_bounds__(kBlock) dc_inner_init_kernel(float* e0, SorCtl* ctl, long long count,
                                                               double rtol, double tol, int itmax,
-                                                              const int* budget) {
+                                                              const int* budget, ResidentReset rr) {
     const long long stride = (long long)gridDim.x * kBlock;
     for (long long q = (long long)blockIdx.x * kBlock + threadIdx.x; q < count; q += stride) e0[q] = 0.0f;
     // the sweep budget comes from the device counter when there is one (captured step)
     if (blockIdx.x == 0 && threadIdx.x < 2) ctl_reset(ctl + threadIdx.x, tol, rtol, budget ? *budget : itmax);
+    resident_reset_at(rr);
 }
 
 // device sweep budget of a refined solve: fin == nullptr resets it to itmax, otherwise the inner
@@ -111,12 +117,12 @@ int dc_correct_launch(double* psi, const float* e0, const float* e1, const SorCt
 }
 
 int dc_inner_init_launch(float* e0, SorCtl* ctl, int n, int ld, double rtol, double tol, int itmax,
-                         hipStream_t st, const int* budget) {
+                         hipStream_t st, const int* budget, const ResidentReset& rr) {
     const long long count = (long long)n * ld;
-    unsigned nb = blocks_for(count);
+    unsigned nb = blocks_for(count + rr.exch);
     if (nb > 2048) nb = 2048;
     hipLaunchKernelGGL(dc_inner_init_kernel, dim3(nb), dim3(kBlock), 0, st, e0, ctl, count, rtol, tol, itmax,
-                       budget);
+                       budget, rr);
     return launched();
 }
 

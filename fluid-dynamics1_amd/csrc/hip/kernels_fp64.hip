@@ -10,6 +10,7 @@
 
 #include "cnv_device.h"
 #include "sor_rb.h"
+#include "sor_resident.h"
 #include "step_kernels.h"
 
 namespace cnv {
@@ -33,12 +34,13 @@ __global__ void __launch_bounds__(kBlock) transport_fp64_kernel(const double* __
 // ---- start of a Poisson solve: psi = 0 (src/poisson.c:229-230), reset the control block ----
 __global__ void __launch_bounds__(kBlock) poisson_init_kernel(double* psi0, SorCtl* ctl, Diag* diag,
                                                              long long count, double tol, int itmax,
-                                                             int zero) {
+                                                             int zero, ResidentReset rr) {
     const long long stride = (long long)gridDim.x * kBlock;
     if (zero)
         for (long long q = (long long)blockIdx.x * kBlock + threadIdx.x; q < count; q += stride) psi0[q] = 0.0;
     if (blockIdx.x == 0 && threadIdx.x < 2) ctl_reset(ctl + threadIdx.x, tol, 0.0, itmax);
     if (blockIdx.x == 0 && threadIdx.x == 0 && diag) diag_reset(diag);
+    resident_reset_at(rr);
 }
 
 // warm start (opt-in): the previous solve's final iterate, psi[fin->parity], becomes psi0, the
@@ -119,12 +121,33 @@ __global__ void __launch_bounds__(kBlock) snapshot_kernel(const double* __restri
     }
 }
 
+// marks and zeros before a resident solve (ResidentReset)
+__global__ void __launch_bounds__(kBlock) resident_reset_kernel(ResidentReset rr) { resident_reset_at(rr); }
+
 // ---- host wrappers -------------------------------------------------------------------------
 static inline int launched() { return hipGetLastError() == hipSuccess ? 0 : 1; }
 static inline unsigned blocks_for(long long count) { return (unsigned)((count + kBlock - 1) / kBlock); }
 
 int sor_fp64_launch(const SorArgs<double>& a, TileShape shape, bool gs, hipStream_t st) {
     return sor_dispatch<double>(a, shape, gs, st);
+}
+
+int sor_fp64_resident(const SorArgs<double>& a, const SorResident& r, TileShape shape, bool gs, hipStream_t st) {
+    return sor_resident_dispatch<double>(a, r, shape, gs, st);
+}
+
+bool sor_resident_supported(TileShape sh) {
+#define CNV_RES_OK(s_, nw_, rb_) if (sh.s == s_ && sh.nw == nw_ && sh.rb == rb_) return true;
+    CNV_RESIDENT_SHAPES(CNV_RES_OK)
+#undef CNV_RES_OK
+    return false;
+}
+
+int resident_reset_launch(const ResidentReset& rr, hipStream_t st) {
+    unsigned nb = blocks_for(rr.exch + rr.part + rr.zero);
+    if (nb > 2048) nb = 2048;
+    hipLaunchKernelGGL(resident_reset_kernel, dim3(nb), dim3(kBlock), 0, st, rr);
+    return launched();
 }
 
 bool sor_shape_supported(TileShape sh) {
@@ -148,12 +171,12 @@ int transport_fp64_launch(const double* w_in, double* w_out, const double* u, co
 }
 
 int poisson_init_launch(double* psi0, SorCtl* ctl, Diag* diag, int n, int ld, double tol, int itmax,
-                        hipStream_t st, int zero) {
+                        hipStream_t st, int zero, const ResidentReset& rr) {
     const long long count = (long long)n * ld;
-    unsigned nb = blocks_for(count);
+    unsigned nb = blocks_for(count + rr.exch);
     if (nb > 2048) nb = 2048;
     hipLaunchKernelGGL(poisson_init_kernel, dim3(nb), dim3(kBlock), 0, st, psi0, ctl, diag, count, tol, itmax,
-                       zero);
+                       zero, rr);
     return launched();
 }
 

@@ -175,176 +175,167 @@ __device__ inline T* sor_plane(const SorArgs<T>& a, int idx) {
     else return idx == 0 ? a.psi0 : (idx == 1 ? a.psi1 : a.psi2);
 }
 
-// One sweeping workgroup's launch on tile `tile` of the solve described by `a` (NW*64 threads).
-// It reads the state slot the previous launch's decider wrote: RUNNING -- sweep on from plane
-// L % NB (the previous launch's output) into plane (L+1) % NB, as many sweeps as the budget
-// leaves, and leave this tile's per-sweep L1 sums for the next launch's decider; ROLLBACK -- the
-// solve converged inside the launch before last: redo rb_n sweeps from plane rb_src into plane
-// `parity`, which then holds the final iterate; anything else -- the solve has ended: return.
+// A workgroup's tile in registers (NW waves of 64 lanes): wave w holds rows [w*RB, w*RB + RB) of the
+// extended tile, lane m columns 2m and 2m+1.
 template <typename T, int S, int NW, int RB, bool GS, bool XR, bool NORM>
-__device__ __forceinline__ void sor_rb_sweeper(const SorArgs<T>& a, const int L, const int tile) {
-#pragma clang fp contract(off)
-    constexpr int NB = SorPlanes<T>::value;
-    constexpr int H = 2 * S;
+struct SorTile {
+    static constexpr int H = 2 * S;
+    static constexpr int EJ = 128;  // extended tile columns; lane m holds columns 2m, 2m+1
+    static constexpr int TJ = EJ - 2 * H;
+    static constexpr int EI = NW * RB;  // extended tile rows; wave w holds rows [w*RB, w*RB+RB)
+    static constexpr int TI = EI - 2 * H;
+    static_assert(TI > 0 && TJ > 0, "halo larger than the tile");
+    static_assert(RB % 2 == 0, "even row blocks keep each wave's colour pattern static");
     // the iterate's L1 norm is needed by the relative stopping rule (rtol): always on FP32
     // planes, on request (NORM) for FP64.  It is measured once per launch, after its last sweep.
-    constexpr bool kNorm = sizeof(T) == 4 || NORM;
+    static constexpr bool kNorm = sizeof(T) == 4 || NORM;
     // FP32 planes (the inner solves of defect correction) are a preconditioner with no bit-parity
     // requirement: their stopping rule is applied to a launch's last sweep only (and only on the
     // launches the test mask selects), so the other sweeps skip the L1 update (a solve runs at
     // most (test_mask + 1) * S - 1 sweeps past the first sweep that met the rule).  FP64 applies
     // it to every sweep, as src/poisson.c:272-278 does.
-    constexpr bool kLastOnly = sizeof(T) == 4;
-    constexpr int SE = kLastOnly ? 1 : S;  // L1 update sums per launch
-    constexpr int EJ = 128;          // extended tile columns; lane m holds columns 2m, 2m+1
-    constexpr int TJ = EJ - 2 * H;
-    constexpr int EI = NW * RB;      // extended tile rows; wave w holds rows [w*RB, w*RB+RB)
-    constexpr int TI = EI - 2 * H;
-    static_assert(TI > 0 && TJ > 0, "halo larger than the tile");
-    static_assert(RB % 2 == 0, "even row blocks keep each wave's colour pattern static");
+    static constexpr bool kLastOnly = sizeof(T) == 4;
+    static constexpr int SE = kLastOnly ? 1 : S;  // L1 update sums per launch
     typedef typename std::conditional<sizeof(T) == 4, float, double>::type Acc;
+    typedef typename PairOf<T>::type Pair;
 
-    __shared__ T xch[2][NW][2][64];  // [half-sweep parity][wave][first/last row][lane]
-    // one column per thread: this launch's per-lane L1 update sums, one row per summed sweep,
-    // and the per-lane iterate norm after the last sweep
-    __shared__ double lred[SE][NW * 64];
-    __shared__ double lnrm[kNorm ? NW * 64 : 1];
-
-    const SorCtl* prev = a.ctl + ((L + 1) & 1);
-    const int tid = threadIdx.x;
-    const int ntiles = a.tiles_i * a.tiles_j;
-    const int ti = tile / a.tiles_j;
-    const int tj = tile - ti * a.tiles_j;
-    const int gi0 = ti * TI - H;  // even, so the colour of local (li, lj) is (li + lj) & 1
-    const int gj0 = tj * TJ - H;
-    const int nr = a.nr, nc = a.nc;
-    const long long ld = a.ld;
-    const int lane = threadIdx.x & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform (SGPR)
-    const int row0 = wv * RB;        // even: the colour of (row0 + r, 2m + q) is (r + q) & 1
-
-    // Column facts of the lane's pair (gj, gj+1), gj even: q = 0 -> column gj, q = 1 -> gj+1.
-    const int gj = gj0 + 2 * lane;
-    bool colin[2], ownc[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        colin[q] = gj + q >= 1 && gj + q <= nc - 2;
-        ownc[q] = 2 * lane + q >= H && 2 * lane + q < H + TJ && gj + q < nc;  // ownc[1] implies ownc[0]
-    }
-    // Every load reads a pair inside the data: rows clamped into [0, nr), the pair's first column
-    // into [0, nc-2].  So no lane needs a select on what it loads: a point outside the domain may
-    // start from any finite value (it is read only by points outside the domain and by the domain
-    // boundary, whose relaxation factor is 0), and each domain-boundary point is read from its own
-    // position (+-0 there).  With nc odd, the lane of column nc-1 reads the pair (nc-2, nc-1) and
-    // takes its second element (fixed after the loads); its column nc is outside.
-    const unsigned bld = (unsigned)(gj < 0 ? 0 : (gj > nc - 2 ? nc - 2 : gj)) * sizeof(T);
-    auto row_of = [&](const T* plane, int gi) -> const T* {  // wave-uniform row pointer
-        return plane + (gi < 0 ? 0 : (gi >= nr ? nr - 1 : gi)) * ld;
+    // LDS: the waves' first and last rows, and one column per thread of per-lane sums
+    struct Shared {
+        T xch[2][NW][2][64];  // [half-sweep parity][wave][first/last row][lane]
+        double lred[SE][NW * 64];  // this launch's per-lane L1 update sums, one row per summed sweep
+        double lnrm[kNorm ? NW * 64 : 1];  // the per-lane iterate norm after the last sweep
     };
 
-    // relaxation factor of an updated point: FP64 beta (1 for Gauss-Seidel), applied before the
-    // division; FP32 beta/B (1/B), which folds the division in.  Per column, 0 off the interior
-    // columns; per point, also 0 on the boundary rows and outside the domain.
-    T bcoef;
-    if constexpr (sizeof(T) == 8) bcoef = GS ? T(1) : a.beta;
-    else bcoef = GS ? a.rB : a.beta * a.rB;
-    const T c3s = a.negate ? -a.c3 : a.c3;  // f = -src folded in: c3*(-x) == (-c3)*x exactly
-    T bcol[2], cncol[2], cecol[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        bcol[q] = colin[q] ? bcoef : T(0);
-        cncol[q] = colin[q] ? bcoef * a.c1 : T(0);
-        cecol[q] = colin[q] ? bcoef * a.c2 : T(0);
-    }
-
-    // Speculative tile load for the common case (sweep on from the previous launch's output),
-    // issued before the state slot is read so that both are in flight together.
-    const T* __restrict__ srcN = sor_plane(a, L % NB);
     T v[2][RB];   // v[q][r]: value at (row0 + r, 2*lane + q)
     T fc[2][RB];  // FP64: c3*f (the hoisted c3*f product of the update); FP32: -be*c3*f
     T be[2][RB];  // FP64: bcoef at interior points, 0 on the domain boundary and outside it
     T cn[2][RB];  // FP32: be*c1 and be*c2, the relaxation folded into the stencil coefficients
     T ce[2][RB];
     Acc w[RB];    // 1 for owned rows inside the domain, else 0 (wave-uniform)
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-        const int li = row0 + r;
-        const int gi = gi0 + li;
-        const bool rint = gi >= 1 && gi <= nr - 2;
-        w[r] = (li >= H && li < H + TI && gi < nr) ? Acc(1) : Acc(0);
-        const typename PairOf<T>::type d = load_pair(row_of(srcN, gi), bld);
-        const typename PairOf<T>::type f = load_pair(row_of(a.src_f, gi), bld);
-        v[0][r] = d.x;
-        v[1][r] = d.y;
+    T c1, c2, B, rB, omb;
+    int gi0, gj0, gj, lane, wv, row0, nr, nc;
+    unsigned bld;
+    bool colin[2], ownc[2];
+
+    __device__ __forceinline__ void place(const SorArgs<T>& a, int ti, int tj) {
+        gi0 = ti * TI - H;  // even, so the colour of local (li, lj) is (li + lj) & 1
+        gj0 = tj * TJ - H;
+        nr = a.nr;
+        nc = a.nc;
+        lane = threadIdx.x & 63;
+        wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform (SGPR)
+        row0 = wv * RB;  // even: the colour of (row0 + r, 2m + q) is (r + q) & 1
+        // Column facts of the lane's pair (gj, gj+1), gj even: q = 0 -> column gj, q = 1 -> gj+1.
+        gj = gj0 + 2 * lane;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-            // a non-interior point's source is not read by the reference: 0, whatever it holds
-            const bool inter = rint && colin[q];
-            const T fq = q ? f.y : f.x;
-            if constexpr (sizeof(T) == 8) {
-                fc[q][r] = inter ? c3s * fq : T(0);
-                be[q][r] = rint ? bcol[q] : T(0);
-            } else {
-                fc[q][r] = inter ? bcoef * -(c3s * fq) : T(0);
-                cn[q][r] = rint ? cncol[q] : T(0);
-                ce[q][r] = rint ? cecol[q] : T(0);
-            }
+            colin[q] = gj + q >= 1 && gj + q <= nc - 2;
+            ownc[q] = 2 * lane + q >= H && 2 * lane + q < H + TJ && gj + q < nc;  // ownc[1] implies ownc[0]
         }
+        // Every load reads a pair inside the data: rows clamped into [0, nr), the pair's first column
+        // into [0, nc-2].  So no lane needs a select on what it loads: a point outside the domain may
+        // start from any finite value (it is read only by points outside the domain and by the domain
+        // boundary, whose relaxation factor is 0), and each domain-boundary point is read from its own
+        // position (+-0 there).  With nc odd, the lane of column nc-1 reads the pair (nc-2, nc-1) and
+        // takes its second element (fixed after the loads); its column nc is outside.
+        bld = (unsigned)(gj < 0 ? 0 : (gj > nc - 2 ? nc - 2 : gj)) * sizeof(T);
+    }
+    __device__ __forceinline__ const T* row_of(const SorArgs<T>& a, const T* plane, int gi) const {  // wave-uniform row pointer
+        return plane + (gi < 0 ? 0 : (gi >= nr ? nr - 1 : gi)) * (long long)a.ld;
     }
 
-    // what this launch does: the state after launch L-2 and the sweeps launch L-1 performed
-    const int pstatus = prev->status;
-    bool rollback = false;
-    int s_run = 0;
-    T* __restrict__ dst = nullptr;
-    if (pstatus == SOR_RUNNING) {
-        const int budget = prev->itmax - (prev->k + prev->s_done);
-        s_run = budget < S ? budget : S;
-        dst = sor_plane(a, (L + 1) % NB);
-    } else if (pstatus == SOR_ROLLBACK) {
-        rollback = true;
-        s_run = prev->rb_n;
-        dst = sor_plane(a, prev->parity);
-    }
-    if (s_run <= 0) return;  // the solve has ended, or its budget is spent
-    // FP32: whether this launch's last sweep is tested (FP64: every sweep of every launch)
-    const bool tested = sizeof(T) == 8 || (L & a.test_mask) == a.test_mask;
-    if (rollback) {
-        // the converged launch's input replaces the speculatively loaded tile
-        const T* __restrict__ srcR = sor_plane(a, prev->rb_src);
+    // the tile's values from plane src, its source term and its coefficients
+    __device__ __forceinline__ void load(const SorArgs<T>& a, const T* __restrict__ src) {
+#pragma clang fp contract(off)
+        // relaxation factor of an updated point: FP64 beta (1 for Gauss-Seidel), applied before the
+        // division; FP32 beta/B (1/B), which folds the division in.  Per column, 0 off the interior
+        // columns; per point, also 0 on the boundary rows and outside the domain.
+        T bcoef;
+        if constexpr (sizeof(T) == 8) bcoef = GS ? T(1) : a.beta;
+        else bcoef = GS ? a.rB : a.beta * a.rB;
+        const T c3s = a.negate ? -a.c3 : a.c3;  // f = -src folded in: c3*(-x) == (-c3)*x exactly
+        T bcol[2], cncol[2], cecol[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            bcol[q] = colin[q] ? bcoef : T(0);
+            cncol[q] = colin[q] ? bcoef * a.c1 : T(0);
+            cecol[q] = colin[q] ? bcoef * a.c2 : T(0);
+        }
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
-            const typename PairOf<T>::type d = load_pair(row_of(srcR, gi0 + row0 + r), bld);
+            const int li = row0 + r;
+            const int gi = gi0 + li;
+            const bool rint = gi >= 1 && gi <= nr - 2;
+            w[r] = (li >= H && li < H + TI && gi < nr) ? Acc(1) : Acc(0);
+            const Pair d = load_pair(row_of(a, src, gi), bld);
+            const Pair f = load_pair(row_of(a, a.src_f, gi), bld);
+            v[0][r] = d.x;
+            v[1][r] = d.y;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                // a non-interior point's source is not read by the reference: 0, whatever it holds
+                const bool inter = rint && colin[q];
+                const T fq = q ? f.y : f.x;
+                if constexpr (sizeof(T) == 8) {
+                    fc[q][r] = inter ? c3s * fq : T(0);
+                    be[q][r] = rint ? bcol[q] : T(0);
+                } else {
+                    fc[q][r] = inter ? bcoef * -(c3s * fq) : T(0);
+                    cn[q][r] = rint ? cncol[q] : T(0);
+                    ce[q][r] = rint ? cecol[q] : T(0);
+                }
+            }
+        }
+        c1 = a.c1;
+        c2 = a.c2;
+        B = a.B;
+        rB = a.rB;
+        omb = a.omb;
+    }
+    __device__ __forceinline__ void load_values(const SorArgs<T>& a, const T* __restrict__ src) {
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            const Pair d = load_pair(row_of(a, src, gi0 + row0 + r), bld);
             v[0][r] = d.x;
             v[1][r] = d.y;
         }
     }
-    if (nc & 1) {  // wave-uniform: the lane of column nc-1 read the pair (nc-2, nc-1)
-        if (gj == nc - 1) {
+    __device__ __forceinline__ void fix_odd_edge() {
+        if (nc & 1) {  // wave-uniform: the lane of column nc-1 read the pair (nc-2, nc-1)
+            if (gj == nc - 1) {
 #pragma unroll
-            for (int r = 0; r < RB; ++r) v[0][r] = v[1][r];
+                for (int r = 0; r < RB; ++r) v[0][r] = v[1][r];
+            }
         }
     }
+    __device__ __forceinline__ bool owns_rows() const {  // wave-uniform: the wave holds an owned row
+        bool owns = false;
+#pragma unroll
+        for (int r = 0; r < RB; ++r) owns = owns || w[r] != Acc(0);
+        return owns;
+    }
 
-    const T c1 = a.c1, c2 = a.c2, B = a.B, rB = a.rB, omb = a.omb;
     // half-sweep 0 updates colour 0 and reads its neighbours' colour-1 boundary rows: colour 1
     // sits in column q = (r + 1) & 1 of row r
-    auto sweeps_begin = [&]() {
-        xch[1][wv][0][lane] = v[1][0];
-        xch[1][wv][1][lane] = v[(RB - 1 + 1) & 1][RB - 1];
+    __device__ __forceinline__ void begin(Shared& sh) {
+        sh.xch[1][wv][0][lane] = v[1][0];
+        sh.xch[1][wv][1][lane] = v[(RB - 1 + 1) & 1][RB - 1];
         __syncthreads();
-    };
+    }
     // sweep s (red half-sweep, then black) of a pass; with_norm: also sum the iterate's norm
-    // (FP32: and the update, which only the last sweep sums); l1 (std::true_type or false_type):
-    // sum the L1 norms at all, which a wave holding no owned row skips (its sums are 0)
-    auto one_sweep = [&](const int s, const bool with_norm, auto l1) {
-        constexpr bool kL1 = decltype(l1)::value;
+    // (FP32: and the update, which only the last sweep sums); kL1: sum the L1 norms at all, which
+    // a wave holding no owned row skips (its sums are 0); more: another sweep follows, which needs
+    // the other waves' boundary rows
+    template <bool kL1>
+    __device__ __forceinline__ void sweep(Shared& sh, const int s, const bool with_norm, const bool more) {
+#pragma clang fp contract(off)
+        const int tid = threadIdx.x;
         Acc acc[2] = {Acc(0), Acc(0)}, nrm[2] = {Acc(0), Acc(0)};
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             // boundary rows of the neighbouring waves (colour 1-c, written by half-sweep h-1)
-            const T sb = xch[c ^ 1][wv > 0 ? wv - 1 : 0][1][lane];
-            const T nb = xch[c ^ 1][wv < NW - 1 ? wv + 1 : NW - 1][0][lane];
+            const T sb = sh.xch[c ^ 1][wv > 0 ? wv - 1 : 0][1][lane];
+            const T nb = sh.xch[c ^ 1][wv < NW - 1 ? wv + 1 : NW - 1][0][lane];
             // rows 1..RB-2 first: they do not wait for the LDS reads of sb / nb
 #pragma unroll
             for (int rr = 0; rr < RB; ++rr) {
@@ -380,85 +371,143 @@ __device__ __forceinline__ void sor_rb_sweeper(const SorArgs<T>& a, const int L,
                     }
                 }
             }
-            xch[c][wv][0][lane] = v[c & 1][0];
-            xch[c][wv][1][lane] = v[(c + RB - 1) & 1][RB - 1];
-            __syncthreads();
+            if (c == 0 || more) {
+                sh.xch[c][wv][0][lane] = v[c & 1][0];
+                sh.xch[c][wv][1][lane] = v[(c + RB - 1) & 1][RB - 1];
+                __syncthreads();
+            }
         }
         // per-lane sums of this sweep, owned columns only; reduced once after the last sweep
         if (!kLastOnly || with_norm)
-            lred[kLastOnly ? 0 : s][tid] = (double)((ownc[0] ? acc[0] : Acc(0)) + (ownc[1] ? acc[1] : Acc(0)));
+            sh.lred[kLastOnly ? 0 : s][tid] = (double)((ownc[0] ? acc[0] : Acc(0)) + (ownc[1] ? acc[1] : Acc(0)));
         if (kNorm && with_norm)
-            lnrm[tid] = (double)((ownc[0] ? nrm[0] : Acc(0)) + (ownc[1] ? nrm[1] : Acc(0)));
-    };
-    // the common full pass, unrolled: the values stay in their registers from sweep to sweep (a
-    // rolled loop makes the compiler rotate them through copies at every iteration); not for the
-    // FP64 shapes whose unrolled pass no longer fits the register budget of their wave count.
-    // A rollback or a budget-limited last launch takes the loop, which sums the FP64 norm in
-    // every sweep (the last one's stays).
-    // The waves that hold only halo rows (a quarter of them at 1024^2) run it without the FP64
-    // L1 sums, two of the point update's 14 instructions.
-    constexpr bool kUnroll = sizeof(T) == 4 || (S * RB <= 40 && NW != 12 && !(kNorm && S * RB > 20));
-    bool owns = false;  // wave-uniform: the wave holds an owned row
-#pragma unroll
-    for (int r = 0; r < RB; ++r) owns = owns || w[r] != Acc(0);
-    sweeps_begin();
-    if (kUnroll && s_run == S) {
-        // FP32: an untested launch skips the last sweep's sums.  Small shapes get a pass of their
-        // own without them (6.10 against 6.29 us per launch at 1024^2 with (5, 16, 4)); large ones
-        // branch on the uniform flag in the last sweep, since a second unrolled pass of their
-        // size made the kernel slower (the batched (8, 8, 10) FP32 sweep 4.05 -> 4.7 us)
-        constexpr bool kSplit = sizeof(T) == 4 && S * RB <= 24;
-        if (kSplit && !tested) {
-#pragma unroll
-            for (int s = 0; s < S; ++s) one_sweep(s, false, std::false_type{});
-        } else if (owns || sizeof(T) == 4) {
-#pragma unroll
-            for (int s = 0; s < S; ++s) one_sweep(s, s == S - 1 && (kSplit || tested), std::true_type{});
-        } else {
-#pragma unroll
-            for (int s = 0; s < S; ++s) one_sweep(s, s == S - 1, std::false_type{});
-        }
-    } else {
-        for (int s = 0; s < s_run; ++s) one_sweep(s, kLastOnly ? tested && s == s_run - 1 : kNorm, std::true_type{});
+            sh.lnrm[tid] = (double)((ownc[0] ? nrm[0] : Acc(0)) + (ownc[1] ? nrm[1] : Acc(0)));
     }
+    // s_run sweeps of a launch or epoch, with the L1 sums its stopping test needs (tested)
+    __device__ __forceinline__ void sweeps(Shared& sh, const int s_run, const bool tested, const bool owns) {
+        // the common full pass, unrolled: the values stay in their registers from sweep to sweep (a
+        // rolled loop makes the compiler rotate them through copies at every iteration); not for the
+        // FP64 shapes whose unrolled pass no longer fits the register budget of their wave count.
+        // A rollback or a budget-limited last launch takes the loop, which sums the FP64 norm in
+        // every sweep (the last one's stays).
+        // The waves that hold only halo rows (a quarter of them at 1024^2) run it without the FP64
+        // L1 sums, two of the point update's 14 instructions.
+        constexpr bool kUnroll = sizeof(T) == 4 || (S * RB <= 40 && NW != 12 && !(kNorm && S * RB > 20));
+        if (kUnroll && s_run == S) {
+            // FP32: an untested launch skips the last sweep's sums.  Small shapes get a pass of their
+            // own without them (6.10 against 6.29 us per launch at 1024^2 with (5, 16, 4)); large ones
+            // branch on the uniform flag in the last sweep, since a second unrolled pass of their
+            // size made the kernel slower (the batched (8, 8, 10) FP32 sweep 4.05 -> 4.7 us)
+            constexpr bool kSplit = sizeof(T) == 4 && S * RB <= 24;
+            if (kSplit && !tested) {
+#pragma unroll
+                for (int s = 0; s < S; ++s) sweep<false>(sh, s, false, s < S - 1);
+            } else if (owns || sizeof(T) == 4) {
+#pragma unroll
+                for (int s = 0; s < S; ++s) sweep<true>(sh, s, s == S - 1 && (kSplit || tested), s < S - 1);
+            } else {
+#pragma unroll
+                for (int s = 0; s < S; ++s) sweep<false>(sh, s, s == S - 1, s < S - 1);
+            }
+        } else {
+            for (int s = 0; s < s_run; ++s)
+                sweep<true>(sh, s, kLastOnly ? tested && s == s_run - 1 : kNorm, s < s_run - 1);
+        }
+    }
+    // the owned tile to plane dst; domain-boundary points hold +-0: store +0
+    __device__ __forceinline__ void store(const SorArgs<T>& a, T* __restrict__ dst) const {
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            const int li = row0 + r;
+            const int gi = gi0 + li;
+            if (li >= H && li < H + TI && gi < nr) {  // owned row (wave-uniform)
+                const bool rint = gi >= 1 && gi <= nr - 2;
+                // owned columns lie inside the row: 0 <= gj < nc
+                if (ownc[0])
+                    store_pair(dst + gi * (long long)a.ld, (unsigned)gj * sizeof(T), ownc[1], (rint && colin[0]) ? v[0][r] : T(0),
+                               (rint && colin[1]) ? v[1][r] : T(0));
+            }
+        }
+    }
+    // this wave's rows of the tile's per-sweep sums (the per-lane sums in lred, the norm in lnrm;
+    // wave w reduces rows w, w + NW, ..., each in a fixed order), handed to put(row, sum) by lane 0;
+    // row i < nupd is an update sum, row nupd the norm
+    template <typename Put>
+    __device__ __forceinline__ void reduce(const Shared& sh, const int nupd, Put put) const {
+        const int nrows = nupd + (kNorm ? 1 : 0);
+        for (int row = wv; row < nrows; row += NW) {
+            const double* col = row < nupd ? sh.lred[row] : sh.lnrm;
+            // the NW lane sums of this column, pairwise (depth log2 NW, not a chain of NW adds)
+            double t[NW];
+#pragma unroll
+            for (int j = 0; j < NW; ++j) t[j] = col[lane + 64 * j];
+#pragma unroll
+            for (int d = 1; d < NW; d *= 2)
+#pragma unroll
+                for (int j = 0; j + d < NW; j += 2 * d) t[j] += t[j + d];
+            const double acc = wave_sum(t[0]);
+            if (lane == 0) put(row, acc);
+        }
+    }
+};
+
+// One sweeping workgroup's launch on tile `tile` of the solve described by `a` (NW*64 threads).
+// It reads the state slot the previous launch's decider wrote: RUNNING -- sweep on from plane
+// L % NB (the previous launch's output) into plane (L+1) % NB, as many sweeps as the budget
+// leaves, and leave this tile's per-sweep L1 sums for the next launch's decider; ROLLBACK -- the
+// solve converged inside the launch before last: redo rb_n sweeps from plane rb_src into plane
+// `parity`, which then holds the final iterate; anything else -- the solve has ended: return.
+template <typename T, int S, int NW, int RB, bool GS, bool XR, bool NORM>
+__device__ __forceinline__ void sor_rb_sweeper(const SorArgs<T>& a, const int L, const int tile) {
+    typedef SorTile<T, S, NW, RB, GS, XR, NORM> Tile;
+    constexpr int NB = SorPlanes<T>::value;
+    __shared__ typename Tile::Shared sh;
+    const SorCtl* prev = a.ctl + ((L + 1) & 1);
+    const int ntiles = a.tiles_i * a.tiles_j;
+    const int ti = tile / a.tiles_j;
+    const int tj = tile - ti * a.tiles_j;
+    Tile t;
+    t.place(a, ti, tj);
+    // Speculative tile load for the common case (sweep on from the previous launch's output),
+    // issued before the state slot is read so that both are in flight together.
+    t.load(a, sor_plane(a, L % NB));
+
+    // what this launch does: the state after launch L-2 and the sweeps launch L-1 performed
+    const int pstatus = prev->status;
+    bool rollback = false;
+    int s_run = 0;
+    T* __restrict__ dst = nullptr;
+    if (pstatus == SOR_RUNNING) {
+        const int budget = prev->itmax - (prev->k + prev->s_done);
+        s_run = budget < S ? budget : S;
+        dst = sor_plane(a, (L + 1) % NB);
+    } else if (pstatus == SOR_ROLLBACK) {
+        rollback = true;
+        s_run = prev->rb_n;
+        dst = sor_plane(a, prev->parity);
+    }
+    if (s_run <= 0) return;  // the solve has ended, or its budget is spent
+    // FP32: whether this launch's last sweep is tested (FP64: every sweep of every launch)
+    const bool tested = sizeof(T) == 8 || (L & a.test_mask) == a.test_mask;
+    // the converged launch's input replaces the speculatively loaded tile
+    if (rollback) t.load_values(a, sor_plane(a, prev->rb_src));
+    t.fix_odd_edge();
+    const bool owns = t.owns_rows();
+    t.begin(sh);
+    t.sweeps(sh, s_run, tested, owns);
 
     // every wave's lane sums are in LDS; the stores below do not wait for this barrier's peers,
     // so the reducing waves start as soon as their own stores are issued
     if (!rollback && tested) __syncthreads();
-    // the owned tile to its plane; domain-boundary points hold +-0: store +0
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-        const int li = row0 + r;
-        const int gi = gi0 + li;
-        if (li >= H && li < H + TI && gi < nr) {  // owned row (wave-uniform)
-            const bool rint = gi >= 1 && gi <= nr - 2;
-            // owned columns lie inside the row: 0 <= gj < nc
-            if (ownc[0])
-                store_pair(dst + gi * ld, (unsigned)gj * sizeof(T), ownc[1], (rint && colin[0]) ? v[0][r] : T(0),
-                           (rint && colin[1]) ? v[1][r] : T(0));
-        }
-    }
+    t.store(a, dst);
     if (rollback || !tested) return;  // the final iterate, or an untested launch: no partials
 
-    // this tile's per-sweep partials (the per-lane sums in lred, the norm in lnrm) for the next
-    // launch's decider: wave w reduces rows w, w + NW, ..., each in a fixed order
-    const size_t pstride = (size_t)kMaxSweepsPerLaunch * ntiles * 2;
-    const int nupd = kLastOnly ? 1 : s_run;  // update rows (FP32: the last sweep's)
-    const int nrows = nupd + (kNorm ? 1 : 0);
-    for (int row = wv; row < nrows; row += NW) {
-        const double* col = row < nupd ? lred[row] : lnrm;
-        // the NW lane sums of this column, pairwise (depth log2 NW, not a chain of NW adds)
-        double t[NW];
-#pragma unroll
-        for (int j = 0; j < NW; ++j) t[j] = col[lane + 64 * j];
-#pragma unroll
-        for (int d = 1; d < NW; d *= 2)
-#pragma unroll
-            for (int j = 0; j + d < NW; j += 2 * d) t[j] += t[j + d];
-        const double acc = wave_sum(t[0]);
-        const size_t slot = row < nupd ? ((size_t)row * ntiles + tile) * 2 : (size_t)tile * 2 + 1;
-        if (lane == 0) a.partial[(L & 1) * pstride + slot] = acc;
-    }
+    // this tile's per-sweep partials for the next launch's decider (FP32: the last sweep's update)
+    double* part = a.partial + (L & 1) * ((size_t)kMaxSweepsPerLaunch * ntiles * 2);
+    const int nupd = Tile::kLastOnly ? 1 : s_run;
+    t.reduce(sh, nupd, [&](int row, double sum) {
+        part[row < nupd ? ((size_t)row * ntiles + tile) * 2 : (size_t)tile * 2 + 1] = sum;
+    });
 }
 
 // The deciding workgroup of launch L (NW*64 threads): decides on launch L-1's sweeps from their

@@ -108,6 +108,15 @@ __device__ inline void transport_fp64_at(const double* __restrict__ w, double* _
     wout[(size_t)i * ld + j] = (-uu * dwdx - vv * dwdy + rRe * (d2wdx2 + d2wdy2)) * dt + w[(size_t)i * ld + j];
 }
 
+// ---- what a resident solve finds at its start (all threads of the grid together) ------------
+__device__ inline void resident_reset_at(const ResidentReset& rr) {
+    if (!rr.base) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *rr.abort = 0;
+    const long long stride = (long long)gridDim.x * kBlock, total = rr.exch + rr.part + rr.zero;
+    for (long long q = (long long)blockIdx.x * kBlock + threadIdx.x; q < total; q += stride)
+        rr.base[q] = q < rr.exch ? rr.mark : (q < rr.exch + rr.part ? kMark64 : 0ull);
+}
+
 // ---- one state slot of a fresh solve (launch 0 reads slot 1; both are written) -------------
 __device__ inline void ctl_reset(SorCtl* sl, double tol, double rtol, int itmax) {
     sl->k = 0;

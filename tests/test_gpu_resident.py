@@ -1,0 +1,95 @@
+"""Resident Poisson solves (csrc/hip/sor_resident.h) against the oracle and against the same solves as
+launches: every tile shape at the edges of its range of grids, solves that end in the first
+epoch, inside an epoch, on its last sweep, on a spent budget, and from so far out that the tiles kept
+nothing to go back to; the refined form's inner solves; two solves at once from two threads."""
+import threading
+
+import numpy as np
+import pytest
+
+import cnv
+from oracle import orc
+
+pytestmark = pytest.mark.gpu
+
+
+def field(n, seed=3):
+    x = np.arange(n) / n
+    rng = np.random.default_rng(seed)
+    return np.sin(7 * x)[:, None] * np.cos(4 * x)[None, :] + 0.1 * rng.standard_normal((n, n))
+
+
+def check(n, f, beta, tol, itmax, ptype=2):
+    """One solve against the oracle: the iterate bit for bit, k, and the update to rounding."""
+    p = orc.make_params(n, tol=tol, itmax=itmax, ordering=orc.REDBLACK, beta_=beta, threads=8, poisson_type=ptype)
+    want, st = orc.poisson(p, f)
+    with cnv.Cavity(cnv.default_params(n, tol=tol, itmax=itmax, beta=beta, poisson_type=ptype)) as cav:
+        rc, psi, k, e = cav.poisson(f)
+    assert k == (st.k if rc == cnv.OK else itmax - 1), (n, k, st.k)  # the oracle logs no k for a failed solve
+    assert abs(e - st.e) <= 1e-12 * abs(st.e)
+    assert np.array_equal(psi, want)
+    return rc, k
+
+
+# sides around the largest grid of each tile shape (8 x 104, 12 x 108, 16 x 112, 24 x 104, 40 x 104,
+# 44 x 108 owned points, at most 32 tiles on each of 8 XCDs), the smallest grid, and beyond the last
+@pytest.mark.parametrize("n", [8, 9, 64, 97, 104, 105, 416, 417, 432, 512, 540, 541, 560, 672, 673, 728, 960, 1000,
+                               1001, 1055, 1056, 1057])
+def test_solves_equal_the_oracle(n):
+    f = field(n)
+    e = [orc.poisson(orc.make_params(n, tol=-1.0, itmax=s, ordering=orc.REDBLACK, beta_=0.9, threads=8), f)[1].e
+         for s in (1, 17, 24)]
+    for tol in (2 * e[0], e[1] * (1 + 1e-9), e[2] * (1 + 1e-9)):  # the first sweep, inside an epoch, and later
+        assert check(n, f, 0.9, tol, 1000)[0] == cnv.OK
+    assert check(n, f, 0.9, -1.0, 23)[0] == cnv.NOT_CONVERGED  # a budget that ends inside an epoch
+    assert check(n, f, 1.0, e[1], 1000, ptype=1)[0] == cnv.OK
+
+
+@pytest.mark.parametrize("n", [300, 600, 1024])
+def test_solve_that_ends_from_far_out(n):
+    # a short-wave source under weak relaxation: its update falls about twofold a sweep, so when it
+    # crosses the tolerance the tiles held in device memory have kept no epoch's start
+    i, j = np.indices((n, n))
+    f = np.sin(2 * np.pi * i / 5) * np.sin(2 * np.pi * j / 5)
+    e = {s: orc.poisson(orc.make_params(n, tol=-1.0, itmax=s, ordering=orc.REDBLACK, beta_=0.6, threads=8), f)[1].e
+         for s in (4, 13, 15, 16, 17, 18, 20, 21)}
+    assert e[4] > 50 * e[13]
+    for s, v in e.items():
+        assert check(n, f, 0.6, v * (1 + 1e-9), 1000)[1] == s - 1
+
+
+@pytest.mark.parametrize("n,launches", [(64, (5, 8, 8)), (257, (5, 8, 8)), (600, (6, 8, 8)), (900, (6, 8, 8)),
+                                        (1030, (5, 8, 8))])
+def test_refined_equals_launches(n, launches):
+    # the named shape is compiled for launches only; the sweeps and their order are the same
+    kw = dict(precision=cnv.PREC_FP32_DC, Re=400.0, dt=1e-5, tol=1e-8, itmax=100000)
+    out = []
+    for shape in ({}, dict(zip(("sweeps_per_launch", "tile_waves", "wave_rows"), launches))):
+        with cnv.Cavity(cnv.default_params(n, **kw, **shape)) as cav:
+            st = cav.step(2)
+            out.append(([(s.status, s.sweeps, s.outer) for s in st], cav.get_state()))
+    assert out[0][0] == out[1][0]
+    for name in ("w", "psi", "u", "v"):
+        assert np.array_equal(out[0][1][name], out[1][1][name]), name
+
+
+def test_two_solves_at_once():
+    n, f = 1024, field(1024)
+    kw = dict(tol=1e-4, itmax=100000, beta=1.9)
+    with cnv.Cavity(cnv.default_params(n, **kw)) as cav:
+        alone = cav.poisson(f)
+    got = {}
+
+    def work(name):
+        with cnv.Cavity(cnv.default_params(n, **kw)) as cav:
+            got[name] = [cav.poisson(f) for _ in range(3)]
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for t in range(2):
+        for rc, psi, k, e in got[t]:
+            assert (rc, k) == (alone[0], alone[2]) and abs(e - alone[3]) <= 1e-12 * e
+            assert np.array_equal(psi, alone[1])
