@@ -12,6 +12,17 @@
 
 constexpr int kSlots = 4;  // pinned copies of the control block in flight
 
+// How a grid's solves run resident: tile shape, launch arguments, memory (resident.hip).
+struct ResidentPlan {
+    cnv::TileShape shape{5, 16, 4};
+    int tiles_i = 0, tiles_j = 0;
+    int units = 0;             // CUs per XCD it holds while it runs
+    long long words = 0;       // 64-bit words of exchange planes, partial sums, decision words, counters
+    long long snap = 0;        // doubles of kept epoch starts (0: none, or in LDS)
+    cnv::SorResident r{};
+    cnv::ResidentReset reset{};
+};
+
 struct cnv_ctx {
     cnv_params p;
     int n, ld;
@@ -62,15 +73,11 @@ struct cnv_ctx {
     hipGraphExec_t g_resid[2] = {nullptr, nullptr};
     hipGraphExec_t g_correct = nullptr;
     hipGraphExec_t g_post = nullptr;
-    // resident solves (sor_resident.h): usable, their memory and arguments, CUs they need (resident.hip)
+    // resident solves (sor_resident.h, resident.hip): usable, their plan and memory
     bool res_on = false;
+    ResidentPlan res;
     unsigned long long* d_res = nullptr;
     double* d_res_snap = nullptr;
-    cnv::SorResident res{};
-    cnv::ResidentReset res_reset{};
-    int res_units = 0;
-    cnv::TileShape res_shape{5, 16, 4};
-    int res_tiles_i = 0, res_tiles_j = 0;
     int* d_budget = nullptr;  // refined form, captured: the solve's remaining sweep budget
     // output snapshots (cnv_snapshot_begin/wait): a device copy of (w, psi, u, v) taken in stream
     // order, then transferred to pinned host memory on a stream of its own
@@ -244,10 +251,24 @@ inline int run_sor_launches(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* f
 }
 
 // ---- resident solves (resident.hip) -----------------------------------------------------------
+// The plan for n x n grids on a device; base: the launches' shape, named: the caller chose it (then
+// that one or none; else an FP32 solve keeps its sweeps per launch).  false: they run as launches.
+bool resident_plan(int n, bool fp64, int dev, cnv::TileShape base, bool named, ResidentPlan* p);
+// Gives a plan its memory: words and snap as it says, the solve's slots (the abort flag after them).
+void resident_bind(ResidentPlan* p, unsigned long long* words, double* snap, cnv::SorCtl* ctl);
+// Takes a plan's share of the device for the time of a solve (false: not now).
+bool resident_enter(int dev, int units);
+void resident_leave(int dev, int units);
+// The kernels of one solve, between the two calls above, on fresh slots and reset memory.  h: three
+// slots of host memory.  *resume < 0: it has ended (*fin, in slot *fin_slot), else the launch index
+// to go on from as launches (a wave gave up waiting).
+template <typename T>
+int resident_chunks(cnv_ctx* c, const ResidentPlan& p, cnv::SorArgs<T> a, bool gs, int itmax, hipStream_t st,
+                    cnv::SorCtl* h, cnv::SorCtl* fin, int* fin_slot, int* resume);
 // Sets up the context's resident solves where its grid and the device allow them.
 int resident_setup(cnv_ctx* c);
 // What the init kernels reset for a solve that may run resident.
-inline cnv::ResidentReset resident_reset_of(const cnv_ctx* c) { return c->res_on ? c->res_reset : cnv::ResidentReset{}; }
+inline cnv::ResidentReset resident_reset_of(const cnv_ctx* c) { return c->res_on ? c->res.reset : cnv::ResidentReset{}; }
 // The solve as resident kernels when they can run now (*ran = false: nothing was done).
 template <typename T>
 int run_sor_resident(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* final_ctl, bool* ran);

@@ -1,8 +1,8 @@
 // noalloc.hip -- the Poisson solve of cnv_poisson_device without a context and without any
 // device allocation (include/cnv.h: cnv_poisson_device_noalloc).
 //
-// The solve's scratch -- the second and third SOR iterate planes, the per-tile L1 partial sums and
-// the two state slots -- lives in `scratch`, a file-scope device array of the library
+// The solve's scratch -- the second and third SOR iterate planes, the per-tile L1 partial sums, the
+// state slots and the memory of a resident solve (sor_resident.h) -- lives in `scratch`, a file-scope device array of the library
 // sized for grids up to kNoAllocMaxN per side; each GPU the library runs on holds its own copy
 // until the process ends.  Host code never passes the array's name to a kernel (on the host it
 // is only a stand-in for the symbol): the first call on each device, with that device current,
@@ -30,8 +30,12 @@ constexpr size_t kIterDoubles = 2 * kPlaneDoubles;  // planes 1 and 2 (plane 0 i
 // tiles of the thinnest compiled default tile (4 x 108 owned points) at the largest side
 constexpr size_t kMaxTiles = 2560;
 constexpr size_t kPartialDoubles = (size_t)2 * 2 * kMaxSweepsPerLaunch * kMaxTiles;
-constexpr size_t kCtlDoubles = 2 * sizeof(SorCtl) / sizeof(double);
-constexpr size_t kScratchDoubles = kIterDoubles + kPartialDoubles + kCtlDoubles;
+constexpr size_t kCtlDoubles = 4 * sizeof(SorCtl) / sizeof(double);  // two slots, the abort flag
+// a resident solve: three exchange planes, partial sums and words of at most 256 tiles, and two
+// copies of each extended tile of at most 64 x 128 points
+constexpr size_t kResidentWords = 3 * (size_t)(kNoAllocMaxN + 32) * kNoAllocMaxN + 256 * (4 * kResidentRows + 8) + 1024;
+constexpr size_t kSnapDoubles = 2 * (size_t)256 * 64 * 128;
+constexpr size_t kScratchDoubles = kIterDoubles + kPartialDoubles + kCtlDoubles + kResidentWords + kSnapDoubles;
 static_assert(sizeof(SorCtl) % sizeof(double) == 0, "state slots pack into doubles");
 static_assert(((kIterDoubles + kPartialDoubles) * sizeof(double)) % 256 == 0, "slots stay 256-byte aligned");
 
@@ -92,23 +96,41 @@ int cnv_poisson_device_noalloc(int n, double dx, double dy, double beta, double 
     double* partial = base + kIterDoubles;
     SorCtl* ctl = reinterpret_cast<SorCtl*>(base + kIterDoubles + kPartialDoubles);
     hipStream_t st = nullptr;  // the null stream
-    if (poisson_init_launch(d_psi, ctl, nullptr, n, n, tol, itmax, st))
+    ResidentPlan plan;
+    bool resident = resident_plan(n, true, dev, sh, false, &plan) && plan.words <= (long long)kResidentWords &&
+                    plan.snap <= (long long)kSnapDoubles && resident_enter(dev, plan.units);
+    if (resident) {
+        double* const words = base + kIterDoubles + kPartialDoubles + kCtlDoubles;
+        resident_bind(&plan, reinterpret_cast<unsigned long long*>(words), words + kResidentWords, ctl);
+    }
+    if (poisson_init_launch(d_psi, ctl, nullptr, n, n, tol, itmax, st, 1, resident ? plan.reset : ResidentReset{})) {
+        if (resident) resident_leave(dev, plan.units);
         return cnv_fail(nullptr, CNV_ERR_HIP, "Poisson init launch failed: %s", hipGetErrorString(hipGetLastError()));
+    }
     SorArgs<double> a = sor_args_for<double>(n, n, dx, dy, beta, ti, tj, partial, ctl, d_f, d_psi, psi1, psi2, 0);
     const bool gs = poisson_type == 1;
     const long long cap = (long long)itmax / sh.s + 4LL * kLaunchesPerPoll + 8;  // working launches <= itmax/S + 3
     long long queued = 0;
     SorCtl fin{};
-    while (true) {
+    int resume = 0;  // launch index to go on from; < 0: the solve has ended
+    if (resident) {
+        SorCtl h[3];
+        int slot = 0;
+        rc = resident_chunks<double>(nullptr, plan, a, gs, itmax, st, h, &fin, &slot, &resume);
+        if (rc) (void)hipStreamSynchronize(st);
+        resident_leave(dev, plan.units);
+        if (rc) return rc;
+    }
+    while (resume >= 0) {
         for (int l = 0; l < kLaunchesPerPoll; ++l) {
-            a.launch = (int)(queued + l);
+            a.launch = resume + (int)(queued + l);
             if (sor_fp64_launch(a, sh, gs, st))
                 return cnv_fail(nullptr, CNV_ERR_HIP, "SOR launch failed: %s", hipGetErrorString(hipGetLastError()));
         }
         queued += kLaunchesPerPoll;
         // the slot the last queued launch wrote; a copy into pageable host memory returns when the
         // launches before it have run
-        const hipError_t ec = hipMemcpyAsync(&fin, ctl + ((queued - 1) & 1), sizeof(SorCtl), hipMemcpyDeviceToHost, st);
+        const hipError_t ec = hipMemcpyAsync(&fin, ctl + ((resume + queued - 1) & 1), sizeof(SorCtl), hipMemcpyDeviceToHost, st);
         if (ec != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
             return cnv_fail(nullptr, CNV_ERR_HIP, "reading the SOR state failed: %s", hipGetErrorString(hipGetLastError()));
         if (sor_done(fin.status)) break;

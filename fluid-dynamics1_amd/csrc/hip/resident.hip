@@ -41,10 +41,8 @@ std::atomic<int> g_units[kMaxDevices];  // CUs per XCD in use by resident solves
 // sor_rb.h the default shapes took 1.27 us at 64^2, 1.34 at 257^2 and 2.0 at 1024^2.
 constexpr TileShape kShapes[] = {{6, 16, 2}, {5, 16, 2}, {4, 16, 2}, {6, 12, 4}, {6, 16, 4}, {5, 16, 4}};
 
-}  // namespace
-
 // Workgroups per XCD of a resident solve with tiles of shape sh (0: they do not fit together).
-static int resident_slots(int n, TileShape sh, int per_xcd, SorResident* r) {
+int resident_slots(int n, TileShape sh, int per_xcd, SorResident* r) {
     const int ti = (n + tile_rows(sh) - 1) / tile_rows(sh), tj = (n + tile_cols(sh) - 1) / tile_cols(sh);
     // every XCD gets as many workgroups as the largest band has tiles, or one of them one more: a
     // workgroup without a tile decides
@@ -57,135 +55,151 @@ static int resident_slots(int n, TileShape sh, int per_xcd, SorResident* r) {
     return slots <= (sh.nw > 4 ? per_xcd : 2 * per_xcd) ? slots : 0;
 }
 
-int resident_setup(cnv_ctx* c) {
-    const int dev = c->p.device;
+int cus_per_xcd(int dev) {
     int cus = 0;
-    if (dev >= kMaxDevices || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus < 8 * kBands)
-        return CNV_OK;
-    const int per_xcd = cus / kBands;
-    const bool fp64 = c->p.precision == CNV_PREC_FP64;
-    SorResident& r = c->res;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    return cus / kBands;
+}
+
+int launch_resident(const SorArgs<double>& a, const SorResident& r, TileShape sh, bool gs, hipStream_t st) {
+    return sor_fp64_resident(a, r, sh, gs, st);
+}
+int launch_resident(const SorArgs<float>& a, const SorResident& r, TileShape sh, bool gs, hipStream_t st) {
+    return sor_fp32_resident(a, r, sh, gs, st);
+}
+
+}  // namespace
+
+bool resident_plan(int n, bool fp64, int dev, TileShape base, bool named, ResidentPlan* p) {
+    const int per_xcd = dev < kMaxDevices ? cus_per_xcd(dev) : 0;
+    if (per_xcd < 8) return false;
+    *p = ResidentPlan{};
+    SorResident& r = p->r;
     int slots = 0;
-    const bool named = c->p.sweeps_per_launch > 0 || c->p.tile_waves > 0 || c->p.wave_rows > 0;
     if (named) {
-        c->res_shape = c->shape;
-        if (sor_resident_supported(c->shape)) slots = resident_slots(c->n, c->shape, per_xcd, &r);
+        p->shape = base;
+        if (sor_resident_supported(base)) slots = resident_slots(n, base, per_xcd, &r);
     } else {
         for (const TileShape& sh : kShapes) {
-            if (!fp64 && sh.s != c->shape.s) continue;
-            c->res_shape = sh;
-            slots = resident_slots(c->n, sh, per_xcd, &r);
+            if (!fp64 && sh.s != base.s) continue;
+            p->shape = sh;
+            slots = resident_slots(n, sh, per_xcd, &r);
             if (slots) break;
         }
     }
-    if (!slots) return CNV_OK;
-    const TileShape sh = c->res_shape;
-    c->res_tiles_i = (c->n + tile_rows(sh) - 1) / tile_rows(sh);
-    c->res_tiles_j = (c->n + tile_cols(sh) - 1) / tile_cols(sh);
-    c->res_units = std::min(slots, per_xcd);
+    if (!slots) return false;
+    const TileShape sh = p->shape;
+    p->tiles_i = (n + tile_rows(sh) - 1) / tile_rows(sh);
+    p->tiles_j = (n + tile_cols(sh) - 1) / tile_cols(sh);
+    p->units = std::min(slots, per_xcd);
     // exchange rows start on 128-byte lines: rows of two bands share none
-    r.ldx = (c->n + 1 + 31) / 32 * 32;
-    r.xplane = (long long)r.ldx * c->n;
-    ResidentReset& rr = c->res_reset;
+    r.ldx = (n + 1 + 31) / 32 * 32;
+    r.xplane = (long long)r.ldx * n;
+    r.epochs = kEpochs;
+    ResidentReset& rr = p->reset;
     rr.exch = 3 * r.xplane / (fp64 ? 1 : 2);
     rr.part = 4LL * r.ntiles * kResidentRows;
-    const long long words = 8LL * r.ntiles;  // decision words
-    rr.zero = words + (kBands + 1) * kClaimStride / 2;
+    rr.zero = 8LL * r.ntiles + (kBands + 1) * kClaimStride / 2;  // decision words, counters
     rr.mark = fp64 ? kMark64 : ((unsigned long long)kMark32 << 32 | kMark32);
-    rr.abort = reinterpret_cast<int*>(c->ctl + 2);
-    HIPC(c, hipMalloc(&c->d_res, sizeof(*c->d_res) * (rr.exch + rr.part + rr.zero)));
-    rr.base = c->d_res;
-    r.exch = c->d_res;
-    r.part = reinterpret_cast<double*>(c->d_res + rr.exch);
-    r.dec = c->d_res + rr.exch + rr.part;
-    r.claim = reinterpret_cast<int*>(r.dec + words);
+    p->words = rr.exch + rr.part + rr.zero;
+    p->snap = fp64 && !resident_snap_lds(sh.nw, sh.rb) ? 2LL * r.ntiles * sh.nw * sh.rb * 128 : 0;
+    return true;
+}
+
+void resident_bind(ResidentPlan* p, unsigned long long* words, double* snap, SorCtl* ctl) {
+    ResidentReset& rr = p->reset;
+    rr.base = words;
+    rr.abort = reinterpret_cast<int*>(ctl + 2);
+    SorResident& r = p->r;
+    r.exch = words;
+    r.part = reinterpret_cast<double*>(words + rr.exch);
+    r.dec = words + rr.exch + rr.part;
+    r.claim = reinterpret_cast<int*>(r.dec + 8LL * r.ntiles);
+    r.snap = snap;
     r.abort = rr.abort;
-    if (fp64 && !resident_snap_lds(sh.nw, sh.rb)) {
-        HIPC(c, hipMalloc(&c->d_res_snap, sizeof(double) * 2 * (size_t)r.ntiles * sh.nw * sh.rb * 128));
-        r.snap = c->d_res_snap;
-    }
-    r.epochs = kEpochs;
+}
+
+int resident_setup(cnv_ctx* c) {
+    const bool named = c->p.sweeps_per_launch > 0 || c->p.tile_waves > 0 || c->p.wave_rows > 0;
+    ResidentPlan p;
+    if (!resident_plan(c->n, c->p.precision == CNV_PREC_FP64, c->p.device, c->shape, named, &p)) return CNV_OK;
+    HIPC(c, hipMalloc(&c->d_res, sizeof(*c->d_res) * p.words));
+    if (p.snap) HIPC(c, hipMalloc(&c->d_res_snap, sizeof(double) * p.snap));
+    resident_bind(&p, c->d_res, c->d_res_snap, c->ctl);
+    c->res = p;
     c->res_on = true;
     return CNV_OK;
 }
 
-static int resident_launch(cnv_ctx* c, SorArgs<double> a, const SorResident& r, bool gs) {
-    a.tiles_i = c->res_tiles_i;
-    a.tiles_j = c->res_tiles_j;
-    return sor_fp64_resident(a, r, c->res_shape, gs, c->stream);
+bool resident_enter(int dev, int units) {
+    std::atomic<int>& used = g_units[dev];
+    if (used.fetch_add(units) + units <= cus_per_xcd(dev)) return true;
+    used.fetch_sub(units);
+    return false;
 }
-static int resident_launch(cnv_ctx* c, SorArgs<float> a, const SorResident& r, bool gs) {
-    a.tiles_i = c->res_tiles_i;
-    a.tiles_j = c->res_tiles_j;
-    return sor_fp32_resident(a, r, c->res_shape, gs, c->stream);
-}
+void resident_leave(int dev, int units) { g_units[dev].fetch_sub(units); }
 
-// The chunks of a solve; *resume < 0 when it has ended, else the launch index to go on from (a
-// wave of the last chunk gave up waiting: its input is where that launch reads).
 template <typename T>
-static int resident_chunks(cnv_ctx* c, const SorArgs<T>& a, SorCtl* final_ctl, int* resume) {
+int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, int itmax, hipStream_t st, SorCtl* h,
+                    SorCtl* fin, int* fin_slot, int* resume) {
     constexpr int NB = SorPlanes<T>::value;
-    const bool gs = c->p.poisson_type == 1;
-    SorResident r = c->res;
+    SorResident r = p.r;
+    a.tiles_i = p.tiles_i;
+    a.tiles_j = p.tiles_j;
     r.launch0 = 0;
     r.stop = 0;
     r.src = 0;
     r.rslot = 0;
     *resume = -1;
-    const long long most = (long long)c->p.itmax / c->res_shape.s + 2LL * kEpochs;  // epochs of a whole budget
+    const long long most = (long long)itmax / p.shape.s + 2LL * kEpochs;  // epochs of a whole budget
     while (r.launch0 <= most) {
         r.dst = (r.src + 1) % NB;
         r.wslot = r.rslot ^ 1;
-        LAUNCH(c, resident_launch(c, a, r, gs));
-        HIPC(c, hipMemcpyAsync(c->h_ctl, c->ctl, 3 * sizeof(SorCtl), hipMemcpyDeviceToHost, c->stream));
-        HIPC(c, hipStreamSynchronize(c->stream));
+        LAUNCH(c, launch_resident(a, r, p.shape, gs, st));
+        HIPC(c, hipMemcpyAsync(h, a.ctl, 3 * sizeof(SorCtl), hipMemcpyDeviceToHost, st));
+        HIPC(c, hipStreamSynchronize(st));
         int aborted = 0;
-        memcpy(&aborted, &c->h_ctl[2], sizeof(aborted));
+        memcpy(&aborted, h + 2, sizeof(aborted));
         if (aborted) {
             // both slots as the chunk found them; FP32 planes: into plane 0, where launch 0 reads
-            HIPC(c, hipMemcpyAsync(c->ctl + r.wslot, c->ctl + r.rslot, sizeof(SorCtl), hipMemcpyDeviceToDevice, c->stream));
+            HIPC(c, hipMemcpyAsync(a.ctl + r.wslot, a.ctl + r.rslot, sizeof(SorCtl), hipMemcpyDeviceToDevice, st));
             if (NB == 2 && r.src == 1)
-                HIPC(c, hipMemcpyAsync(a.psi0, a.psi1, sizeof(T) * c->cells, hipMemcpyDeviceToDevice, c->stream));
+                HIPC(c, hipMemcpyAsync(a.psi0, a.psi1, sizeof(T) * (size_t)a.nr * a.ld, hipMemcpyDeviceToDevice, st));
             *resume = NB == 2 ? 0 : r.src;
             return CNV_OK;
         }
-        const SorCtl st = c->h_ctl[r.wslot];
-        if (sor_done(st.status) && st.rb_n == kNotStored && r.stop == 0) {
-            r.stop = st.k;  // once more, to exactly the sweep the solve ended with
-            LAUNCH(c, resident_reset_launch(c->res_reset, c->stream));
-            continue;
+        const SorCtl s = h[r.wslot];
+        if (sor_done(s.status)) {
+            if (s.rb_n != kNotStored || r.stop > 0) {
+                *fin = s;
+                *fin_slot = r.wslot;
+                return CNV_OK;
+            }
+            r.stop = s.k;  // once more, to exactly the sweep the solve ended with
+        } else {
+            r.src = r.dst;
+            r.rslot = r.wslot;
+            r.launch0 += kEpochs;
         }
-        if (sor_done(st.status)) {
-            *final_ctl = st;
-            c->fin_slot = r.wslot;
-            return CNV_OK;
-        }
-        LAUNCH(c, resident_reset_launch(c->res_reset, c->stream));
-        r.src = r.dst;
-        r.rslot = r.wslot;
-        r.launch0 += kEpochs;
+        LAUNCH(c, resident_reset_launch(p.reset, st));
     }
     return cnv_fail(c, CNV_ERR_HIP, "SOR state did not terminate after %d epochs", r.launch0);
 }
+template int resident_chunks<double>(cnv_ctx*, const ResidentPlan&, SorArgs<double>, bool, int, hipStream_t, SorCtl*,
+                                     SorCtl*, int*, int*);
 
 template <typename T>
 int run_sor_resident(cnv_ctx* c, const SorArgs<T>& a, SorCtl* final_ctl, bool* ran) {
-    *ran = false;
-    if (!c->res_on) return CNV_OK;
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->p.device) != hipSuccess) return CNV_OK;
-    std::atomic<int>& used = g_units[c->p.device];
-    if (used.fetch_add(c->res_units) + c->res_units > cus / kBands) {
-        used.fetch_sub(c->res_units);
-        return CNV_OK;  // other resident solves are running: this one runs as launches
-    }
-    *ran = true;
+    const int dev = c->p.device;
+    // with other resident solves running that leave too few CUs, this one runs as launches
+    *ran = c->res_on && resident_enter(dev, c->res.units);
+    if (!*ran) return CNV_OK;
     int resume = -1;
-    const int rc = resident_chunks<T>(c, a, final_ctl, &resume);
+    const int rc = resident_chunks<T>(c, c->res, a, c->p.poisson_type == 1, c->p.itmax, c->stream, c->h_ctl, final_ctl,
+                                      &c->fin_slot, &resume);
     // a failed call may leave its kernel running, which holds its place until it has ended
     if (rc) (void)hipStreamSynchronize(c->stream);
-    used.fetch_sub(c->res_units);
+    resident_leave(dev, c->res.units);
     if (rc || resume < 0) return rc;
     c->res_on = false;
     return run_sor_launches<T>(c, a, final_ctl, resume);

@@ -173,9 +173,9 @@ int cnv_poisson_device(cnv_ctx *ctx, const double *d_f, double *d_psi, int *k, d
  * n*n doubles (psi is written; f is read only).  Runs on the null stream of the current device
  * and returns when psi is complete; f must be complete when it is called (work queued on a
  * non-blocking stream is not waited for).  The solve's scratch (the second and third iterate
- * planes, the per-tile partial sums, the state slots) is a static device array of the library,
- * sized for n <= CNV_NOALLOC_MAX_N (about 17 MB, held on each device the library runs on until
- * the process ends); larger n is refused with CNV_ERR_ARG.  Calls that overlap on one device
+ * planes, the per-tile partial sums, the state slots, the exchange planes and kept values of a
+ * resident solve) is a static device array of the library, sized for n <= CNV_NOALLOC_MAX_N
+ * (about 77 MB, held on each device the library runs on until the process ends); larger n is refused with CNV_ERR_ARG.  Calls that overlap on one device
  * share that array and race.  Results, k and e equal cnv_poisson_device's on a context created
  * with the same n, dx, dy, beta, tol, itmax, poisson_type and the default launch shape. */
 #define CNV_NOALLOC_MAX_N 1024

@@ -2,6 +2,7 @@
 launches: every tile shape at the edges of its range of grids, solves that end in the first
 epoch, inside an epoch, on its last sweep, on a spent budget, and from so far out that the tiles kept
 nothing to go back to; the refined form's inner solves; two solves at once from two threads."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -71,6 +72,20 @@ def test_refined_equals_launches(n, launches):
     assert out[0][0] == out[1][0]
     for name in ("w", "psi", "u", "v"):
         assert np.array_equal(out[0][1][name], out[1][1][name]), name
+
+
+@pytest.mark.parametrize("n", [8, 65, 417, 600, 1001, 1024])
+def test_noalloc_equals_context(n):
+    f = field(n)
+    with cnv.Cavity(cnv.default_params(n, tol=1e-3, itmax=100000, beta=1.5)) as cav:
+        rc, psi, k, e = cav.poisson(f)
+        cav.set_state(w=f)
+        dw, du = C.c_void_p(), C.c_void_p()
+        cnv._check(cnv.lib().cnv_device_state(cav.h, C.byref(dw), None, C.byref(du), None), cav.h)
+        k2, e2 = C.c_int(), C.c_double()
+        assert cnv.lib().cnv_poisson_device_noalloc(n, 1.0 / n, 1.0 / n, 1.5, 1e-3, 100000, 2, dw, du, C.byref(k2),
+                                                    C.byref(e2)) == rc  # the larger grids run out of sweeps
+        assert (k, e) == (k2.value, e2.value) and np.array_equal(cav.get_state()["u"], psi)
 
 
 def test_two_solves_at_once():
