@@ -151,6 +151,17 @@ struct ResidentReset {
     int* abort;
 };
 
+// The start of a Poisson solve, made by the transport launch before it (psi0 == nullptr: none).
+struct SolveInit {
+    double* psi0;     // zeroed unless keep (the refined form's accumulator, kept by a warm start)
+    SorCtl* ctl;      // both slots
+    Diag* diag;
+    int* budget;      // refined form: the solve's sweep budget
+    double tol;
+    int itmax, keep;
+    ResidentReset rr;
+};
+
 // Batched SOR launch: workgroup -> (solve, tile); inst < 0 marks padding workgroups, tile ==
 // the solve's tile count its deciding workgroup.
 struct SorBlock {
@@ -180,10 +191,11 @@ int wall_vorticity_launch(double* w, const double* u, const double* v, int n, in
                           const Stencils& s, const WallBC& bc, hipStream_t st);
 int transport_fp64_launch(const double* w_in, double* w_out, const double* u, const double* v,
                           int n, int ld, const Stencils& s, const WallBC& bc, double rRe,
-                          double dt, hipStream_t st);
+                          double dt, hipStream_t st, const SolveInit& si = SolveInit{});
 int transport_fp32_launch(const double* w_in, double* w_out, const double* u, const double* v,
                           int n, int ld, const Stencils& s, const WallBC& bc, double rRe,
-                          double dt, hipStream_t st);
+                          double dt, hipStream_t st, const SolveInit& si = SolveInit{});
+int diag_reset_launch(Diag* diag, hipStream_t st);
 // zero = 0 keeps psi0 (warm start) and only resets the state slots and the diagnostic
 int poisson_init_launch(double* psi0, SorCtl* ctl, Diag* diag, int n, int ld, double tol,
                         int itmax, hipStream_t st, int zero = 1, const ResidentReset& rr = ResidentReset{});
@@ -206,15 +218,15 @@ int snapshot_launch(const double* w, const Planes& psi, const double* u, const d
 // refined-form velocities from psi with FP32 stencils
 int velocity_fp32_launch(const double* psi, double* u, double* v, int n, int ld, const Stencils& s,
                          hipStream_t st);
+// go != nullptr: do nothing unless *go (the inner solve before was added to psi)
 int dc_residual_launch(const double* w, const double* psi, float* r32, int n, int ld, double c1,
-                       double c2, double c3, double B, hipStream_t st);
-int dc_correct_launch(double* psi, const float* e0, const float* e1, const SorCtl* fin, int n,
-                      int ld, hipStream_t st);
-// budget != nullptr: the inner solve's sweep budget is read from that device counter
-int dc_inner_init_launch(float* e0, SorCtl* ctl, int n, int ld, double rtol, double tol,
-                         int itmax, hipStream_t st, const int* budget = nullptr,
-                         const ResidentReset& rr = ResidentReset{});
-// the device budget counter: fin == nullptr sets it to itmax, else subtracts fin->k
-int dc_budget_launch(int* budget, int itmax, const SorCtl* fin, hipStream_t st);
+                       double c2, double c3, double B, hipStream_t st, const int* go = nullptr);
+// psi += e and *budget -= the inner solve's sweeps, if that solve (slot fin) has ended; *go says so
+int dc_correct_launch(double* psi, const float* e0, const float* e1, const SorCtl* fin, const int* abort,
+                      int* budget, int* go, int n, int ld, hipStream_t st);
+// the inner solve's sweep budget: *budget, or itmax without one
+int dc_inner_init_launch(float* e0, SorCtl* ctl, int n, int ld, double rtol, double tol, int itmax, hipStream_t st,
+                         const int* budget = nullptr, const ResidentReset& rr = ResidentReset{},
+                         const int* go = nullptr);
 
 }  // namespace cnv

@@ -281,12 +281,11 @@ void cnv_destroy(cnv_ctx* c) {
     if (c->snap_stream) (void)hipStreamSynchronize(c->snap_stream);
     drop_graphs(c);
     void* dev[] = {c->w[0], c->w[1], c->psi[0], c->psi[1], c->psi[2], c->u, c->v, c->d_start, c->d_tab, c->d_ftab,
-                   c->ctl, c->diag, c->partial, c->e32[0], c->e32[1], c->r32, c->d_budget, c->d_snap,
+                   c->ctl, c->partial, c->e32[0], c->e32[1], c->r32, c->d_budget, c->d_snap,
                    c->d_res, c->d_res_snap};
     for (void* p : dev)
         if (p) (void)hipFree(p);
     if (c->h_ctl) (void)hipHostFree(c->h_ctl);
-    if (c->h_diag) (void)hipHostFree(c->h_diag);
     if (c->h_snap) (void)hipHostFree(c->h_snap);
     if (c->ev_snap_ready) (void)hipEventDestroy(c->ev_snap_ready);
     if (c->ev_snap_done) (void)hipEventDestroy(c->ev_snap_done);
@@ -358,20 +357,19 @@ int cnv_create_ctx(const cnv_params* p, cnv_ctx** out, bool resident) {
         for (int b = 0; b < 3; ++b) HIPC(c, hipMalloc(&c->psi[b], bytes));
         HIPC(c, hipMalloc(&c->u, bytes));
         HIPC(c, hipMalloc(&c->v, bytes));
-        HIPC(c, hipMalloc(&c->ctl, 3 * sizeof(SorCtl)));
-        HIPC(c, hipMalloc(&c->diag, sizeof(Diag)));
-        HIPC(c, hipMemset(c->ctl, 0, 3 * sizeof(SorCtl)));
-        HIPC(c, hipMemset(c->diag, 0, sizeof(Diag)));
+        static_assert(sizeof(Diag) <= sizeof(SorCtl), "the diagnostic takes the fourth slot");
+        HIPC(c, hipMalloc(&c->ctl, kSlots * sizeof(SorCtl)));
+        HIPC(c, hipMemset(c->ctl, 0, kSlots * sizeof(SorCtl)));
+        c->diag = reinterpret_cast<Diag*>(c->ctl + 3);
         HIPC(c, hipMalloc(&c->partial, sizeof(double) * 2 * 2 * kMaxSweepsPerLaunch * (size_t)c->tiles_i * c->tiles_j));
         HIPC(c, hipHostMalloc(&c->h_ctl, sizeof(SorCtl) * kSlots, hipHostMallocDefault));
-        HIPC(c, hipHostMalloc(&c->h_diag, sizeof(Diag), hipHostMallocDefault));
         for (int s = 0; s < kSlots; ++s) HIPC(c, hipEventCreateWithFlags(&c->ev[s], hipEventDisableTiming));
         HIPC(c, hipEventCreate(&c->t0));
         HIPC(c, hipEventCreate(&c->t1));
         if (p->precision == CNV_PREC_FP32_DC) {
             for (int b = 0; b < 2; ++b) HIPC(c, hipMalloc(&c->e32[b], sizeof(float) * c->cells));
             HIPC(c, hipMalloc(&c->r32, sizeof(float) * c->cells));
-            HIPC(c, hipMalloc(&c->d_budget, sizeof(int)));
+            HIPC(c, hipMalloc(&c->d_budget, 2 * sizeof(int)));
         }
         int rc = upload_tables(c);
         if (!rc && resident) rc = resident_setup(c);
@@ -405,38 +403,6 @@ static int poisson_fp64(cnv_ctx* c, const double* f_src, int negate, SorCtl* fin
     return CNV_OK;
 }
 
-// defect correction: psi[0] accumulates in FP64, e32 ping-pong holds the inner FP32 iterates
-static int poisson_dc(cnv_ctx* c, const double* w_src, SorCtl* fin, int* outer) {
-    // psi[0] is the FP64 accumulator: a warm start keeps the previous step's final iterate there
-    LAUNCH(c, poisson_init_launch(c->psi[0], c->ctl, c->diag, c->n, c->ld, c->p.tol, c->p.itmax, c->stream,
-                                  !c->p.warm_start));
-    const double dx = c->p.dx, dy = c->p.dy;
-    const double c1 = dy * dy, c2 = dx * dx, c3 = dx * dx * dy * dy, B = 2 * (dx * dx + dy * dy);
-    SorArgs<float> a = sor_args32(c);
-    int total = 0;
-    const int max_outer = c->p.max_outer > 0 ? c->p.max_outer : 50;
-    *fin = SorCtl{};
-    fin->status = SOR_FAILED;
-    for (int o = 0; o < max_outer && total < c->p.itmax; ++o) {
-        LAUNCH(c, dc_residual_launch(w_src, c->psi[0], c->r32, c->n, c->ld, c1, c2, c3, B, c->stream));
-        LAUNCH(c, dc_inner_init_launch(c->e32[0], c->ctl, c->n, c->ld, c->p.inner_rtol, c->p.tol, c->p.itmax - total,
-                                       c->stream, nullptr, resident_reset_of(c)));
-        SorCtl snap{};
-        c->k_prev = o < cnv_ctx::kDcPred ? c->k_dc[o] : 0;  // this outer iteration's last length
-        int rc = run_sor<float>(c, a, &snap);
-        if (rc) return rc;
-        if (o < cnv_ctx::kDcPred) c->k_dc[o] = snap.k;
-        LAUNCH(c, dc_correct_launch(c->psi[0], c->e32[0], c->e32[1], c->ctl + c->fin_slot, c->n, c->ld, c->stream));
-        total += snap.k;
-        *outer = o + 1;
-        *fin = snap;
-        fin->k = total;
-        if (dc_final(snap.status)) return CNV_OK;
-    }
-    fin->status = SOR_FAILED;
-    return CNV_OK;
-}
-
 // ---- captured step (use_graph) -------------------------------------------------------------
 // Launch index L only matters through L mod 2 (state slots, partial sums), L mod 3 (FP64
 // iterate planes) and L mod 4 (the FP32 inner solves' stopping tests), and every solve's state
@@ -445,10 +411,10 @@ static int poisson_dc(cnv_ctx* c, const double* w_src, SorCtl* fin, int* outer) 
 // previous one's rotation, and after whole chunks the final slot is 1.  Two chunk sizes:
 // launches_per_poll for the predicted length of the solve and tail_chunk for its end, so that
 // the no-op launches queued after convergence stay few.
-static int capture(cnv_ctx* c, hipGraphExec_t* out, int (*body)(cnv_ctx*, int), int arg) {
+static int capture(cnv_ctx* c, hipGraphExec_t* out, int (*body)(cnv_ctx*, int, int), int arg, int arg2) {
     hipGraph_t g = nullptr;
     HIPC(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    const int rc = body(c, arg);
+    const int rc = body(c, arg, arg2);
     const hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (rc) {
         if (g) (void)hipGraphDestroy(g);
@@ -465,29 +431,28 @@ static bool is_dc(const cnv_ctx* c) { return c->p.precision == CNV_PREC_FP32_DC;
 // the continuity kernel also finds the largest |u| or |v|, which the blow-up check reads
 static bool wants_diag(const cnv_ctx* c) { return c->p.diagnostics || c->p.blowup_speed > 0; }
 
-// wall vorticity and transport of w[wc] into w[wc^1], then a fresh Poisson solve
-static int body_pre(cnv_ctx* c, int wc) {
+// The parts of a step.  Captured they read the solve's end from slot 1, where a replayed or resident
+// solve leaves it; launched directly, from the context's final slot.
+//
+// wall vorticity and transport of w[wc] into w[wc^1], and the start of the Poisson solve
+static int body_pre(cnv_ctx* c, int wc, int slot) {
     const int n = c->n, ld = c->ld;
+    const bool dc = is_dc(c);
+    const double rRe = 1. / c->p.Re;  // src/fluiddyn.c:98 "(1. / Re)"
     LAUNCH(c, wall_vorticity_launch(c->w[wc], c->u, c->v, n, ld, c->st, c->bc, c->stream));
-    if (is_dc(c)) {
-        if (c->p.transport_fp32)
-            LAUNCH(c, transport_fp32_launch(c->w[wc], c->w[wc ^ 1], c->u, c->v, n, ld, c->st, c->bc, 1. / c->p.Re,
-                                            c->p.dt, c->stream));
-        else
-            LAUNCH(c, transport_fp64_launch(c->w[wc], c->w[wc ^ 1], c->u, c->v, n, ld, c->st, c->bc, 1. / c->p.Re,
-                                            c->p.dt, c->stream));
-        // psi[0] is the FP64 accumulator (a warm start keeps it); the solve's sweep budget
-        LAUNCH(c, poisson_init_launch(c->psi[0], c->ctl, c->diag, n, ld, c->p.tol, c->p.itmax, c->stream,
-                                      !c->p.warm_start));
-        LAUNCH(c, dc_budget_launch(c->d_budget, c->p.itmax, nullptr, c->stream));
-        return CNV_OK;
-    }
-    LAUNCH(c, transport_fp64_launch(c->w[wc], c->w[wc ^ 1], c->u, c->v, n, ld, c->st, c->bc, 1. / c->p.Re, c->p.dt,
-                                    c->stream));
-    // warm start: whole chunks end on slot 1, which holds the previous solve's final state
-    if (c->p.warm_start) LAUNCH(c, warm_start_launch(c->psi[0], planes_of(c), c->ctl + 1, n, ld, c->stream));
-    LAUNCH(c, poisson_init_launch(c->psi[0], c->ctl, c->diag, n, ld, c->p.tol, c->p.itmax, c->stream,
-                                  !c->p.warm_start, resident_reset_of(c)));
+    // FP64 warm start: the previous solve's final iterate becomes the first one before the slots,
+    // which say where it is, are reset
+    if (c->p.warm_start && !dc) LAUNCH(c, warm_start_launch(c->psi[0], planes_of(c), c->ctl + slot, n, ld, c->stream));
+    // psi[0]: the first iterate (FP64), the accumulator (refined, which resets its inner solves' own
+    // memory at the start of each)
+    const SolveInit si{c->psi[0], c->ctl, c->diag, dc ? c->d_budget : nullptr, c->p.tol, c->p.itmax, c->p.warm_start,
+                       dc ? ResidentReset{} : resident_reset_of(c)};
+    if (dc && c->p.transport_fp32)
+        LAUNCH(c, transport_fp32_launch(c->w[wc], c->w[wc ^ 1], c->u, c->v, n, ld, c->st, c->bc, rRe, c->p.dt,
+                                        c->stream, si));
+    else
+        LAUNCH(c, transport_fp64_launch(c->w[wc], c->w[wc ^ 1], c->u, c->v, n, ld, c->st, c->bc, rRe, c->p.dt,
+                                        c->stream, si));
     return CNV_OK;
 }
 // m SOR launches, L = 0..m-1: FP64 on the source w[src] (f = -w), or the refined form's FP32
@@ -505,28 +470,26 @@ static int body_chunk_of(cnv_ctx* c, int src, int m) {
         if (launch_sor(c, a, l, gs)) return cnv_fail(c, CNV_ERR_HIP, "SOR launch failed while capturing");
     return CNV_OK;
 }
-static int body_chunk(cnv_ctx* c, int src) { return body_chunk_of(c, src, c->launches_per_poll); }
-static int body_tail(cnv_ctx* c, int src) { return body_chunk_of(c, src, c->tail_chunk); }
-// refined form, one outer iteration: FP64 residual of psi[0] against w[src], inner solve init
-// with the remaining budget (device counter) ...
-static int body_resid(cnv_ctx* c, int src) {
+// refined form, one outer iteration: FP64 residual of psi[0] against w[src], inner solve init with
+// the remaining budget (device counter); behind: only if the correction before it was made ...
+static int body_resid(cnv_ctx* c, int src, int behind) {
     const double dx = c->p.dx, dy = c->p.dy;
+    const int* go = behind ? c->d_budget + 1 : nullptr;
     LAUNCH(c, dc_residual_launch(c->w[src], c->psi[0], c->r32, c->n, c->ld, dy * dy, dx * dx,
-                                 dx * dx * dy * dy, 2 * (dx * dx + dy * dy), c->stream));
+                                 dx * dx * dy * dy, 2 * (dx * dx + dy * dy), c->stream, go));
     LAUNCH(c, dc_inner_init_launch(c->e32[0], c->ctl, c->n, c->ld, c->p.inner_rtol, c->p.tol, 0, c->stream,
-                                   c->d_budget, resident_reset_of(c)));
+                                   c->d_budget, resident_reset_of(c), go));
     return CNV_OK;
 }
-// ... and after the inner solve (final slot 1): psi[0] += e, budget -= its sweeps
-static int body_correct(cnv_ctx* c, int) {
-    LAUNCH(c, dc_correct_launch(c->psi[0], c->e32[0], c->e32[1], c->ctl + 1, c->n, c->ld, c->stream));
-    LAUNCH(c, dc_budget_launch(c->d_budget, 0, c->ctl + 1, c->stream));
+// ... and after the inner solve: psi[0] += e, budget -= its sweeps
+static int body_correct(cnv_ctx* c, int slot, int behind) {
+    LAUNCH(c, dc_correct_launch(c->psi[0], c->e32[0], c->e32[1], c->ctl + slot, behind ? c->res.r.abort : nullptr,
+                                c->d_budget, c->d_budget + 1, c->n, c->ld, c->stream));
     return CNV_OK;
 }
-// velocities from the final iterate (slot 1 after whole chunks; psi[0] in the refined form),
-// continuity diagnostic
-static int body_post(cnv_ctx* c, int) {
-    LAUNCH(c, velocities(c, c->ctl + 1));
+// velocities from the final iterate (psi[0] in the refined form), continuity diagnostic
+static int body_post(cnv_ctx* c, int slot, int) {
+    LAUNCH(c, velocities(c, c->ctl + slot));
     if (wants_diag(c)) LAUNCH(c, continuity_launch(c->u, c->v, c->diag, c->n, c->ld, c->st, c->stream));
     return CNV_OK;
 }
@@ -536,15 +499,15 @@ static int build_graphs(cnv_ctx* c) {
     const int u = c->tail_chunk;
     c->launches_per_poll = (c->launches_per_poll + u - 1) / u * u;
     for (int wc = 0; wc < 2; ++wc) {
-        int rc = capture(c, &c->g_pre[wc], body_pre, wc);
-        if (!rc && is_dc(c)) rc = capture(c, &c->g_resid[wc], body_resid, wc);
+        int rc = capture(c, &c->g_pre[wc], body_pre, wc, 1);
+        if (!rc && is_dc(c)) rc = capture(c, &c->g_resid[wc], body_resid, wc, 0);
         if (rc) return rc;
     }
     if (is_dc(c)) {
-        const int rc = capture(c, &c->g_correct, body_correct, 0);
+        const int rc = capture(c, &c->g_correct, body_correct, 1, 0);
         if (rc) return rc;
     }
-    return capture(c, &c->g_post, body_post, 0);
+    return capture(c, &c->g_post, body_post, 1, 0);
 }
 
 // Replays chunk graphs until a polled slot is terminal.  With a prediction of P launches, big
@@ -552,19 +515,9 @@ static int build_graphs(cnv_ctx* c) {
 // tail chunks follow, as many per poll as make up the eager solve's chunk for that prediction
 // (poll_chunk); without one, big chunks one per poll.
 static int replay_solve(cnv_ctx* c, int src, int predicted_sweeps, SorCtl* final_ctl) {
-    bool ran = false;
-    int rc = is_dc(c) ? run_sor_resident<float>(c, sor_args32(c), final_ctl, &ran)
-                      : run_sor_resident<double>(c, sor_args64(c, c->w[src], 1), final_ctl, &ran);
-    if (rc) return rc;
-    if (ran) {  // the captured launches that follow read slot 1
-        if (c->fin_slot != 1)
-            HIPC(c, hipMemcpyAsync(c->ctl + 1, c->ctl, sizeof(SorCtl), hipMemcpyDeviceToDevice, c->stream));
-        c->fin_slot = 1;
-        return CNV_OK;
-    }
     if (!c->g_tail[src]) {  // captured when a solve first needs them
-        rc = capture(c, &c->g_chunk[src], body_chunk, src);
-        if (!rc) rc = capture(c, &c->g_tail[src], body_tail, src);
+        int rc = capture(c, &c->g_chunk[src], body_chunk_of, src, c->launches_per_poll);
+        if (!rc) rc = capture(c, &c->g_tail[src], body_chunk_of, src, c->tail_chunk);
         if (rc) return rc;
     }
     const int M = c->launches_per_poll, Mt = c->tail_chunk;
@@ -612,31 +565,6 @@ static int replay_solve(cnv_ctx* c, int src, int predicted_sweeps, SorCtl* final
     }
 }
 
-// the refined form's solve from captured graphs: outer iterations driven by the host, each a
-// residual graph, replayed inner chunks and a correction graph (as poisson_dc)
-static int poisson_dc_graph(cnv_ctx* c, int src, SorCtl* fin, int* outer) {
-    int total = 0;
-    const int max_outer = c->p.max_outer > 0 ? c->p.max_outer : 50;
-    *fin = SorCtl{};
-    fin->status = SOR_FAILED;
-    for (int o = 0; o < max_outer && total < c->p.itmax; ++o) {
-        HIPC(c, hipGraphLaunch(c->g_resid[src], c->stream));
-        SorCtl snap{};
-        int rc = replay_solve(c, 0, o < cnv_ctx::kDcPred ? c->k_dc[o] : 0, &snap);
-        if (rc) return rc;
-        if (o < cnv_ctx::kDcPred) c->k_dc[o] = snap.k;
-        HIPC(c, hipGraphLaunch(c->g_correct, c->stream));
-        total += snap.k;
-        *outer = o + 1;
-        *fin = snap;
-        fin->k = total;
-        if (dc_final(snap.status)) return CNV_OK;
-    }
-    fin->status = SOR_FAILED;
-    return CNV_OK;
-}
-
-static int one_step(cnv_ctx* c, cnv_step_stats* stats);
 
 // A step's statistics from its final solve slot and the diagnostics; the blow-up check.
 static int finish_step(cnv_ctx* c, const SorCtl& fin, int outer, cnv_step_stats* stats) {
@@ -648,11 +576,14 @@ static int finish_step(cnv_ctx* c, const SorCtl& fin, int outer, cnv_step_stats*
     s.outer = outer;
     double speed = 0.0;
     if (wants_diag(c)) {
-        HIPC(c, hipMemcpyAsync(c->h_diag, c->diag, sizeof(Diag), hipMemcpyDeviceToHost, c->stream));
-        HIPC(c, hipStreamSynchronize(c->stream));
-        s.cont_max = dkey_inv(c->h_diag->kmax);
-        s.cont_min = dkey_inv(c->h_diag->kmin);
-        speed = dkey_inv(c->h_diag->kspd);
+        Diag* const d = reinterpret_cast<Diag*>(c->h_ctl + 3);
+        if (!c->diag_read) {
+            HIPC(c, hipMemcpyAsync(d, c->diag, sizeof(Diag), hipMemcpyDeviceToHost, c->stream));
+            HIPC(c, hipStreamSynchronize(c->stream));
+        }
+        s.cont_max = dkey_inv(d->kmax);
+        s.cont_min = dkey_inv(d->kmin);
+        speed = dkey_inv(d->kspd);
     }
     if (s.status == CNV_OK && c->p.blowup_speed > 0 && !(speed <= c->p.blowup_speed)) s.status = CNV_DIVERGED;
     if (stats) *stats = s;
@@ -667,44 +598,115 @@ static int finish_step(cnv_ctx* c, const SorCtl& fin, int outer, cnv_step_stats*
     return CNV_OK;
 }
 
-static int one_step_graph(cnv_ctx* c, cnv_step_stats* stats) {
-    if (!c->g_post) {
+// A part of the step, replayed (use_graph) or launched.
+static int part(cnv_ctx* c, hipGraphExec_t g, int (*body)(cnv_ctx*, int, int), int arg, int arg2) {
+    if (!c->p.use_graph) return body(c, arg, arg2);
+    HIPC(c, hipGraphLaunch(g, c->stream));
+    return CNV_OK;
+}
+static int part_correct(cnv_ctx* c) { return part(c, c->g_correct, body_correct, c->fin_slot, 0); }
+static int part_resid(cnv_ctx* c, int src) { return part(c, c->g_resid[src], body_resid, src, 0); }
+
+// What follows a solve in its step, queued behind its first resident kernel (Behind): FP64 and the
+// inner solve that is expected to be a refined solve's last.  The diagnostic comes back with the slots.
+static int behind_post(cnv_ctx* c, int) {
+    int rc = CNV_OK;
+    if (is_dc(c)) rc = body_correct(c, 1, 1);
+    return rc ? rc : body_post(c, 1, 0);
+}
+// An earlier inner solve: its correction and the next one's start.
+static int behind_next(cnv_ctx* c, int src) {
+    const int rc = body_correct(c, 1, 1);
+    return rc ? rc : body_resid(c, src, 1);
+}
+
+// One solve with whatever form it takes; *behind says whether what was queued behind it counts.
+// With use_graph its end is in slot 1, where the captured launches read it.
+template <typename T>
+static int solve(cnv_ctx* c, const SorArgs<T>& a, int src, int predicted, SorCtl* fin, Behind* behind) {
+    bool ran = false;
+    int rc = run_sor_resident<T>(c, a, fin, &ran, behind);
+    if (ran) {
+        if (!rc && c->p.use_graph && c->fin_slot != 1) {
+            HIPC(c, hipMemcpyAsync(c->ctl + 1, c->ctl, sizeof(SorCtl), hipMemcpyDeviceToDevice, c->stream));
+            c->fin_slot = 1;
+        }
+        return rc;
+    }
+    if (c->p.use_graph) return replay_solve(c, src, predicted, fin);
+    c->k_prev = predicted;
+    return run_sor_launches<T>(c, a, fin);
+}
+
+// the refined form's solve on w[src]: outer iterations driven by the host, each an FP64 residual, an
+// FP32 inner solve (e32 ping-pong) and the correction of psi[0]; *posted: the step's last launches
+// are queued too
+static int poisson_dc(cnv_ctx* c, int src, SorCtl* fin, int* outer, bool* posted) {
+    int total = 0;
+    const int max_outer = c->p.max_outer > 0 ? c->p.max_outer : 50;
+    *fin = SorCtl{};
+    fin->status = SOR_FAILED;
+    const SorArgs<float> a = sor_args32(c);
+    bool ready = false;  // this outer iteration's inner solve has been prepared
+    for (int o = 0; o < max_outer && total < c->p.itmax; ++o) {
+        int rc = ready ? CNV_OK : part_resid(c, src);
+        if (rc) return rc;
+        SorCtl snap{};
+        const bool last = o + 1 == c->outer_prev;
+        Behind behind;
+        behind.queue = last ? behind_post : behind_next;
+        behind.arg = src;
+        if (!last) behind.read = c->ev[0];
+        rc = solve<float>(c, a, 0, o < cnv_ctx::kDcPred ? c->k_dc[o] : 0, &snap, &behind);
+        if (rc) return rc;
+        if (o < cnv_ctx::kDcPred) c->k_dc[o] = snap.k;
+        if (!behind.counts && (rc = part_correct(c))) return rc;
+        ready = behind.counts && !last;
+        total += snap.k;
+        *outer = o + 1;
+        *fin = snap;
+        fin->k = total;
+        *posted = behind.counts && last && dc_final(snap.status);
+        // a diagnostic that was taken too early starts over
+        if (last && !*posted) LAUNCH(c, diag_reset_launch(c->diag, c->stream));
+        if (dc_final(snap.status)) break;
+    }
+    c->outer_prev = *outer;
+    if (!dc_final(fin->status)) fin->status = SOR_FAILED;
+    return CNV_OK;
+}
+
+static int one_step(cnv_ctx* c, cnv_step_stats* stats) {
+    if (c->p.use_graph && !c->g_post) {
         const int rc = build_graphs(c);
         if (rc) {
             drop_graphs(c);
             return rc;
         }
     }
-    HIPC(c, hipGraphLaunch(c->g_pre[c->wcur], c->stream));
+    int rc = part(c, c->g_pre[c->wcur], body_pre, c->wcur, c->fin_slot);
+    if (rc) return rc;
     c->wcur ^= 1;
     SorCtl fin{};
     int outer = 0;
-    int rc = is_dc(c) ? poisson_dc_graph(c, c->wcur, &fin, &outer) : replay_solve(c, c->wcur, c->k_prev, &fin);
+    bool posted = false, early = false;
+    if (is_dc(c)) {
+        rc = poisson_dc(c, c->wcur, &fin, &outer, &posted);
+    } else {
+        Behind behind;
+        behind.queue = behind_post;
+        rc = solve<double>(c, sor_args64(c, c->w[c->wcur], 1), c->wcur, c->k_prev, &fin, &behind);
+        c->k_prev = fin.k;
+        posted = behind.counts;
+        early = !posted && c->res_on;  // the diagnostic was taken before the solve's end
+    }
     if (rc) return rc;
-    if (!is_dc(c)) c->k_prev = fin.k;
-    HIPC(c, hipGraphLaunch(c->g_post, c->stream));
-    return finish_step(c, fin, outer, stats);
-}
-
-static int one_step(cnv_ctx* c, cnv_step_stats* stats) {
-    if (c->p.use_graph) return one_step_graph(c, stats);
-    const int n = c->n, ld = c->ld;
-    const double rRe = 1. / c->p.Re;  // src/fluiddyn.c:98 "(1. / Re)"
-    double* w_in = c->w[c->wcur];
-    double* w_out = c->w[c->wcur ^ 1];
-    const bool dc = c->p.precision == CNV_PREC_FP32_DC;
-    LAUNCH(c, wall_vorticity_launch(w_in, c->u, c->v, n, ld, c->st, c->bc, c->stream));
-    if (dc && c->p.transport_fp32)
-        LAUNCH(c, transport_fp32_launch(w_in, w_out, c->u, c->v, n, ld, c->st, c->bc, rRe, c->p.dt, c->stream));
-    else
-        LAUNCH(c, transport_fp64_launch(w_in, w_out, c->u, c->v, n, ld, c->st, c->bc, rRe, c->p.dt, c->stream));
-    c->wcur ^= 1;
-    SorCtl fin{};
-    int outer = 0;
-    int rc = dc ? poisson_dc(c, w_out, &fin, &outer) : poisson_fp64(c, w_out, 1, &fin);
-    if (rc) return rc;
-    LAUNCH(c, velocities(c, c->ctl + c->fin_slot));
-    if (wants_diag(c)) LAUNCH(c, continuity_launch(c->u, c->v, c->diag, n, ld, c->st, c->stream));
+    if (!posted) {
+        if (early) LAUNCH(c, diag_reset_launch(c->diag, c->stream));
+        rc = part(c, c->g_post, body_post, c->fin_slot, 0);
+        if (rc) return rc;
+    }
+    c->diag_read = posted;
     return finish_step(c, fin, outer, stats);
 }
 

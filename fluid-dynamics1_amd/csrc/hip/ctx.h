@@ -40,12 +40,14 @@ struct cnv_ctx {
     float* d_ftab = nullptr;
     cnv::Stencils st{};
     // solver control
-    cnv::SorCtl* ctl = nullptr;  // the Poisson solve's two state slots, then the resident abort flag
+    // the Poisson solve's two state slots, the resident abort flag and the diagnostic, 64 bytes each,
+    // so that one copy brings them all to h_ctl
+    cnv::SorCtl* ctl = nullptr;
     int fin_slot = 0;            // slot written by the last SOR launch of the last solve
-    cnv::Diag* diag = nullptr;
+    cnv::Diag* diag = nullptr;     // ctl + 3
     double* partial = nullptr;
     cnv::SorCtl* h_ctl = nullptr;  // pinned, kSlots entries
-    cnv::Diag* h_diag = nullptr;   // pinned
+    bool diag_read = false;        // h_ctl holds this step's diagnostic already
     hipEvent_t ev[kSlots] = {};
     hipEvent_t t0 = nullptr, t1 = nullptr;
     // defect correction
@@ -78,7 +80,9 @@ struct cnv_ctx {
     ResidentPlan res;
     unsigned long long* d_res = nullptr;
     double* d_res_snap = nullptr;
-    int* d_budget = nullptr;  // refined form, captured: the solve's remaining sweep budget
+    int* d_budget = nullptr;  // refined form: the solve's remaining sweep budget, and whether the last
+                              // inner solve was added (dc_correct_kernel)
+    int outer_prev = 0;       // outer iterations of the last refined solve
     // output snapshots (cnv_snapshot_begin/wait): a device copy of (w, psi, u, v) taken in stream
     // order, then transferred to pinned host memory on a stream of its own
     double* d_snap = nullptr;
@@ -259,19 +263,30 @@ void resident_bind(ResidentPlan* p, unsigned long long* words, double* snap, cnv
 // Takes a plan's share of the device for the time of a solve (false: not now).
 bool resident_enter(int dev, int units);
 void resident_leave(int dev, int units);
-// The kernels of one solve, between the two calls above, on fresh slots and reset memory.  h: three
+// Launches queued behind a solve's first resident kernel before the host knows whether that kernel
+// ended the solve (in slot 1): queued(c, arg) queues them; if it did not, they have had no effect
+// that queueing them again later does not replace.
+struct Behind {
+    int (*queue)(cnv_ctx* c, int arg) = nullptr;
+    int arg = 0;
+    // the slots are read back before them (they change the slots), and the host waits for this
+    // event; else after them, with the diagnostic
+    hipEvent_t read = nullptr;
+    bool counts = false;  // set: the first kernel did end the solve, what was queued counts
+};
+// The kernels of one solve, between the two calls above, on fresh slots and reset memory.  h: four
 // slots of host memory.  *resume < 0: it has ended (*fin, in slot *fin_slot), else the launch index
 // to go on from as launches (a wave gave up waiting).
 template <typename T>
 int resident_chunks(cnv_ctx* c, const ResidentPlan& p, cnv::SorArgs<T> a, bool gs, int itmax, hipStream_t st,
-                    cnv::SorCtl* h, cnv::SorCtl* fin, int* fin_slot, int* resume);
+                    cnv::SorCtl* h, cnv::SorCtl* fin, int* fin_slot, int* resume, Behind* behind = nullptr);
 // Sets up the context's resident solves where its grid and the device allow them.
 int resident_setup(cnv_ctx* c);
 // What the init kernels reset for a solve that may run resident.
 inline cnv::ResidentReset resident_reset_of(const cnv_ctx* c) { return c->res_on ? c->res.reset : cnv::ResidentReset{}; }
 // The solve as resident kernels when they can run now (*ran = false: nothing was done).
 template <typename T>
-int run_sor_resident(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* final_ctl, bool* ran);
+int run_sor_resident(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* final_ctl, bool* ran, Behind* behind = nullptr);
 
 template <typename T>
 inline int run_sor(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* final_ctl) {

@@ -40,37 +40,42 @@ __global__ void __launch_bounds__(kBlock) dc_residual_kernel(const double* __res
                                                             const double* __restrict__ psi,
                                                             float* __restrict__ r32, int n, int ld,
                                                             double c1, double c2, double c3,
-                                                            double B) {
+                                                            double B, const int* go) {
+    if (go && !*go) return;
     const int j = blockIdx.x * 64 + (threadIdx.x & 63);
     const int i = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (i < n && j < n) dc_residual_at(w, psi, r32, n, ld, c1, c2, c3, B, i, j);
 }
 
-// psi64 += e32 (the inner solve's final iterate, chosen by the control block's parity)
+// psi64 += e32 (the inner solve's final iterate, chosen by the control block's parity), and the
+// solve's sweep budget less the inner solve's sweeps -- if the inner solve has ended: this may be
+// queued behind a resident kernel that did not finish it, and the launches behind this one, which
+// prepare the next inner solve, look at *go
 __global__ void __launch_bounds__(kBlock) dc_correct_kernel(double* __restrict__ psi, const float* e0,
-                                                           const float* e1, const SorCtl* fin,
-                                                           long long count) {
+                                                           const float* e1, const SorCtl* fin, const int* abort,
+                                                           int* budget, int* go, long long count) {
+    const int st = fin->status;
+    const bool ended = st != SOR_RUNNING && st != SOR_ROLLBACK && !(abort && *abort);
     const float* e = fin->parity ? e1 : e0;
     const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (q < count) psi[q] += (double)e[q];
+    if (q == 0) {
+        *go = ended;
+        if (ended) *budget -= fin->k;
+    }
+    if (ended && q < count) psi[q] += (double)e[q];
 }
 
 // start of an inner solve: e = 0, control block reset with the absolute tolerance (the plain
 // solver's stopping rule) and the FP32 fold ratio
 __global__ void __launch_bounds__(kBlock) dc_inner_init_kernel(float* e0, SorCtl* ctl, long long count,
                                                               double rtol, double tol, int itmax,
-                                                              const int* budget, ResidentReset rr) {
-    const long long stride = (long long)gridDim.x * kBlock;
-    for (long long q = (long long)blockIdx.x * kBlock + threadIdx.x; q < count; q += stride) e0[q] = 0.0f;
-    // the sweep budget comes from the device counter when there is one (captured step)
-    if (blockIdx.x == 0 && threadIdx.x < 2) ctl_reset(ctl + threadIdx.x, tol, rtol, budget ? *budget : itmax);
-    resident_reset_at(rr);
-}
-
-// device sweep budget of a refined solve: fin == nullptr resets it to itmax, otherwise the inner
-// solve that ended in slot fin spent fin->k sweeps of it
-__global__ void dc_budget_kernel(int* budget, int itmax, const SorCtl* fin) {
-    if (threadIdx.x == 0) *budget = fin ? *budget - fin->k : itmax;
+                                                              const int* budget, ResidentReset rr, const int* go) {
+    if (go && !*go) return;
+    const long long q0 = (long long)blockIdx.x * kBlock + threadIdx.x, stride = (long long)gridDim.x * kBlock;
+    for (long long q = q0; q < count; q += stride) e0[q] = 0.0f;
+    // the sweep budget comes from the device counter when there is one
+    if (q0 < 2) ctl_reset(ctl + q0, tol, rtol, budget ? *budget : itmax);
+    resident_reset_at(rr, q0, stride);
 }
 
 __global__ void __launch_bounds__(kBlock) transport_fp32_kernel(const double* __restrict__ w,
@@ -78,10 +83,12 @@ __global__ void __launch_bounds__(kBlock) transport_fp32_kernel(const double* __
                                                                const double* __restrict__ u,
                                                                const double* __restrict__ v, int n,
                                                                int ld, Stencils s, WallBC b,
-                                                               double rRe, double dt) {
+                                                               double rRe, double dt, SolveInit si) {
     const int j = blockIdx.x * 64 + (threadIdx.x & 63);
     const int i = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (i < n && j < n) transport_fp32_at(w, wout, u, v, n, ld, s, b, rRe, dt, i, j);
+    solve_init_at(si, (long long)n * ld, ((long long)blockIdx.y * gridDim.x + blockIdx.x) * kBlock + threadIdx.x,
+                  (long long)gridDim.x * gridDim.y * kBlock);
 }
 
 // refined-form velocities from the FP64 accumulator with FP32 stencils (velocity_fp32_at)
@@ -103,38 +110,35 @@ int velocity_fp32_launch(const double* psi, double* u, double* v, int n, int ld,
 }
 
 int dc_residual_launch(const double* w, const double* psi, float* r32, int n, int ld, double c1,
-                       double c2, double c3, double B, hipStream_t st) {
+                       double c2, double c3, double B, hipStream_t st, const int* go) {
     dim3 grid((n + 63) / 64, (n + 3) / 4);
-    hipLaunchKernelGGL(dc_residual_kernel, grid, dim3(kBlock), 0, st, w, psi, r32, n, ld, c1, c2, c3, B);
+    hipLaunchKernelGGL(dc_residual_kernel, grid, dim3(kBlock), 0, st, w, psi, r32, n, ld, c1, c2, c3, B, go);
     return launched();
 }
 
-int dc_correct_launch(double* psi, const float* e0, const float* e1, const SorCtl* fin, int n, int ld,
-                      hipStream_t st) {
+int dc_correct_launch(double* psi, const float* e0, const float* e1, const SorCtl* fin, const int* abort,
+                      int* budget, int* go, int n, int ld, hipStream_t st) {
     const long long count = (long long)n * ld;
-    hipLaunchKernelGGL(dc_correct_kernel, dim3(blocks_for(count)), dim3(kBlock), 0, st, psi, e0, e1, fin, count);
+    hipLaunchKernelGGL(dc_correct_kernel, dim3(blocks_for(count)), dim3(kBlock), 0, st, psi, e0, e1, fin, abort,
+                       budget, go, count);
     return launched();
 }
 
-int dc_inner_init_launch(float* e0, SorCtl* ctl, int n, int ld, double rtol, double tol, int itmax,
-                         hipStream_t st, const int* budget, const ResidentReset& rr) {
+int dc_inner_init_launch(float* e0, SorCtl* ctl, int n, int ld, double rtol, double tol, int itmax, hipStream_t st,
+                         const int* budget, const ResidentReset& rr, const int* go) {
     const long long count = (long long)n * ld;
     unsigned nb = blocks_for(count + rr.exch);
     if (nb > 2048) nb = 2048;
-    hipLaunchKernelGGL(dc_inner_init_kernel, dim3(nb), dim3(kBlock), 0, st, e0, ctl, count, rtol, tol, itmax,
-                       budget, rr);
-    return launched();
-}
-
-int dc_budget_launch(int* budget, int itmax, const SorCtl* fin, hipStream_t st) {
-    hipLaunchKernelGGL(dc_budget_kernel, dim3(1), dim3(64), 0, st, budget, itmax, fin);
+    hipLaunchKernelGGL(dc_inner_init_kernel, dim3(nb), dim3(kBlock), 0, st, e0, ctl, count, rtol, tol, itmax, budget,
+                       rr, go);
     return launched();
 }
 
 int transport_fp32_launch(const double* w_in, double* w_out, const double* u, const double* v, int n, int ld,
-                          const Stencils& s, const WallBC& bc, double rRe, double dt, hipStream_t st) {
+                          const Stencils& s, const WallBC& bc, double rRe, double dt, hipStream_t st,
+                          const SolveInit& si) {
     dim3 grid((n + 63) / 64, (n + 3) / 4);
-    hipLaunchKernelGGL(transport_fp32_kernel, grid, dim3(kBlock), 0, st, w_in, w_out, u, v, n, ld, s, bc, rRe, dt);
+    hipLaunchKernelGGL(transport_fp32_kernel, grid, dim3(kBlock), 0, st, w_in, w_out, u, v, n, ld, s, bc, rRe, dt, si);
     return launched();
 }
 

@@ -25,22 +25,21 @@ __global__ void __launch_bounds__(kBlock) transport_fp64_kernel(const double* __
                                                                const double* __restrict__ u,
                                                                const double* __restrict__ v, int n,
                                                                int ld, Stencils s, WallBC b,
-                                                               double rRe, double dt) {
+                                                               double rRe, double dt, SolveInit si) {
     const int j = blockIdx.x * 64 + (threadIdx.x & 63);
     const int i = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (i < n && j < n) transport_fp64_at(w, wout, u, v, n, ld, s, b, rRe, dt, i, j);
+    solve_init_at(si, (long long)n * ld, ((long long)blockIdx.y * gridDim.x + blockIdx.x) * kBlock + threadIdx.x,
+                  (long long)gridDim.x * gridDim.y * kBlock);
 }
 
-// ---- start of a Poisson solve: psi = 0 (src/poisson.c:229-230), reset the control block ----
-__global__ void __launch_bounds__(kBlock) poisson_init_kernel(double* psi0, SorCtl* ctl, Diag* diag,
-                                                             long long count, double tol, int itmax,
-                                                             int zero, ResidentReset rr) {
-    const long long stride = (long long)gridDim.x * kBlock;
-    if (zero)
-        for (long long q = (long long)blockIdx.x * kBlock + threadIdx.x; q < count; q += stride) psi0[q] = 0.0;
-    if (blockIdx.x == 0 && threadIdx.x < 2) ctl_reset(ctl + threadIdx.x, tol, 0.0, itmax);
-    if (blockIdx.x == 0 && threadIdx.x == 0 && diag) diag_reset(diag);
-    resident_reset_at(rr);
+// ---- start of a Poisson solve (solve_init_at) where no transport launch makes it ------------
+__global__ void __launch_bounds__(kBlock) poisson_init_kernel(SolveInit si, long long count) {
+    solve_init_at(si, count, (long long)blockIdx.x * kBlock + threadIdx.x, (long long)gridDim.x * kBlock);
+}
+
+__global__ void diag_reset_kernel(Diag* diag) {
+    if (threadIdx.x == 0) diag_reset(diag);
 }
 
 // warm start (opt-in): the previous solve's final iterate, psi[fin->parity], becomes psi0, the
@@ -122,7 +121,9 @@ __global__ void __launch_bounds__(kBlock) snapshot_kernel(const double* __restri
 }
 
 // marks and zeros before a resident solve (ResidentReset)
-__global__ void __launch_bounds__(kBlock) resident_reset_kernel(ResidentReset rr) { resident_reset_at(rr); }
+__global__ void __launch_bounds__(kBlock) resident_reset_kernel(ResidentReset rr) {
+    resident_reset_at(rr, (long long)blockIdx.x * kBlock + threadIdx.x, (long long)gridDim.x * kBlock);
+}
 
 // ---- host wrappers -------------------------------------------------------------------------
 static inline int launched() { return hipGetLastError() == hipSuccess ? 0 : 1; }
@@ -164,9 +165,10 @@ int wall_vorticity_launch(double* w, const double* u, const double* v, int n, in
 }
 
 int transport_fp64_launch(const double* w_in, double* w_out, const double* u, const double* v, int n, int ld,
-                          const Stencils& s, const WallBC& bc, double rRe, double dt, hipStream_t st) {
+                          const Stencils& s, const WallBC& bc, double rRe, double dt, hipStream_t st,
+                          const SolveInit& si) {
     dim3 grid((n + 63) / 64, (n + 3) / 4);
-    hipLaunchKernelGGL(transport_fp64_kernel, grid, dim3(kBlock), 0, st, w_in, w_out, u, v, n, ld, s, bc, rRe, dt);
+    hipLaunchKernelGGL(transport_fp64_kernel, grid, dim3(kBlock), 0, st, w_in, w_out, u, v, n, ld, s, bc, rRe, dt, si);
     return launched();
 }
 
@@ -175,8 +177,13 @@ int poisson_init_launch(double* psi0, SorCtl* ctl, Diag* diag, int n, int ld, do
     const long long count = (long long)n * ld;
     unsigned nb = blocks_for(count + rr.exch);
     if (nb > 2048) nb = 2048;
-    hipLaunchKernelGGL(poisson_init_kernel, dim3(nb), dim3(kBlock), 0, st, psi0, ctl, diag, count, tol, itmax,
-                       zero, rr);
+    const SolveInit si{psi0, ctl, diag, nullptr, tol, itmax, !zero, rr};
+    hipLaunchKernelGGL(poisson_init_kernel, dim3(nb), dim3(kBlock), 0, st, si, count);
+    return launched();
+}
+
+int diag_reset_launch(Diag* diag, hipStream_t st) {
+    hipLaunchKernelGGL(diag_reset_kernel, dim3(1), dim3(64), 0, st, diag);
     return launched();
 }
 

@@ -114,7 +114,7 @@ int cnv_poisson_device_noalloc(int n, double dx, double dy, double beta, double 
     SorCtl fin{};
     int resume = 0;  // launch index to go on from; < 0: the solve has ended
     if (resident) {
-        SorCtl h[3];
+        SorCtl h[4];
         int slot = 0;
         rc = resident_chunks<double>(nullptr, plan, a, gs, itmax, st, h, &fin, &slot, &resume);
         if (rc) (void)hipStreamSynchronize(st);

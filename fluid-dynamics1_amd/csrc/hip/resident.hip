@@ -141,7 +141,7 @@ void resident_leave(int dev, int units) { g_units[dev].fetch_sub(units); }
 
 template <typename T>
 int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, int itmax, hipStream_t st, SorCtl* h,
-                    SorCtl* fin, int* fin_slot, int* resume) {
+                    SorCtl* fin, int* fin_slot, int* resume, Behind* behind) {
     constexpr int NB = SorPlanes<T>::value;
     SorResident r = p.r;
     a.tiles_i = p.tiles_i;
@@ -156,8 +156,17 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, in
         r.dst = (r.src + 1) % NB;
         r.wslot = r.rslot ^ 1;
         LAUNCH(c, launch_resident(a, r, p.shape, gs, st));
-        HIPC(c, hipMemcpyAsync(h, a.ctl, 3 * sizeof(SorCtl), hipMemcpyDeviceToHost, st));
-        HIPC(c, hipStreamSynchronize(st));
+        const bool first = r.launch0 == 0 && r.stop == 0 && behind && behind->queue;
+        int rc = first && !behind->read ? behind->queue(c, behind->arg) : CNV_OK;
+        if (rc) return rc;
+        HIPC(c, hipMemcpyAsync(h, a.ctl, 4 * sizeof(SorCtl), hipMemcpyDeviceToHost, st));
+        if (first && behind->read) {
+            HIPC(c, hipEventRecord(behind->read, st));
+            if ((rc = behind->queue(c, behind->arg))) return rc;
+            HIPC(c, hipEventSynchronize(behind->read));
+        } else {
+            HIPC(c, hipStreamSynchronize(st));
+        }
         int aborted = 0;
         memcpy(&aborted, h + 2, sizeof(aborted));
         if (aborted) {
@@ -173,6 +182,7 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, in
             if (s.rb_n != kNotStored || r.stop > 0) {
                 *fin = s;
                 *fin_slot = r.wslot;
+                if (behind) behind->counts = first;
                 return CNV_OK;
             }
             r.stop = s.k;  // once more, to exactly the sweep the solve ended with
@@ -186,17 +196,17 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, in
     return cnv_fail(c, CNV_ERR_HIP, "SOR state did not terminate after %d epochs", r.launch0);
 }
 template int resident_chunks<double>(cnv_ctx*, const ResidentPlan&, SorArgs<double>, bool, int, hipStream_t, SorCtl*,
-                                     SorCtl*, int*, int*);
+                                     SorCtl*, int*, int*, Behind*);
 
 template <typename T>
-int run_sor_resident(cnv_ctx* c, const SorArgs<T>& a, SorCtl* final_ctl, bool* ran) {
+int run_sor_resident(cnv_ctx* c, const SorArgs<T>& a, SorCtl* final_ctl, bool* ran, Behind* behind) {
     const int dev = c->p.device;
     // with other resident solves running that leave too few CUs, this one runs as launches
     *ran = c->res_on && resident_enter(dev, c->res.units);
     if (!*ran) return CNV_OK;
     int resume = -1;
     const int rc = resident_chunks<T>(c, c->res, a, c->p.poisson_type == 1, c->p.itmax, c->stream, c->h_ctl, final_ctl,
-                                      &c->fin_slot, &resume);
+                                      &c->fin_slot, &resume, behind);
     // a failed call may leave its kernel running, which holds its place until it has ended
     if (rc) (void)hipStreamSynchronize(c->stream);
     resident_leave(dev, c->res.units);
@@ -204,5 +214,5 @@ int run_sor_resident(cnv_ctx* c, const SorArgs<T>& a, SorCtl* final_ctl, bool* r
     c->res_on = false;
     return run_sor_launches<T>(c, a, final_ctl, resume);
 }
-template int run_sor_resident<double>(cnv_ctx*, const SorArgs<double>&, SorCtl*, bool*);
-template int run_sor_resident<float>(cnv_ctx*, const SorArgs<float>&, SorCtl*, bool*);
+template int run_sor_resident<double>(cnv_ctx*, const SorArgs<double>&, SorCtl*, bool*, Behind*);
+template int run_sor_resident<float>(cnv_ctx*, const SorArgs<float>&, SorCtl*, bool*, Behind*);

@@ -108,13 +108,12 @@ __device__ inline void transport_fp64_at(const double* __restrict__ w, double* _
     wout[(size_t)i * ld + j] = (-uu * dwdx - vv * dwdy + rRe * (d2wdx2 + d2wdy2)) * dt + w[(size_t)i * ld + j];
 }
 
-// ---- what a resident solve finds at its start (all threads of the grid together) ------------
-__device__ inline void resident_reset_at(const ResidentReset& rr) {
+// ---- what a resident solve finds at its start, thread q of `threads` in the grid -------------
+__device__ inline void resident_reset_at(const ResidentReset& rr, long long q, long long threads) {
     if (!rr.base) return;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *rr.abort = 0;
-    const long long stride = (long long)gridDim.x * kBlock, total = rr.exch + rr.part + rr.zero;
-    for (long long q = (long long)blockIdx.x * kBlock + threadIdx.x; q < total; q += stride)
-        rr.base[q] = q < rr.exch ? rr.mark : (q < rr.exch + rr.part ? kMark64 : 0ull);
+    if (q == 0) *rr.abort = 0;
+    const long long total = rr.exch + rr.part + rr.zero;
+    for (; q < total; q += threads) rr.base[q] = q < rr.exch ? rr.mark : (q < rr.exch + rr.part ? kMark64 : 0ull);
 }
 
 // ---- one state slot of a fresh solve (launch 0 reads slot 1; both are written) -------------
@@ -136,6 +135,18 @@ __device__ inline void diag_reset(Diag* d) {
     d->kmax = dkey(-DBL_MAX);
     d->kmin = dkey(DBL_MAX);
     d->kspd = dkey(0.0);
+}
+
+// ---- start of a Poisson solve: psi = 0 (src/poisson.c:229-230), fresh slots, diagnostic; thread q of
+//      `threads` in the grid ----------------------------------------------------------------
+__device__ inline void solve_init_at(const SolveInit& si, long long count, long long q, long long threads) {
+    if (!si.psi0) return;
+    if (!si.keep)
+        for (long long p = q; p < count; p += threads) si.psi0[p] = 0.0;
+    if (q < 2) ctl_reset(si.ctl + q, si.tol, 0.0, si.itmax);
+    if (q == 0 && si.diag) diag_reset(si.diag);
+    if (q == 0 && si.budget) *si.budget = si.itmax;
+    resident_reset_at(si.rr, q, threads);
 }
 
 // ---- velocities u = DY psi, v = -(DX psi) at (i, j) (src/main.c:366-383) -------------------
