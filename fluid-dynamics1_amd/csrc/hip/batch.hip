@@ -19,6 +19,10 @@
 // |u| or |v| after a step exceeds its blowup_speed -- is taken out of the workgroup maps: later
 // steps launch nothing for it and the other cavities go on (cnv_batch_status reports it).
 //
+// Where the device and the cavities allow it, all solves of a step (or of an outer iteration) run in one
+// resident kernel instead (sor_resident.h): its workgroups take the cavities' tiles from one queue
+// per XCD, the longest solves first, and every cavity goes at its own pace.
+//
 // The SOR launch shape (sweeps per launch, waves, rows per wave) is one per batch; the autotuner
 // (cnv_batch_autotune) times every compiled shape on the batch itself and keeps the fastest.
 #pragma clang fp contract(off)
@@ -35,6 +39,7 @@
 #include "cnv_device.h"
 #include "ctx.h"
 #include "sor_rb.h"
+#include "sor_resident.h"
 #include "step_kernels.h"
 
 using namespace cnv;
@@ -102,9 +107,18 @@ __global__ void __launch_bounds__(kBlock) batch_transport_kernel(const StepItem*
         transport_fp64_at(I.w[wcur], I.w[wcur ^ 1], I.u, I.v, I.n, I.ld, I.st, I.bc, I.rRe, I.dt, i, j);
 }
 
+// what a resident launch finds: cavity m.inst's marks and words, and the queues' counters
+__device__ inline void batch_resident_reset(const ResidentReset* __restrict__ rr, int* counters, const BlockRef& m) {
+    if (!rr) return;
+    if (blockIdx.x == 0)
+        for (int q = threadIdx.x; q < kQueueCounters; q += kBlock) counters[q] = 0;
+    resident_reset_at(rr[m.inst], (long long)m.lb * kBlock + threadIdx.x, (long long)m.nb * kBlock);
+}
+
 // psi = 0 (src/poisson.c:229-230), both state slots reset, diagnostic reset
 __global__ void __launch_bounds__(kBlock) batch_poisson_init_kernel(const StepItem* __restrict__ it,
-                                                                    const BlockRef* __restrict__ map) {
+                                                                    const BlockRef* __restrict__ map,
+                                                                    const ResidentReset* __restrict__ rr, int* counters) {
     const BlockRef m = map[blockIdx.x];
     if (m.inst < 0) return;
     const StepItem& I = it[m.inst];
@@ -113,6 +127,7 @@ __global__ void __launch_bounds__(kBlock) batch_poisson_init_kernel(const StepIt
         I.psi[0][q] = 0.0;
     if (m.lb == 0 && threadIdx.x < 2) ctl_reset(I.ctl + threadIdx.x, I.tol, 0.0, I.itmax);
     if (m.lb == 0 && threadIdx.x == 0) diag_reset(I.diag);
+    batch_resident_reset(rr, counters, m);
 }
 
 // DC: the refined form's accumulator psi[0]; F32: its FP32 stencils (velocity_fp32_at)
@@ -165,7 +180,8 @@ __global__ void __launch_bounds__(kBlock) batch_dc_residual_kernel(const StepIte
 // slots, so the batched SOR launches pass over them
 __global__ void __launch_bounds__(kBlock) batch_dc_inner_init_kernel(const StepItem* __restrict__ it,
                                                                      const BlockRef* __restrict__ map,
-                                                                     const DcSlot* __restrict__ dc, double rtol) {
+                                                                     const DcSlot* __restrict__ dc, double rtol,
+                                                                     const ResidentReset* __restrict__ rr, int* counters) {
     const BlockRef m = map[blockIdx.x];
     if (m.inst < 0) return;
     const StepItem& I = it[m.inst];
@@ -179,6 +195,7 @@ __global__ void __launch_bounds__(kBlock) batch_dc_inner_init_kernel(const StepI
         ctl_reset(I.ctl + threadIdx.x, I.tol, rtol, d.itmax);
         if (!d.active) I.ctl[threadIdx.x].status = SOR_CONVERGED;
     }
+    if (blockIdx.x == 0 || d.active) batch_resident_reset(rr, counters, m);
 }
 
 // psi64 += e32 (the inner solve's final iterate) for active cavities
@@ -270,6 +287,23 @@ struct cnv_batch {
     int nb_sor = 0;
     std::vector<size_t> part_off;  // per cavity, doubles into d_partial
     size_t part_total = 0;
+    // resident solves: plans and memory of each cavity, the queues, tables of this batch's arguments
+    // with the resident shape's tiles (res_on: usable)
+    bool res_on = false, res_dirty = true;  // res_dirty: the queues are to be made again
+    std::vector<ResidentPlan> plan;
+    std::vector<int> last_k;                // sweeps of each cavity's first steps, what orders the queues
+    int order_steps = 0;
+    TileShape res_shape{5, 16, 4};
+    unsigned long long* d_rwords = nullptr;
+    double* d_rsnap = nullptr;
+    int* d_rcount = nullptr;                // the queues' counters, then the abort flag
+    SorResident* d_res = nullptr;
+    ResidentReset* d_rreset = nullptr;
+    SorArgs<double>* d_rargs64[2] = {nullptr, nullptr};
+    SorArgs<float>* d_rargs32 = nullptr;
+    ResidentJob* d_jobs = nullptr;
+    int* d_order = nullptr;
+    ResidentQueues queues{};
     // host mirrors (pinned)
     SorCtl* h_ctl = nullptr;  // [kSlots][count][2]
     Diag* h_diag = nullptr;
@@ -459,6 +493,257 @@ static int run_sor_batch(cnv_batch* b, bool fp32, std::vector<SorCtl>& snaps) {
     }
 }
 
+// ---- resident solves of a batch ---------------------------------------------------------------
+constexpr int kPerXcd = 32;           // workgroups of one launch on each XCD, one a CU
+constexpr int kBatchSpins = 1 << 24;  // polls of a wait: a solve also waits for the ones before it
+
+// Which tiles run where and in which order: the longest solves first, each as soon as its tiles have
+// room, in bands of whole tile rows on as few XCDs as that takes; a shorter one goes ahead where a
+// longer one has to wait.  Played through with the solves' expected lengths, so that the queues
+// hold the solves in the order in which they start: on the 64-cavity workload within 16% of a full
+// GPU at all times (longest first without looking for room: 36%).
+struct ResidentSchedule {
+    std::vector<int> order;
+    std::vector<ResidentJob> jobs[kBands];
+    double length = 0.0;  // sweeps from the first solve's start to the last one's end
+};
+static bool resident_schedule(cnv_batch* b, const std::vector<int>& todo, ResidentSchedule* sc) {
+    struct Running {
+        double end;
+        int rows[kBands], tiles_j;
+    };
+    std::vector<int> waiting(todo);
+    std::stable_sort(waiting.begin(), waiting.end(), [&](int x, int y) { return b->last_k[x] > b->last_k[y]; });
+    std::vector<Running> running;
+    int room[kBands];
+    for (int& r : room) r = kPerXcd - 1;  // an XCD's workgroups less a deciding one
+    double now = 0.0;
+    while (!waiting.empty()) {
+        for (size_t w = 0; w < waiting.size();) {
+            const int i = waiting[w];
+            const ResidentPlan& p = b->plan[i];
+            int total = 0, fit = -1;  // tile rows there is room for; the fullest XCD that takes all
+            for (int x = 0; x < kBands; ++x) {
+                const int rows = room[x] / p.tiles_j;
+                total += rows;
+                if (rows >= p.tiles_i && (fit < 0 || room[x] < room[fit])) fit = x;
+            }
+            if (total < p.tiles_i) {
+                ++w;
+                continue;
+            }
+            Running r{now + std::max(b->last_k[i], 1), {}, p.tiles_j};
+            for (int lo = 0; lo < p.tiles_i;) {
+                int x = fit;
+                for (int y = 0; y < kBands && fit < 0; ++y)
+                    if (x < 0 || room[y] > room[x]) x = y;
+                const int hi = std::min(p.tiles_i, lo + room[x] / p.tiles_j);
+                for (int t = lo * p.tiles_j; t < hi * p.tiles_j; ++t) sc->jobs[x].push_back({i, t, lo, hi});
+                r.rows[x] = hi - lo;
+                room[x] -= (hi - lo) * p.tiles_j;
+                lo = hi;
+            }
+            running.push_back(r);
+            sc->order.push_back(i);
+            waiting.erase(waiting.begin() + w);
+        }
+        if (waiting.empty()) break;
+        if (running.empty()) return false;  // a solve that does not fit an empty GPU
+        const auto next = std::min_element(running.begin(), running.end(),
+                                           [](const Running& x, const Running& y) { return x.end < y.end; });
+        now = next->end;
+        for (int x = 0; x < kBands; ++x) room[x] += next->rows[x] * next->tiles_j;
+        running.erase(next);
+    }
+    for (const Running& r : running) sc->length = std::max(sc->length, r.end);
+    return true;
+}
+
+// Plans and memory; res_on stays false where a cavity's solve cannot run resident.
+static int resident_batch_setup(cnv_batch* b) {
+    const cnv_params& p0 = b->ctx[0]->p;
+    const bool named = p0.sweeps_per_launch > 0 || p0.tile_waves > 0 || p0.wave_rows > 0;
+    std::vector<int> all(b->count);
+    b->last_k.assign(b->count, 0);
+    for (int i = 0; i < b->count; ++i) {
+        all[i] = i;
+        b->last_k[i] = b->ctx[i]->n;  // an optimally relaxed solve's sweeps go with n
+    }
+    // the shape named, or the one that is expected to finish first
+    TileShape sh{0, 0, 0};
+    double best = 0.0;
+    for (const ResidentBatchShape& c : b->dc ? resident_batch_shapes<float>() : resident_batch_shapes<double>()) {
+        if (named && (b->shape.s != c.shape.s || b->shape.nw != c.shape.nw || b->shape.rb != c.shape.rb)) continue;
+        bool fits = true;  // 8 rows a wave: dx = dy only
+        for (int i = 0; i < b->count; ++i) fits = fits && (c.shape.rb < 8 || b->ctx[i]->p.dx == b->ctx[i]->p.dy);
+        if (!fits) continue;
+        b->plan.assign(b->count, ResidentPlan{});
+        for (int i = 0; i < b->count; ++i) resident_layout(b->ctx[i]->n, !b->dc, c.shape, &b->plan[i]);
+        ResidentSchedule sc;
+        if (!resident_schedule(b, all, &sc)) continue;
+        if (sh.s == 0 || sc.length * c.us < best) {
+            best = sc.length * c.us;
+            sh = c.shape;
+        }
+    }
+    if (sh.s == 0) return CNV_OK;
+    long long words = 0;
+    for (int i = 0; i < b->count; ++i) {
+        b->plan[i] = ResidentPlan{};
+        resident_layout(b->ctx[i]->n, !b->dc, sh, &b->plan[i]);
+        words += (b->plan[i].words + 15) / 16 * 16;
+    }
+    const int blocks = kBands * kPerXcd;
+    BHIP(b, hipMalloc(&b->d_rwords, sizeof(*b->d_rwords) * words));
+    if (!b->dc && !resident_snap_lds(sh.nw, sh.rb))
+        BHIP(b, hipMalloc(&b->d_rsnap, sizeof(double) * 2 * (size_t)blocks * sh.nw * sh.rb * 128));
+    BHIP(b, hipMalloc(&b->d_rcount, sizeof(int) * (kQueueCounters + kClaimStride)));
+    words = 0;
+    std::vector<ResidentReset> rr;
+    std::vector<SorArgs<double>> a64[2];
+    std::vector<SorArgs<float>> a32;
+    for (int i = 0; i < b->count; ++i) {
+        ResidentPlan& p = b->plan[i];
+        resident_bind(&p, b->d_rwords + words, b->d_rsnap, b->d_ctl + 2 * i);
+        p.r.abort = p.reset.abort = b->d_rcount + kQueueCounters;
+        p.r.spins = kBatchSpins;
+        words += (p.words + 15) / 16 * 16;
+        rr.push_back(p.reset);
+        cnv_ctx* c = b->ctx[i];
+        auto tiled = [&](auto a) {
+            a.ctl = b->d_ctl + 2 * i;
+            a.tiles_i = p.tiles_i;
+            a.tiles_j = p.tiles_j;
+            return a;
+        };
+        for (int w = 0; w < 2; ++w) a64[w].push_back(tiled(sor_args64(c, c->w[w], 1)));
+        if (b->dc) {
+            a32.push_back(tiled(sor_args32(c)));
+            a32.back().test_mask = inner_test_every(c->p, 1) - 1;
+        }
+    }
+    int rc = upload(b, &b->d_rreset, rr);
+    for (int w = 0; w < 2 && !rc && !b->dc; ++w) rc = upload(b, &b->d_rargs64[w], a64[w]);
+    if (!rc && b->dc) rc = upload(b, &b->d_rargs32, a32);
+    b->res_shape = sh;
+    b->res_on = rc == CNV_OK;
+    return rc;
+}
+
+// The queues of the cavities in `todo`.
+static int resident_queues(cnv_batch* b, const std::vector<int>& todo) {
+    ResidentSchedule sc;
+    if (!resident_schedule(b, todo, &sc)) return bfail(b, CNV_ERR_ARG, "a cavity does not fit the GPU");
+    const std::vector<int>& order = sc.order;
+    const std::vector<ResidentJob>* jobs = sc.jobs;
+    // a deciding wave for each of the solves that run at once; later ones take the earlier ones' waves
+    const int deciders = std::min(kBands, ((int)order.size() + 15) / 16);
+    std::vector<ResidentJob> all;
+    for (int x = 0; x < kBands; ++x) {
+        b->queues.start[x] = (int)all.size();
+        all.insert(all.end(), jobs[x].begin(), jobs[x].end());
+    }
+    b->queues.start[kBands] = (int)all.size();
+    int rc = upload(b, &b->d_jobs, all);
+    if (!rc) rc = upload(b, &b->d_order, order);
+    b->queues.jobs = b->d_jobs;
+    b->queues.order = b->d_order;
+    b->queues.count = (int)order.size();
+    b->queues.deciders = deciders;
+    b->queues.counters = b->d_rcount;
+    return rc;
+}
+
+// The solves of every live cavity (FP32: the inner solves of one outer iteration) in resident
+// kernels, on slots and memory that the init kernel before has reset.  *ran: they have ended (final
+// slot 1, snaps); else they are as before, and the init kernel is to be repeated if *spoilt.
+static int run_batch_resident(cnv_batch* b, bool fp32, std::vector<SorCtl>& snaps, bool* ran, bool* spoilt) {
+    *ran = *spoilt = false;
+    if (!b->res_on || !resident_enter(b->device, kPerXcd)) return CNV_OK;
+    const size_t per = (size_t)2 * b->count;
+    auto body = [&]() -> int {
+        std::vector<int> todo;
+        for (int i = 0; i < b->count; ++i)
+            if (b->alive[i]) todo.push_back(i);
+        std::vector<SorResident> res(b->count);
+        for (int i = 0; i < b->count; ++i) {
+            res[i] = b->plan[i].r;
+            res[i].dst = 1;
+            res[i].wslot = 1;
+        }
+        int rc = CNV_OK;
+        if (b->res_dirty) {
+            rc = resident_queues(b, todo);
+            if (!rc) rc = upload(b, &b->d_res, res);
+            if (rc) return rc;
+            b->res_dirty = false;
+        }
+        snaps.resize(b->count);
+        bool again = false;
+        while (true) {
+            const int e = fp32 ? sor_resident_batch_launch<float>(b->d_rargs32, b->d_res, b->queues, b->res_shape,
+                                                                  kBands * kPerXcd, b->gs, b->stream)
+                               : sor_resident_batch_launch<double>(b->d_rargs64[b->wcur], b->d_res, b->queues,
+                                                                   b->res_shape, kBands * kPerXcd, b->gs, b->stream);
+            if (e) return bfail(b, CNV_ERR_HIP, "batched resident launch failed: %s", hipGetErrorString(hipGetLastError()));
+            int* const h_abort = reinterpret_cast<int*>(b->h_ctl + per);
+            BHIP(b, hipMemcpyAsync(b->h_ctl, b->d_ctl, sizeof(SorCtl) * per, hipMemcpyDeviceToHost, b->stream));
+            BHIP(b, hipMemcpyAsync(h_abort, b->d_rcount + kQueueCounters, sizeof(int), hipMemcpyDeviceToHost, b->stream));
+            BHIP(b, hipStreamSynchronize(b->stream));
+            if (*h_abort) {
+                *spoilt = true;
+                return CNV_OK;
+            }
+            // what is left: solves of more epochs than one kernel runs, and those to be run again to
+            // exactly their last sweep
+            std::vector<int> left;
+            for (int i : todo) {
+                const SorCtl st = b->h_ctl[2 * i + 1];
+                SorResident& r = res[i];
+                if (sor_done(st.status) && (st.rb_n != kNotStored || r.stop > 0)) {
+                    snaps[i] = st;
+                    continue;
+                }
+                left.push_back(i);
+                if (sor_done(st.status)) {
+                    r.stop = st.k;  // from the same slot and plane
+                } else {
+                    const int planes = fp32 ? 2 : 3;
+                    r.src = r.dst;
+                    r.dst = (r.dst + 1) % planes;
+                    r.launch0 += r.epochs;
+                    BHIP(b, hipMemcpyAsync(b->d_ctl + 2 * i, b->d_ctl + 2 * i + 1, sizeof(SorCtl), hipMemcpyDeviceToDevice,
+                                           b->stream));
+                }
+                if (resident_reset_launch(b->plan[i].reset, b->stream))
+                    return bfail(b, CNV_ERR_HIP, "resident reset failed: %s", hipGetErrorString(hipGetLastError()));
+            }
+            if (left.empty()) break;
+            again = true;
+            todo = left;
+            ResidentReset counters{};
+            counters.base = reinterpret_cast<unsigned long long*>(b->d_rcount);
+            counters.zero = kQueueCounters / 2;
+            counters.abort = b->d_rcount + kQueueCounters;
+            if (resident_reset_launch(counters, b->stream))
+                return bfail(b, CNV_ERR_HIP, "resident reset failed: %s", hipGetErrorString(hipGetLastError()));
+            BHIP(b, hipStreamSynchronize(b->stream));
+            rc = resident_queues(b, todo);
+            if (!rc) rc = upload(b, &b->d_res, res);
+            if (rc) return rc;
+        }
+        if (again) b->res_dirty = true;
+        b->fin_slot = 1;
+        *ran = true;
+        return CNV_OK;
+    };
+    const int rc = body();
+    if (rc) (void)hipStreamSynchronize(b->stream);
+    resident_leave(b->device, kPerXcd);
+    if (*spoilt) b->res_on = false;
+    return rc;
+}
+
 static int batch_one_step(cnv_batch* b, cnv_step_stats* stats) {
     const int cnt = b->count;
     const int win = b->wcur;
@@ -467,6 +752,7 @@ static int batch_one_step(cnv_batch* b, cnv_step_stats* stats) {
         if (!rc) rc = build_sor(b, b->shape);
         if (rc) return rc;
         b->maps_dirty = false;
+        b->res_dirty = true;
     }
     int nalive = 0;
     for (int i = 0; i < cnt; ++i) nalive += b->alive[i];
@@ -490,14 +776,22 @@ static int batch_one_step(cnv_batch* b, cnv_step_stats* stats) {
     b->wcur ^= 1;
     for (int i = 0; i < cnt; ++i)  // a diverged cavity keeps the buffers it was left in
         if (b->alive[i]) b->ctx[i]->wcur = b->wcur;
-    hipLaunchKernelGGL(batch_poisson_init_kernel, dim3(b->nb_lin), dim3(kBlock), 0, b->stream, b->d_items,
-                       b->d_map_lin);
-    BLAUNCH(b);
+    const auto init = [&]() -> int {
+        hipLaunchKernelGGL(batch_poisson_init_kernel, dim3(b->nb_lin), dim3(kBlock), 0, b->stream, b->d_items,
+                           b->d_map_lin, !b->dc && b->res_on ? b->d_rreset : nullptr, b->d_rcount);
+        BLAUNCH(b);
+        return CNV_OK;
+    };
+    int rci = init();
+    if (rci) return rci;
 
     std::vector<SorCtl> fin(cnt), snaps;
     std::vector<int> outer(cnt, 0), total(cnt, 0), active(b->alive);
+    bool ran = false, spoilt = false;
     if (!b->dc) {
-        int rc = run_sor_batch(b, false, snaps);
+        int rc = run_batch_resident(b, false, snaps, &ran, &spoilt);
+        if (!rc && spoilt) rc = init();
+        if (!rc && !ran) rc = run_sor_batch(b, false, snaps);
         if (rc) return rc;
         fin = snaps;
     } else {
@@ -518,11 +812,18 @@ static int batch_one_step(cnv_batch* b, cnv_step_stats* stats) {
             hipLaunchKernelGGL(batch_dc_residual_kernel, dim3(b->nb_cell), dim3(kBlock), 0, b->stream, b->d_items,
                                b->d_map_cell, b->d_dc, b->wcur);
             BLAUNCH(b);
-            hipLaunchKernelGGL(batch_dc_inner_init_kernel, dim3(b->nb_lin), dim3(kBlock), 0, b->stream, b->d_items,
-                               b->d_map_lin, b->d_dc, b->rtol);
-            BLAUNCH(b);
+            const auto inner_init = [&]() -> int {
+                hipLaunchKernelGGL(batch_dc_inner_init_kernel, dim3(b->nb_lin), dim3(kBlock), 0, b->stream, b->d_items,
+                                   b->d_map_lin, b->d_dc, b->rtol, b->res_on ? b->d_rreset : nullptr, b->d_rcount);
+                BLAUNCH(b);
+                return CNV_OK;
+            };
+            int rc = inner_init();
+            if (rc) return rc;
             b->k_prev = o < cnv_batch::kDcPred ? b->k_dc[o] : 0;  // this outer iteration's last length
-            int rc = run_sor_batch(b, true, snaps);
+            rc = run_batch_resident(b, true, snaps, &ran, &spoilt);
+            if (!rc && spoilt) rc = inner_init();
+            if (!rc && !ran) rc = run_sor_batch(b, true, snaps);
             if (rc) return rc;
             hipLaunchKernelGGL(batch_dc_correct_kernel, dim3(b->nb_lin), dim3(kBlock), 0, b->stream, b->d_items,
                                b->d_map_lin, b->d_dc, b->fin_slot);
@@ -550,6 +851,12 @@ static int batch_one_step(cnv_batch* b, cnv_step_stats* stats) {
     for (int i = 0; i < cnt; ++i)
         if (b->alive[i]) kmax = std::max(kmax, b->dc ? 0 : fin[i].k);
     if (!b->dc) b->k_prev = kmax;
+    if (b->res_on && b->order_steps < 2) {  // the queues follow the solves' lengths, as the first steps show them
+        ++b->order_steps;
+        for (int i = 0; i < cnt; ++i)
+            if (b->alive[i]) b->last_k[i] = fin[i].k;
+        b->res_dirty = true;
+    }
 
     if (b->dc && b->transport_fp32)
         hipLaunchKernelGGL((batch_velocity_kernel<true, true>), dim3(b->nb_cell), dim3(kBlock), 0, b->stream,
@@ -607,7 +914,9 @@ void cnv_batch_destroy(cnv_batch* b) {
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     for (cnv_ctx* c : b->ctx) cnv_destroy(c);
     void* dev[] = {b->d_items, b->d_ctl, b->d_diag, b->d_partial, b->d_args64[0], b->d_args64[1], b->d_args32,
-                   b->d_dc, b->d_map_edge, b->d_map_cell, b->d_map_lin, b->d_map_sor};
+                   b->d_dc, b->d_map_edge, b->d_map_cell, b->d_map_lin, b->d_map_sor,
+                   b->d_rwords, b->d_rsnap, b->d_rcount, b->d_res, b->d_rreset, b->d_rargs64[0], b->d_rargs64[1],
+                   b->d_rargs32, b->d_jobs, b->d_order};
     for (void* p : dev)
         if (p) (void)hipFree(p);
     if (b->h_ctl) (void)hipHostFree(b->h_ctl);
@@ -711,6 +1020,7 @@ int cnv_batch_create(const cnv_params* items, int count, cnv_batch** out) {
         // a one-cavity default follows that cavity's size, a batch's spans its cavities
         const bool named = p0.sweeps_per_launch > 0 || p0.tile_waves > 0 || p0.wave_rows > 0;
         if (!rc) rc = build_sor(b, named ? b->ctx[0]->shape : TileShape{5, 16, 4});
+        if (!rc) rc = resident_batch_setup(b);
         if (!rc) BHIP(b, hipDeviceSynchronize());
         return rc;
     };

@@ -122,6 +122,7 @@ constexpr unsigned long long kMark64 = 0x7ff4c0de0badc0deull;  // signalling NaN
 constexpr unsigned kMark32 = 0x7fa5c0deu;
 constexpr int kResidentRows = 16;  // doubles per tile and epoch of partial sums (128 bytes)
 constexpr int kClaimStride = 32;   // ints between two XCDs' counters (128 bytes)
+constexpr int kBands = 8;          // XCDs of an MI355X, each with a band of tile rows
 struct SorResident {
     void* exch;                // three planes of nr rows, pitch ldx, marked where nothing was given yet
     long long xplane;          // elements of one plane
@@ -133,15 +134,30 @@ struct SorResident {
     int blocks;                // workgroups of a launch
     int epochs, launch0;       // epochs at most; index of the first one within the solve
     int stop;                  // > 0: run to exactly this many sweeps of the solve, without tests
+    int spins;                 // polls of one wait before it is given up
     int src, dst;              // planes of the input and of the result
     int rslot, wslot;          // state slots read and written
     int* claim;                // [9][kClaimStride]: tiles taken on each XCD; the deciding workgroup
 };
-constexpr int kBands = 8;      // XCDs of an MI355X, each with a band of tile rows
 __host__ __device__ inline int band_start(int band, int tiles_i) { return band * tiles_i / kBands; }
 constexpr int kNotStored = -1;  // SorCtl::rb_n: the solve has ended, its iterate is not in plane `parity` yet
 // FP64 tiles whose two copies fit in LDS
 constexpr bool resident_snap_lds(int nw, int rb) { return nw * rb <= 32; }
+// Batched resident solves: a tile of a solve, in the band of its tile rows [row_lo, row_hi).
+struct ResidentJob {
+    int inst, tile, row_lo, row_hi;
+};
+// The tiles each XCD takes, in order, and the solves in the same order (sor_resident_batch_kernel).
+struct ResidentQueues {
+    const ResidentJob* jobs;
+    int start[kBands + 1];     // XCD x takes jobs [start[x], start[x + 1])
+    const int* order;
+    int count;                 // solves
+    int deciders;              // workgroups that decide, on XCDs 0 .. deciders - 1
+    int* counters;             // [2 * kBands + 1][kClaimStride], zeroed: workgroups arrived and jobs taken on
+                               // each XCD, solves taken by the deciders
+};
+constexpr int kQueueCounters = (2 * kBands + 1) * kClaimStride;
 // What one reset writes before a resident launch: marks over the exchange planes, marks over the
 // partial sums, zeros over the decision words and tile counters (in that order from base) and in the abort flag.
 struct ResidentReset {

@@ -258,6 +258,8 @@ inline int run_sor_launches(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* f
 // The plan for n x n grids on a device; base: the launches' shape, named: the caller chose it (then
 // that one or none; else an FP32 solve keeps its sweeps per launch).  false: they run as launches.
 bool resident_plan(int n, bool fp64, int dev, cnv::TileShape base, bool named, ResidentPlan* p);
+// The part of a plan that follows from the tile shape alone: tiles, memory, launch arguments.
+void resident_layout(int n, bool fp64, cnv::TileShape sh, ResidentPlan* p);
 // Gives a plan its memory: words and snap as it says, the solve's slots (the abort flag after them).
 void resident_bind(ResidentPlan* p, unsigned long long* words, double* snap, cnv::SorCtl* ctl);
 // Takes a plan's share of the device for the time of a solve (false: not now).

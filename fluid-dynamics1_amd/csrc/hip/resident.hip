@@ -26,6 +26,8 @@ constexpr int kMaxDevices = 64;
 // of 64, the longest test cadence of FP32 inner solves.
 constexpr int kEpochs = 1984;
 
+constexpr int kSpins = 1 << 20;  // polls of a wait: about 0.1 s
+
 std::atomic<int> g_units[kMaxDevices];  // CUs per XCD in use by resident solves
 
 // The shapes in order of speed; a solve takes the first whose tiles fit on the GPU together (an FP32
@@ -88,14 +90,22 @@ bool resident_plan(int n, bool fp64, int dev, TileShape base, bool named, Reside
         }
     }
     if (!slots) return false;
-    const TileShape sh = p->shape;
+    p->units = std::min(slots, per_xcd);
+    resident_layout(n, fp64, p->shape, p);
+    return true;
+}
+
+void resident_layout(int n, bool fp64, TileShape sh, ResidentPlan* p) {
+    SorResident& r = p->r;
+    p->shape = sh;
     p->tiles_i = (n + tile_rows(sh) - 1) / tile_rows(sh);
     p->tiles_j = (n + tile_cols(sh) - 1) / tile_cols(sh);
-    p->units = std::min(slots, per_xcd);
+    r.ntiles = p->tiles_i * p->tiles_j;
     // exchange rows start on 128-byte lines: rows of two bands share none
     r.ldx = (n + 1 + 31) / 32 * 32;
     r.xplane = (long long)r.ldx * n;
     r.epochs = kEpochs;
+    r.spins = kSpins;
     ResidentReset& rr = p->reset;
     rr.exch = 3 * r.xplane / (fp64 ? 1 : 2);
     rr.part = 4LL * r.ntiles * kResidentRows;
@@ -103,7 +113,6 @@ bool resident_plan(int n, bool fp64, int dev, TileShape base, bool named, Reside
     rr.mark = fp64 ? kMark64 : ((unsigned long long)kMark32 << 32 | kMark32);
     p->words = rr.exch + rr.part + rr.zero;
     p->snap = fp64 && !resident_snap_lds(sh.nw, sh.rb) ? 2LL * r.ntiles * sh.nw * sh.rb * 128 : 0;
-    return true;
 }
 
 void resident_bind(ResidentPlan* p, unsigned long long* words, double* snap, SorCtl* ctl) {

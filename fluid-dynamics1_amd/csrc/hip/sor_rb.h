@@ -175,9 +175,18 @@ __device__ inline T* sor_plane(const SorArgs<T>& a, int idx) {
     else return idx == 0 ? a.psi0 : (idx == 1 ? a.psi1 : a.psi2);
 }
 
+// A tile's LDS: the waves' first and last rows, and one column per thread of per-lane sums.
+template <typename T, int NW, int SE, bool kNorm>
+struct SorShared {
+    T xch[2][NW][2][64];  // [half-sweep parity][wave][first/last row][lane]
+    double lred[SE][NW * 64];  // this launch's per-lane L1 update sums, one row per summed sweep
+    double lnrm[kNorm ? NW * 64 : 1];  // the per-lane iterate norm after the last sweep
+};
+
 // A workgroup's tile in registers (NW waves of 64 lanes): wave w holds rows [w*RB, w*RB + RB) of the
 // extended tile, lane m columns 2m and 2m+1.
-template <typename T, int S, int NW, int RB, bool GS, bool XR, bool NORM>
+// ISO (FP32): dx = dy, the two stencil coefficients of a point are one number and held once.
+template <typename T, int S, int NW, int RB, bool GS, bool XR, bool NORM, bool ISO = false>
 struct SorTile {
     static constexpr int H = 2 * S;
     static constexpr int EJ = 128;  // extended tile columns; lane m holds columns 2m, 2m+1
@@ -199,18 +208,13 @@ struct SorTile {
     typedef typename std::conditional<sizeof(T) == 4, float, double>::type Acc;
     typedef typename PairOf<T>::type Pair;
 
-    // LDS: the waves' first and last rows, and one column per thread of per-lane sums
-    struct Shared {
-        T xch[2][NW][2][64];  // [half-sweep parity][wave][first/last row][lane]
-        double lred[SE][NW * 64];  // this launch's per-lane L1 update sums, one row per summed sweep
-        double lnrm[kNorm ? NW * 64 : 1];  // the per-lane iterate norm after the last sweep
-    };
+    typedef SorShared<T, NW, SE, kNorm> Shared;
 
     T v[2][RB];   // v[q][r]: value at (row0 + r, 2*lane + q)
     T fc[2][RB];  // FP64: c3*f (the hoisted c3*f product of the update); FP32: -be*c3*f
     T be[2][RB];  // FP64: bcoef at interior points, 0 on the domain boundary and outside it
     T cn[2][RB];  // FP32: be*c1 and be*c2, the relaxation folded into the stencil coefficients
-    T ce[2][RB];
+    T ce[2][ISO ? 1 : RB];
     Acc w[RB];    // 1 for owned rows inside the domain, else 0 (wave-uniform)
     T c1, c2, B, rB, omb;
     int gi0, gj0, gj, lane, wv, row0, nr, nc;
@@ -282,7 +286,7 @@ struct SorTile {
                 } else {
                     fc[q][r] = inter ? bcoef * -(c3s * fq) : T(0);
                     cn[q][r] = rint ? cncol[q] : T(0);
-                    ce[q][r] = rint ? cecol[q] : T(0);
+                    if constexpr (!ISO) ce[q][r] = rint ? cecol[q] : T(0);
                 }
             }
         }
@@ -362,7 +366,7 @@ struct SorTile {
                     }
                 } else {
                     // relaxation and 1/B folded into cn, ce and fc (0 where the point is fixed)
-                    const T x = __fmaf_rn(cn[q][r], up + dn, __fmaf_rn(ce[q][r], own + far, fc[q][r]));
+                    const T x = __fmaf_rn(cn[q][r], up + dn, __fmaf_rn(ISO ? cn[q][r] : ce[q][ISO ? 0 : r], own + far, fc[q][r]));
                     cand = GS ? x : __fmaf_rn(omb, old, x);
                     v[q][r] = cand;
                     if (kL1 && with_norm) {

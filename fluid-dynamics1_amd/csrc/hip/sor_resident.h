@@ -38,13 +38,14 @@
 // repeats the epochs with sor_rb.h's launches from the kernel's input plane, which it never writes.
 #pragma once
 
+#include <vector>
+
 #include "sor_rb.h"
 
 namespace cnv {
 
 typedef unsigned long long u64;
 constexpr double kNearTol = 4.0;     // an update within this factor of its tolerance may end the solve soon
-constexpr int kSpinLimit = 1 << 20;  // polls of one wait (about 0.1 s)
 constexpr int kAgent = 16;           // cache policy bits of buffer accesses: sc1, agent scope
 
 template <typename T> struct Marked;
@@ -83,6 +84,9 @@ __device__ __forceinline__ void agent_store(u64* p, u64 x) { __hip_atomic_store(
 __device__ __forceinline__ void report_abort(const SorResident& r) {
     __hip_atomic_store(r.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ bool gave_up(const SorResident& r) {
+    return __builtin_amdgcn_readfirstlane(__hip_atomic_load(r.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
+}
 // every memory operation this wave has issued is complete
 __device__ __forceinline__ void wait_memory() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -98,17 +102,23 @@ __device__ __forceinline__ u64 res_word(int decided, bool near, bool near_before
            (unsigned)redo;
 }
 
-// One tile's workgroup: tile (ti, tj), in the band `band` of tile rows [row_lo, row_hi).
-template <typename T, int S, int NW, int RB, bool GS, bool XR, bool NORM>
+typedef double SnapPair __attribute__((ext_vector_type(2)));
+// pairs of the two kept epoch starts in LDS
+template <typename T, int NW, int RB>
+constexpr int kSnapPairs = sizeof(T) == 8 && resident_snap_lds(NW, RB) ? 2 * RB * NW * 64 : 1;
+
+// One tile's workgroup: tile (ti, tj), in the band of tile rows [row_lo, row_hi) that one XCD holds;
+// snap_part: which part of r.snap is its own.
+template <typename T, int S, int NW, int RB, bool GS, bool XR, bool NORM, bool ISO = false>
 __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const SorResident& r, const int ti, const int tj,
-                                                  const int row_lo, const int row_hi) {
-    typedef SorTile<T, S, NW, RB, GS, XR, NORM> Tile;
+                                                  const int row_lo, const int row_hi, const int snap_part,
+                                                  typename SorTile<T, S, NW, RB, GS, XR, NORM>::Shared& sh,
+                                                  SnapPair* const snap_lds) {
+    typedef SorTile<T, S, NW, RB, GS, XR, NORM, ISO> Tile;
     constexpr int H = Tile::H, TI = Tile::TI, TJ = Tile::TJ;
     constexpr bool kSnap = sizeof(T) == 8;
     constexpr bool kSnapLds = kSnap && resident_snap_lds(NW, RB);
-    typedef double Two __attribute__((ext_vector_type(2)));
-    __shared__ typename Tile::Shared sh;
-    __shared__ Two snap_lds[kSnapLds ? 2 * RB * NW * 64 : 1];
+    typedef SnapPair Two;
 
     const int tile = ti * a.tiles_j + tj;
     const SorCtl* P = a.ctl + r.rslot;
@@ -154,7 +164,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
         }
     };
 
-    bool dead = false;
+    bool dead = gave_up(r);  // a batch's kernel goes on to other tiles after a wave has given up
     const u64* dec = r.dec + (size_t)tile * 8;
     // the halo cells of plane `slot` (slot < 0: none) and a decision on `decided` epochs (0: none)
     auto take = [&](int slot, int decided) -> u64 {
@@ -172,7 +182,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
             }
             if (decided) ok = ok && (int)(word >> 32) >= decided;
             if (__all(ok) || dead) break;
-            if (spins >= kSpinLimit) {
+            if (spins >= r.spins) {
                 dead = true;
                 report_abort(r);
             }
@@ -183,7 +193,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     };
 
     // the values at an epoch's start, in two turns (FP64)
-    Two* const mem = kSnapLds ? nullptr : reinterpret_cast<Two*>(r.snap) + (size_t)tile * 2 * RB * NW * 64;
+    Two* const mem = kSnapLds ? nullptr : reinterpret_cast<Two*>(r.snap) + (size_t)snap_part * 2 * RB * NW * 64;
     auto snap_at = [&](int turn, int rr) -> Two* {
         const int q = (turn * RB + rr) * NW * 64 + (int)threadIdx.x;
         return kSnapLds ? snap_lds + q : mem + q;
@@ -280,70 +290,164 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     t.store(a, dst);
 }
 
+// The decisions on a solve's epochs, one after the other; the state of the solve.
+template <typename T, int S, int NW, int RB, bool NORM>
+struct ResidentDecider {
+    static constexpr bool kNorm = sizeof(T) == 4 || NORM;
+    static constexpr bool kLastOnly = sizeof(T) == 4;
+    static constexpr int SE = kLastOnly ? 1 : S;
+    static constexpr int nq = SE + (kNorm ? 1 : 0);
+    // whether the tiles of this kernel keep their values at the start of every epoch, and, else, of
+    // this epoch and the next (what the decisions on the epochs two and one before said)
+    static constexpr bool kAlways = sizeof(T) == 4 || resident_snap_lds(NW, RB);
+    bool kept = true, kept_next = true;
+    int itmax, k, status, launches, rb_n = 0;
+    double tol, rtol, e_last, n_last;
+    int e = 0, k_prev, sd;
+    bool last, tested;
+    unsigned code;
+
+    // false: the solve of slot rslot has ended before, and slot wslot says so too
+    __device__ __forceinline__ bool begin(SorCtl* ctl, const SorResident& r, const bool writes) {
+        const SorCtl* p = ctl + r.rslot;
+        itmax = p->itmax;
+        k = p->k;
+        status = p->status;
+        launches = p->launches;
+        tol = p->tol;
+        rtol = p->rtol;
+        e_last = p->e_last;
+        n_last = p->n_last;
+        if (status == SOR_RUNNING) return true;
+        if (writes) ctl[r.wslot] = *p;
+        return false;
+    }
+    __device__ __forceinline__ void end(SorCtl* ctl, const SorResident& r) const {
+        SorCtl* p = ctl + r.wslot;
+        p->k = k;
+        p->parity = r.dst;
+        p->status = status;
+        p->s_done = 0;
+        p->launches = launches;
+        p->itmax = itmax;
+        p->rb_src = 0;
+        p->rb_n = rb_n;
+        p->e_last = e_last;
+        p->tol = tol;
+        p->rtol = rtol;
+        p->n_last = n_last;
+    }
+    __device__ __forceinline__ void epoch(const SorResident& r, const int test_mask) {
+        k_prev = k;
+        const int budget = itmax - k_prev;
+        sd = budget < S ? budget : S;
+        last = e + 1 == r.epochs || budget <= S;
+        tested = sizeof(T) == 8 || ((r.launch0 + e) & test_mask) == test_mask;
+        code = RES_CONTINUE;
+        k = k_prev + sd;
+        launches += 1;
+    }
+    // the sums of one tile's epoch, marked again
+    __device__ __forceinline__ void sums(const SorResident& r, const int tile, double (&x)[nq], bool& dead) const {
+        const int nupd = kLastOnly ? 1 : sd;
+        u64* pp = reinterpret_cast<u64*>(r.part + ((size_t)(e & 3) * r.ntiles + tile) * kResidentRows);
+        for (int spins = 0;; ++spins) {
+            bool ok = true;
+#pragma unroll
+            for (int i = 0; i < nq; ++i) x[i] = __longlong_as_double((long long)agent_load(pp + i));
+#pragma unroll
+            for (int i = 0; i < nq; ++i)
+                if (i < nupd || i >= SE) ok = ok && Marked<double>::ready(x[i]);
+            if (ok || dead) break;
+            if (spins >= r.spins) {
+                dead = true;
+                report_abort(r);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < nq; ++i) {
+            if (i >= nupd && i < SE) x[i] = 0.0;  // no such sweep in a budget's last epoch
+            agent_store(pp + i, kMark64);
+        }
+    }
+    // the decision on the epoch with the sums tot (as sor_rb_decider's): the tiles' word
+    __device__ __forceinline__ u64 decide(const double (&tot)[nq]) {
+        const double ntot = kNorm ? tot[nq - 1] : 0.0;
+        int s_conv = -1, s_fold = -1, s_bad = -1, redo = 0;
+#pragma unroll
+        for (int i = 0; i < SE; ++i) {
+            const int s = kLastOnly ? sd - 1 : i;
+            if (s < sd && s_conv < 0 && s_fold < 0 && s_bad < 0) {
+                if (!(tot[i] <= DBL_MAX)) s_bad = s;
+                else if (tot[i] < tol) s_conv = s;
+                else if (rtol > 0.0 && tot[i] < rtol * ntot) s_fold = s;
+            }
+        }
+        if (kNorm && s_conv < 0 && s_fold < 0 && s_bad < 0 && !(ntot <= DBL_MAX)) s_bad = sd - 1;
+        const bool inner = s_conv >= 0 && s_conv < sd - 1;
+        const int s_rep = inner ? s_conv : sd - 1;  // reported sweep
+#pragma unroll
+        for (int i = 0; i < SE; ++i)
+            if ((kLastOnly ? sd - 1 : i) == s_rep) e_last = tot[i];
+        n_last = ntot;
+        if (inner) {
+            code = RES_REDO;
+            redo = s_conv + 1;
+            k = k_prev + redo;
+            status = SOR_CONVERGED;
+        } else if (s_conv >= 0 || s_fold >= 0 || s_bad >= 0) {
+            code = RES_END;
+            status = s_conv >= 0 ? SOR_CONVERGED : (s_fold >= 0 ? SOR_FOLD : SOR_DIVERGED);
+        }
+        if (!kAlways && code != RES_CONTINUE) {
+            // the end of this epoch is the next one's start (the tile's own values, if last)
+            if (code == RES_END && !last && !kept_next) {
+                code = RES_REDO;
+                redo = sd;
+            }
+            if (code == RES_REDO && !kept) {
+                code = RES_RERUN;
+                rb_n = kNotStored;
+            }
+        }
+        const bool near = e_last < kNearTol * tol || (rtol > 0.0 && e_last < kNearTol * rtol * ntot);
+        const u64 word = res_word(e + 1, near, kept_next, code, redo);
+        kept = kept_next;
+        kept_next = near;
+        return word;
+    }
+    __device__ __forceinline__ bool ended() {
+        if (code == RES_CONTINUE && k >= itmax) status = SOR_FAILED;
+        return code != RES_CONTINUE || last;
+    }
+};
+
 // The deciding workgroup: after each tested epoch the decision of sor_rb_decider on its sums, left
 // in every tile's word; at the end the solve's state in slot wslot.
 template <typename T, int S, int NW, int RB, bool NORM>
 __device__ __forceinline__ void sor_resident_decider(const SorArgs<T>& a, const SorResident& r) {
-    constexpr bool kNorm = sizeof(T) == 4 || NORM;
-    constexpr bool kLastOnly = sizeof(T) == 4;
-    constexpr int SE = kLastOnly ? 1 : S;
-    constexpr int nq = SE + (kNorm ? 1 : 0);
+    typedef ResidentDecider<T, S, NW, RB, NORM> Decider;
+    constexpr int nq = Decider::nq;
     constexpr int NT = NW * 64;
     __shared__ double lw[NW][nq];
-    const SorCtl P = a.ctl[r.rslot];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (r.stop > 0) return;  // the slot holds the solve's end already
-    if (P.status != SOR_RUNNING) {
-        if (tid == 0) a.ctl[r.wslot] = P;
-        return;
-    }
-    // whether the tiles of this kernel keep their values at the start of every epoch, and, else, of
-    // this epoch and the next (what the decisions on the epochs two and one before said)
-    constexpr bool kAlways = sizeof(T) == 4 || resident_snap_lds(NW, RB);
-    bool kept = true, kept_next = true;
+    Decider d;
+    if (!d.begin(a.ctl, r, tid == 0)) return;
     const int nwp = min(NW, (r.ntiles + 63) >> 6);  // waves holding partials
-    SorCtl next = P;
-    next.s_done = 0;
-    next.parity = r.dst;
-    next.rb_n = 0;
     bool dead = false;
-    for (int e = 0;; ++e) {
-        const int k_prev = next.k;
-        const int budget = P.itmax - k_prev;
-        const int sd = budget < S ? budget : S;
-        const bool last = e + 1 == r.epochs || budget <= S;
-        const bool tested = sizeof(T) == 8 || ((r.launch0 + e) & a.test_mask) == a.test_mask;
-        unsigned code = RES_CONTINUE;
-        int redo = 0;
-        next.k = k_prev + sd;
-        next.launches += 1;
-        if (tested) {
-            const int nupd = kLastOnly ? 1 : sd;
-            double pv[nq];
+    for (;; ++d.e) {
+        d.epoch(r, a.test_mask);
+        if (d.tested) {
+            double pv[nq], tot[nq];
 #pragma unroll
             for (int i = 0; i < nq; ++i) pv[i] = 0.0;
             for (int t = tid; t < r.ntiles; t += NT) {
-                u64* pp = reinterpret_cast<u64*>(r.part + ((size_t)(e & 3) * r.ntiles + t) * kResidentRows);
                 double x[nq];
-                for (int spins = 0;; ++spins) {
-                    bool ok = true;
+                d.sums(r, t, x, dead);
 #pragma unroll
-                    for (int i = 0; i < nq; ++i) x[i] = __longlong_as_double((long long)agent_load(pp + i));
-#pragma unroll
-                    for (int i = 0; i < nq; ++i)
-                        if (i < nupd || i >= SE) ok = ok && Marked<double>::ready(x[i]);
-                    if (ok || dead) break;
-                    if (spins >= kSpinLimit) {
-                        dead = true;
-                        report_abort(r);
-                    }
-                }
-#pragma unroll
-                for (int i = 0; i < nq; ++i) {
-                    if (i < nupd || i >= SE) pv[i] += x[i];
-                    agent_store(pp + i, kMark64);
-                }
+                for (int i = 0; i < nq; ++i) pv[i] += x[i];
             }
             if (wv < nwp) {
                 wave_sum_n(pv);
@@ -354,67 +458,60 @@ __device__ __forceinline__ void sor_resident_decider(const SorArgs<T>& a, const 
             }
             wait_memory();  // the marks come before the decision that lets a tile write there again
             __syncthreads();
-            double etot[SE], ntot = 0.0;
 #pragma unroll
-            for (int s = 0; s < SE; ++s) {
-                etot[s] = 0.0;
-                for (int j = 0; j < nwp; ++j) etot[s] += lw[j][s];
+            for (int i = 0; i < nq; ++i) {
+                tot[i] = 0.0;
+                for (int j = 0; j < nwp; ++j) tot[i] += lw[j][i];
             }
-            if (kNorm)
-                for (int j = 0; j < nwp; ++j) ntot += lw[j][nq - 1];
-            int s_conv = -1, s_fold = -1, s_bad = -1;
-#pragma unroll
-            for (int i = 0; i < SE; ++i) {
-                const int s = kLastOnly ? sd - 1 : i;
-                if (s < sd && s_conv < 0 && s_fold < 0 && s_bad < 0) {
-                    if (!(etot[i] <= DBL_MAX)) s_bad = s;
-                    else if (etot[i] < P.tol) s_conv = s;
-                    else if (P.rtol > 0.0 && etot[i] < P.rtol * ntot) s_fold = s;
-                }
-            }
-            if (kNorm && s_conv < 0 && s_fold < 0 && s_bad < 0 && !(ntot <= DBL_MAX)) s_bad = sd - 1;
-            const bool inner = s_conv >= 0 && s_conv < sd - 1;
-            const int s_rep = inner ? s_conv : sd - 1;  // reported sweep
-#pragma unroll
-            for (int i = 0; i < SE; ++i)
-                if ((kLastOnly ? sd - 1 : i) == s_rep) next.e_last = etot[i];
-            next.n_last = ntot;
-            if (inner) {
-                code = RES_REDO;
-                redo = s_conv + 1;
-                next.k = k_prev + redo;
-                next.status = SOR_CONVERGED;
-            } else if (s_conv >= 0 || s_fold >= 0 || s_bad >= 0) {
-                code = RES_END;
-                next.status = s_conv >= 0 ? SOR_CONVERGED : (s_fold >= 0 ? SOR_FOLD : SOR_DIVERGED);
-            }
-            if (!kAlways && code != RES_CONTINUE) {
-                // the end of this epoch is the next one's start (the tile's own values, if last)
-                if (code == RES_END && !last && !kept_next) {
-                    code = RES_REDO;
-                    redo = sd;
-                }
-                if (code == RES_REDO && !kept) {
-                    code = RES_RERUN;
-                    next.rb_n = kNotStored;
-                }
-            }
-            const bool near = next.e_last < kNearTol * P.tol || (P.rtol > 0.0 && next.e_last < kNearTol * P.rtol * ntot);
-            const u64 word = res_word(e + 1, near, kept_next, code, redo);
-            kept = kept_next;
-            kept_next = near;
+            const u64 word = d.decide(tot);
             for (int t = tid; t < r.ntiles; t += NT) agent_store(r.dec + (size_t)t * 8, word);
             __syncthreads();  // lw is read before the next epoch's sums replace it
         }
-        if (code == RES_CONTINUE && next.k >= P.itmax) next.status = SOR_FAILED;
-        if (code != RES_CONTINUE || last) break;
+        if (d.ended()) break;
     }
-    if (tid == 0) a.ctl[r.wslot] = next;
+    if (tid == 0) d.end(a.ctl, r);
+}
+
+// The same by one wave, with the same sums in the same order.
+template <typename T, int S, int NW, int RB>
+__device__ __forceinline__ void sor_resident_wave_decider(const SorArgs<T>& a, const SorResident& r) {
+    typedef ResidentDecider<T, S, NW, RB, false> Decider;
+    constexpr int nq = Decider::nq;
+    const int lane = threadIdx.x & 63;
+    if (r.stop > 0) return;
+    Decider d;
+    if (!d.begin(a.ctl, r, lane == 0)) return;
+    bool dead = gave_up(r);
+    for (;; ++d.e) {
+        d.epoch(r, a.test_mask);
+        if (d.tested) {
+            double tot[nq];
+#pragma unroll
+            for (int i = 0; i < nq; ++i) tot[i] = 0.0;
+            for (int t0 = 0; t0 < r.ntiles; t0 += 64) {
+                double x[nq];
+#pragma unroll
+                for (int i = 0; i < nq; ++i) x[i] = 0.0;
+                if (t0 + lane < r.ntiles) d.sums(r, t0 + lane, x, dead);
+                wave_sum_n(x);
+#pragma unroll
+                for (int i = 0; i < nq; ++i) tot[i] += x[i];
+            }
+            wait_memory();
+            const u64 word = d.decide(tot);
+            for (int t = lane; t < r.ntiles; t += 64) agent_store(r.dec + (size_t)t * 8, word);
+        }
+        if (d.ended()) break;
+    }
+    if (lane == 0) d.end(a.ctl, r);
 }
 
 template <typename T, int S, int NW, int RB, bool GS, bool XR, bool NORM>
 __global__ void __launch_bounds__(NW * 64) sor_resident_kernel(SorArgs<T> a, SorResident r) {
     // the next free tile of this XCD's band; the first workgroup that finds none decides
+    typedef SorTile<T, S, NW, RB, GS, XR, NORM> Tile;
+    __shared__ typename Tile::Shared sh;
+    __shared__ SnapPair snap_lds[kSnapPairs<T, NW, RB>];
     __shared__ int place;
     const int band = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & (kBands - 1);  // hwreg XCC_ID
     const int row_lo = band_start(band, a.tiles_i), row_hi = band_start(band + 1, a.tiles_i);
@@ -427,10 +524,59 @@ __global__ void __launch_bounds__(NW * 64) sor_resident_kernel(SorArgs<T> a, Sor
     __syncthreads();
     const int at = __builtin_amdgcn_readfirstlane(place);
     if (at >= 0) {
-        const int ti = row_lo + at / a.tiles_j;
-        sor_resident_tile<T, S, NW, RB, GS, XR, NORM>(a, r, ti, at % a.tiles_j, row_lo, row_hi);
+        const int ti = row_lo + at / a.tiles_j, tj = at % a.tiles_j;
+        sor_resident_tile<T, S, NW, RB, GS, XR, NORM>(a, r, ti, tj, row_lo, row_hi, ti * a.tiles_j + tj, sh,
+                                                        snap_lds);
     } else if (at == -1) {
         sor_resident_decider<T, S, NW, RB, NORM>(a, r);
+    }
+}
+
+// Many solves in one launch, a workgroup per CU.  Each XCD has a queue of tiles, solve after solve, and
+// its workgroups take the next one whenever they have finished a tile, so a solve whose tiles find
+// no place yet waits for the ones before it while those run on.  The queues hold the solves in one
+// order, so the first unfinished solve always has its tiles next in line on every XCD it spans
+// (never more of them on one than that has workgroups): some solve can always run.  The waves of
+// the deciding workgroups take the solves in the same order.
+template <typename T, int S, int NW, int RB, bool GS>
+__global__ void __launch_bounds__(NW * 64) sor_resident_batch_kernel(const SorArgs<T>* __restrict__ args,
+                                                                     const SorResident* __restrict__ res,
+                                                                     ResidentQueues q) {
+    typedef SorTile<T, S, NW, RB, GS, true, false> Tile;
+    __shared__ typename Tile::Shared sh;
+    __shared__ SnapPair snap_lds[kSnapPairs<T, NW, RB>];
+    __shared__ int place;
+    const int xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & (kBands - 1);  // hwreg XCC_ID
+    if (threadIdx.x == 0) place = atomicAdd(q.counters + xcc * kClaimStride, 1);
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(place) == 0 && xcc < q.deciders) {
+        while (true) {
+            int c = 0;
+            if ((threadIdx.x & 63) == 0) c = atomicAdd(q.counters + 2 * kBands * kClaimStride, 1);
+            c = __builtin_amdgcn_readfirstlane(c);
+            if (c >= q.count) return;
+            const int i = q.order[c];
+            sor_resident_wave_decider<T, S, NW, RB>(args[i], res[i]);
+        }
+    }
+    while (true) {
+        __syncthreads();
+        if (threadIdx.x == 0) place = atomicAdd(q.counters + (kBands + xcc) * kClaimStride, 1);
+        __syncthreads();
+        const int at = q.start[xcc] + __builtin_amdgcn_readfirstlane(place);
+        if (at >= q.start[xcc + 1]) return;
+        const ResidentJob j = q.jobs[at];
+        const SorArgs<T>& a = args[j.inst];
+        const int ti = j.tile / a.tiles_j, tj = j.tile % a.tiles_j;
+        if constexpr (sizeof(T) == 8) {
+            if (!a.exact_rcp) {
+                sor_resident_tile<T, S, NW, RB, GS, false, false>(a, res[j.inst], ti, tj, j.row_lo, j.row_hi, blockIdx.x, sh,
+                                                                  snap_lds);
+                continue;
+            }
+        }
+        sor_resident_tile<T, S, NW, RB, GS, true, false, RB == 8>(a, res[j.inst], ti, tj, j.row_lo, j.row_hi, blockIdx.x,
+                                                                  sh, snap_lds);
     }
 }
 
@@ -470,6 +616,35 @@ inline int sor_resident_dispatch(const SorArgs<T>& a, const SorResident& r, Tile
     CNV_RESIDENT_SHAPES(CNV_RESIDENT_CASE)
 #undef CNV_RESIDENT_CASE
     return 2;
+}
+
+// The shapes of batched resident solves and the time of one sweep (us, a full GPU).  FP32 tiles of
+// 128 x 128 points (8 rows a wave) fit the registers where dx = dy, FP64 ones do not.
+struct ResidentBatchShape {
+    TileShape shape;
+    double us;
+};
+template <typename T>
+inline const std::vector<ResidentBatchShape>& resident_batch_shapes() {
+    static const std::vector<ResidentBatchShape> f64 = {{{5, 16, 2}, 1.10}, {{5, 16, 4}, 1.56}};
+    static const std::vector<ResidentBatchShape> f32 = {{{5, 16, 2}, 0.75}, {{5, 16, 4}, 1.08}, {{5, 16, 8}, 1.20}};
+    return sizeof(T) == 8 ? f64 : f32;
+}
+
+template <typename T, int RB>
+inline void sor_resident_batch_launch_rb(const SorArgs<T>* args, const SorResident* res, const ResidentQueues& q,
+                                         int blocks, bool gs, hipStream_t st) {
+    const dim3 grid(blocks), block(16 * 64);
+    if (gs) hipLaunchKernelGGL((sor_resident_batch_kernel<T, 5, 16, RB, true>), grid, block, 0, st, args, res, q);
+    else hipLaunchKernelGGL((sor_resident_batch_kernel<T, 5, 16, RB, false>), grid, block, 0, st, args, res, q);
+}
+template <typename T>
+inline int sor_resident_batch_launch(const SorArgs<T>* args, const SorResident* res, const ResidentQueues& q,
+                                     TileShape sh, int blocks, bool gs, hipStream_t st) {
+    if (sh.rb == 2) sor_resident_batch_launch_rb<T, 2>(args, res, q, blocks, gs, st);
+    else if (sh.rb == 4) sor_resident_batch_launch_rb<T, 4>(args, res, q, blocks, gs, st);
+    else if constexpr (sizeof(T) == 4) sor_resident_batch_launch_rb<T, 8>(args, res, q, blocks, gs, st);
+    return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
 }  // namespace cnv
