@@ -135,7 +135,6 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     const bool inside = t.gj >= 0 && t.gj < t.nc;
     const bool owncol = t.ownc[0];
     const bool ringcol = owncol && (2 * t.lane < 2 * H || 2 * t.lane >= TJ);
-    const int voff = t.gj * (int)sizeof(T);
     const int pitch = r.ldx * (int)sizeof(T);
     const int plane = (int)(r.xplane * (long long)sizeof(T));
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(r.exch, 0, 3 * plane, 0x00027000);
@@ -153,12 +152,79 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     };
     const int lo = row_lo > 0 ? row_lo * TI + H : 0;  // rows another band reads: below lo or from hi on
     const int hi = row_hi < a.tiles_i ? row_hi * TI - H : t.nr;
+    // Columns.  A wave whose rows are all owned takes only S pairs at each end of a row, and gives only
+    // the S next to them unless its rows are read from above or below: 10 of 64 lanes.  A memory
+    // instruction costs its 16 cycles whatever its lanes do, so such a wave handles kRows rows with
+    // one: lane m takes pair m % kPairs of row m / kPairs, and the values change lanes through the
+    // wave's part of the half-sweeps' exchange rows (xch[1], which nobody reads between the last
+    // half-sweep and the next epoch's first barrier).  1024^2: FP32 0.97 -> 0.91 us per sweep, FP64
+    // 1.46 -> 1.45; with two rows a wave the detour costs more than the one instruction saved (3% at
+    // 64^2), and so it does on 12 waves in FP64 (2% at 600^2).
+    constexpr int kPairs = 2 * S;
+    constexpr int kRows = RB * kPairs <= 64 ? RB : RB / 2;
+    static_assert(kRows * kPairs <= 64 && RB % kRows == 0, "a chunk of rows is one pair a lane");
+    typedef T Pair2 __attribute__((ext_vector_type(2)));
+    Pair2* const stage = reinterpret_cast<Pair2*>(sh.xch[1][t.wv][0]);  // 64 pairs
+    struct Column {  // this lane's pair of a chunk: there is one, and its offset
+        bool has;
+        int voff;
+    };
+    // (offsets are worked out when they are used: held through the sweeps they cost registers those need)
+    auto lane_now = [&]() -> int {
+        int m = threadIdx.x & 63;
+        asm volatile("" : "+v"(m));
+        return m;
+    };
+    auto row_offset = [&]() -> int { return (t.gj0 + 2 * lane_now()) * (int)sizeof(T); };
+    auto column = [&](bool taken) -> Column {
+        const int m = lane_now();
+        const int mr = m / kPairs, mj = m - mr * kPairs;
+        const int at = taken ? (mj < S ? mj : 64 - kPairs + mj) : (mj < S ? S + mj : 64 - 3 * S + mj);
+        const int gj = t.gj0 + 2 * at;
+        return Column{mr < kRows && gj >= 0 && gj < t.nc, mr * pitch + gj * (int)sizeof(T)};
+    };
+    constexpr bool kColumns = RB >= 4 && (sizeof(T) == 4 || NW >= 16);
+    bool all_own = kColumns, no_ring = kColumns;  // wave-uniform
+#pragma unroll
+    for (int rr = 0; rr < RB; ++rr) {
+        const int li = t.row0 + rr;
+        all_own = all_own && own_row(rr);
+        no_ring = no_ring && own_row(rr) && li >= 2 * H && li < TI;
+    }
     auto give = [&](int slot, bool marks) {
+        T mk = Marked<T>::mark();
+        asm volatile("" : "+v"(mk));
+        if (no_ring) {
+            const bool through = t.gi0 + t.row0 < lo || t.gi0 + t.row0 + RB > hi;
+            const Column col = column(false);
+#pragma unroll
+            for (int c = 0; c < RB; c += kRows) {
+                Pair2 d = {mk, mk};
+                if (!marks) {
+                    // lanes S .. 2S-1 hold the left pairs, 64-2S .. 64-S-1 the right ones
+                    const int m = lane_now();
+                    const bool at_left = m < 2 * S;
+                    const int j = at_left ? m - S : m - 64 + 3 * S;
+                    if (j >= (at_left ? 0 : S) && j < kPairs) {
+#pragma unroll
+                        for (int rr = 0; rr < kRows; ++rr) stage[rr * kPairs + j] = Pair2{t.v[0][c + rr], t.v[1][c + rr]};
+                    }
+                    d = stage[lane_now()];
+                }
+                const int soff = slot * plane + (t.gi0 + t.row0 + c) * pitch;
+                if (col.has) {
+                    if (through) exch_store<T, kAgent>(rs, col.voff, soff, d.x, d.y);
+                    else exch_store<T, 0>(rs, col.voff, soff, d.x, d.y);
+                }
+            }
+            return;
+        }
+        const int voff = row_offset();
 #pragma unroll
         for (int rr = 0; rr < RB; ++rr) {
             const int gi = t.gi0 + t.row0 + rr;
             if (!gives(rr)) continue;
-            const T x0 = marks ? Marked<T>::mark() : t.v[0][rr], x1 = marks ? Marked<T>::mark() : t.v[1][rr];
+            const T x0 = marks ? mk : t.v[0][rr], x1 = marks ? mk : t.v[1][rr];
             if (gi < lo || gi >= hi) exch_store<T, kAgent>(rs, voff, slot * plane + gi * pitch, x0, x1);
             else exch_store<T, 0>(rs, voff, slot * plane + gi * pitch, x0, x1);
         }
@@ -169,10 +235,24 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     // the halo cells of plane `slot` (slot < 0: none) and a decision on `decided` epochs (0: none)
     auto take = [&](int slot, int decided) -> u64 {
         u64 word = 0;
+        struct {
+            T x, y;
+        } got[RB / kRows];
+        const Column col = column(true);
+        const int voff = row_offset();
         for (int spins = 0;; ++spins) {
             bool ok = true;
             if (decided) word = agent_load(dec);
-            if (slot >= 0) {
+            if (slot >= 0 && all_own) {
+                if (col.has) {
+#pragma unroll
+                    for (int c = 0; c < RB / kRows; ++c)
+                        exch_load<T>(rs, col.voff, slot * plane + (t.gi0 + t.row0 + c * kRows) * pitch, got[c].x, got[c].y);
+#pragma unroll
+                    for (int c = 0; c < RB / kRows; ++c)
+                        ok = ok && Marked<T>::ready(got[c].x) && Marked<T>::ready(got[c].y);
+                }
+            } else if (slot >= 0) {
 #pragma unroll
                 for (int rr = 0; rr < RB; ++rr)
                     if (takes(rr)) exch_load<T>(rs, voff, slot * plane + (t.gi0 + t.row0 + rr) * pitch, t.v[0][rr], t.v[1][rr]);
@@ -187,6 +267,22 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
                 report_abort(r);
             }
         }
+        if (slot >= 0 && all_own) {
+            const int m = lane_now();
+            const int j = m < S ? m : m - 64 + kPairs;
+#pragma unroll
+            for (int c = 0; c < RB / kRows; ++c) {
+                stage[m] = Pair2{got[c].x, got[c].y};
+                if (inside && !owncol && j >= 0) {
+#pragma unroll
+                    for (int rr = 0; rr < kRows; ++rr) {
+                        const Pair2 d = stage[rr * kPairs + j];
+                        t.v[0][c * kRows + rr] = d.x;
+                        t.v[1][c * kRows + rr] = d.y;
+                    }
+                }
+            }
+        }
         const unsigned hi32 = __builtin_amdgcn_readfirstlane((unsigned)(word >> 32));
         const unsigned lo32 = __builtin_amdgcn_readfirstlane((unsigned)word);
         return ((u64)hi32 << 32) | lo32;
@@ -195,7 +291,9 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     // the values at an epoch's start, in two turns (FP64)
     Two* const mem = kSnapLds ? nullptr : reinterpret_cast<Two*>(r.snap) + (size_t)snap_part * 2 * RB * NW * 64;
     auto snap_at = [&](int turn, int rr) -> Two* {
-        const int q = (turn * RB + rr) * NW * 64 + (int)threadIdx.x;
+        int m = threadIdx.x;
+        asm volatile("" : "+v"(m));
+        const int q = (turn * RB + rr) * NW * 64 + m;
         return kSnapLds ? snap_lds + q : mem + q;
     };
     auto keep = [&](int turn) {
@@ -627,7 +725,7 @@ struct ResidentBatchShape {
 template <typename T>
 inline const std::vector<ResidentBatchShape>& resident_batch_shapes() {
     static const std::vector<ResidentBatchShape> f64 = {{{5, 16, 2}, 1.10}, {{5, 16, 4}, 1.56}};
-    static const std::vector<ResidentBatchShape> f32 = {{{5, 16, 2}, 0.75}, {{5, 16, 4}, 1.08}, {{5, 16, 8}, 1.20}};
+    static const std::vector<ResidentBatchShape> f32 = {{{5, 16, 2}, 0.76}, {{5, 16, 4}, 1.08}, {{5, 16, 8}, 1.70}};
     return sizeof(T) == 8 ? f64 : f32;
 }
 
