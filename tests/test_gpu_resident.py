@@ -108,3 +108,75 @@ def test_two_solves_at_once():
         for rc, psi, k, e in got[t]:
             assert (rc, k) == (alone[0], alone[2]) and abs(e - alone[3]) <= 1e-12 * e
             assert np.array_equal(psi, alone[1])
+
+
+def batch_equals_alone(ps, steps, states=None):
+    """Each cavity of a batch as it is alone: fields and counts bit for bit, the FP64 update (summed
+    per tile) to rounding; the FP32 solves add theirs in FP32 over a lane's rows, whose number differs."""
+    states = states or [None] * len(ps)
+    with cnv.Batch(ps) as b:
+        for i, s in enumerate(states):
+            if s:
+                b.set_state(i, **s)
+        st = b.step(steps)
+        got = [b.get_state(i) for i in range(len(ps))]
+    for i, p in enumerate(ps):
+        if p.precision == cnv.PREC_FP32_DC:  # its solves test every fifth sweep, as the batch's do
+            p.sweeps_per_launch, p.tile_waves, p.wave_rows = 5, 16, 4
+        with cnv.Cavity(p) as cav:
+            if states[i]:
+                cav.set_state(**states[i])
+            alone, state = cav.step(steps), cav.get_state()
+        for t in range(steps):
+            a, g = alone[t], st[t][i]
+            assert (g.status, g.k, g.sweeps, g.outer) == (a.status, a.k, a.sweeps, a.outer), (i, t)
+            assert p.precision != cnv.PREC_FP64 or abs(g.e - a.e) <= 1e-12 * abs(a.e)
+        for name in ("w", "psi", "u", "v"):
+            assert np.array_equal(got[i][name], state[name]), (i, name)
+    return [s for row in st for s in row]
+
+
+# few cavities (2 rows a wave), many (4; in FP32 8 where dx = dy), one that takes most of the GPU
+@pytest.mark.parametrize("sides", [[8, 9, 97], [64, 104, 105, 33] * 4, [256, 255, 240, 100] * 8, [900, 40, 300, 41]],
+                         ids=["few", "some", "many", "large"])
+@pytest.mark.parametrize("precision", [cnv.PREC_FP64, cnv.PREC_FP32_DC], ids=["fp64", "refined"])
+@pytest.mark.parametrize("kind", ["square", "oblong", "gs"])
+def test_batch_equals_alone(sides, precision, kind):
+    ps = []
+    for i, n in enumerate(sides):
+        p = cnv.default_params(n, Re=100.0 + 50 * i, dt=1e-4 if n < 500 else 1e-5, tol=1e-6, itmax=200000,
+                               precision=precision, inner_test_every=1, poisson_type=1 if kind == "gs" else 2,
+                               beta=cnv.reference_beta(n), u=[0.0, 0.0, 0.0, 1.0 + 0.01 * i])
+        if kind == "oblong":
+            p.dy = 0.8 * p.dx
+        if kind == "gs":
+            p.itmax, p.tol = 400, 1e-3  # plain Gauss-Seidel sweeps; the larger sides run out of them
+        ps.append(p)
+    if kind == "gs":
+        ps = [p for p in ps if p.n <= 105] or ps[:2]
+    if kind == "gs" and precision == cnv.PREC_FP32_DC:
+        for p in ps:
+            p.itmax = 200000
+    print(sides, precision, kind, flush=True)
+    assert all(s.status == cnv.OK for s in batch_equals_alone(ps, 2)) or kind == "gs"
+
+
+@pytest.mark.parametrize("precision", [cnv.PREC_FP64, cnv.PREC_FP32_DC], ids=["fp64", "refined"])
+def test_batch_solves_longer_than_a_kernel(precision):
+    # beta = 1: 10^4 and more sweeps, which is more epochs than one resident kernel runs
+    ps = [cnv.default_params(n, Re=100.0, dt=1e-4, tol=1e-9, itmax=200000, precision=precision, inner_test_every=1,
+                             beta=1.0) for n in (33, 160, 64, 161)]
+    st = batch_equals_alone(ps, 1)
+    assert max(s.sweeps for s in st) > 1984 * 5
+
+
+def test_batch_solves_that_end_from_far_out():
+    # as test_solve_that_ends_from_far_out, each cavity of a batch ending at another sweep
+    n, ends = 256, (4, 13, 15, 16, 17, 18, 20, 21) * 4
+    i, j = np.indices((n, n))
+    f = np.sin(2 * np.pi * i / 5) * np.sin(2 * np.pi * j / 5)
+    e = {s: orc.poisson(orc.make_params(n, tol=-1.0, itmax=s, ordering=orc.REDBLACK, beta_=0.6, threads=8), f)[1].e
+         for s in ends}
+    ps = [cnv.default_params(n, Re=1e6, dt=1e-12, tol=e[s] * (1 + 1e-6), itmax=1000, beta=0.6) for s in ends]
+    st = batch_equals_alone(ps, 1, [dict(w=f, psi=np.zeros((n, n))) for _ in ends])
+    assert {s.k for s in st} == {s - 1 for s in ends}
