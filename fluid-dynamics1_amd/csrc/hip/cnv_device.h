@@ -132,6 +132,7 @@ struct SorResident {
     int* abort;                // set by a wave that gave up waiting
     int ldx, ntiles;
     int blocks;                // workgroups of a launch
+    int runs;                  // an XCD's tiles are an eighth of all, row after row (0: a band of whole tile rows)
     int epochs, launch0;       // epochs at most; index of the first one within the solve
     int stop;                  // > 0: run to exactly this many sweeps of the solve, without tests
     int spins;                 // polls of one wait before it is given up

@@ -40,21 +40,41 @@ std::atomic<int> g_units[kMaxDevices];  // CUs per XCD in use by resident solves
 //   6,16,4  1.202  1.372  1.388  1.405  1.445  1.471  -
 //   5,16,4  1.272  1.479  1.475  1.493  1.486  1.526  1.459
 // so thin tiles first: an epoch's sweeps cost as much as the rows of its tile.  As launches of
-// sor_rb.h the default shapes took 1.27 us at 64^2, 1.34 at 257^2 and 2.0 at 1024^2.
-constexpr TileShape kShapes[] = {{6, 16, 2}, {5, 16, 2}, {4, 16, 2}, {6, 12, 4}, {6, 16, 4}, {5, 16, 4}};
+// sor_rb.h the default shapes took 1.27 us at 64^2, 1.34 at 257^2 and 2.0 at 1024^2.  Larger grids
+// (us per FP64 sweep; "launches" the (5, 16, 4) ones, all that these grids had before; an FP32
+// sweep at 1100^2 1.22 against 1.65, at 1600^2 1.77 against 2.55):
+//   n        1100  1400  1600  1900  2048
+//   5,12,8   2.35  2.38  -
+//   5,12,10  3.04  3.07  3.05  -
+//   3,12,14  5.12  5.16  5.14  5.16  4.90
+//   launches 4.09  4.09  6.56  7.62  8.74
+// Their tiles fill the register files; 12 waves of up to 168 registers a lane run them 20-25% faster
+// than 8 waves of 256, which leave a SIMD two waves to hide an FP64 operation behind.  Beyond 2072^2
+// or so (14 x 18 tiles of 156 x 116 points) the grid does not fit in the registers.
+constexpr TileShape kShapes[] = {{6, 16, 2}, {5, 16, 2}, {4, 16, 2}, {6, 12, 4}, {6, 16, 4}, {5, 16, 4},
+                                 {5, 12, 8}, {5, 12, 10}, {3, 12, 14}};
 
 // Workgroups per XCD of a resident solve with tiles of shape sh (0: they do not fit together).
 int resident_slots(int n, TileShape sh, int per_xcd, SorResident* r) {
     const int ti = (n + tile_rows(sh) - 1) / tile_rows(sh), tj = (n + tile_cols(sh) - 1) / tile_cols(sh);
-    // every XCD gets as many workgroups as the largest band has tiles, or one of them one more: a
-    // workgroup without a tile decides
-    int most = 0;
-    for (int b = 0; b < kBands; ++b) most = std::max(most, (band_start(b + 1, ti) - band_start(b, ti)) * tj);
+    // a workgroup of 16 waves (or of 8 with twice the registers each) fills a CU; two of 4 waves fit
+    const int room = sh.nw > 4 ? per_xcd : 2 * per_xcd;
     r->ntiles = ti * tj;
-    r->blocks = kBands * most + (r->ntiles == kBands * most);
-    const int slots = (r->blocks + kBands - 1) / kBands;
-    // a workgroup of 16 waves (or of 8 with two tile copies in LDS) fills a CU; two of 4 waves fit
-    return slots <= (sh.nw > 4 ? per_xcd : 2 * per_xcd) ? slots : 0;
+    // An XCD's tiles are whole tile rows where they fit so; else an eighth of all tiles, whose cells are
+    // written through more often: up to 2 more neighbours' tiles are on other XCDs.
+    for (r->runs = 0; r->runs < 2; ++r->runs) {
+        if (r->runs && (tile_rows(sh) < 2 * sh.s || tile_cols(sh) < 2 * sh.s)) break;  // halos of one tile only
+        // every XCD gets as many workgroups as the largest share has tiles, or one of them one more:
+        // a workgroup without a tile decides
+        int most = 0;
+        for (int b = 0; b < kBands; ++b)
+            most = std::max(most, r->runs ? band_start(b + 1, r->ntiles) - band_start(b, r->ntiles)
+                                          : (band_start(b + 1, ti) - band_start(b, ti)) * tj);
+        r->blocks = kBands * most + (r->ntiles == kBands * most);
+        const int slots = (r->blocks + kBands - 1) / kBands;
+        if (slots <= room) return slots;
+    }
+    return 0;
 }
 
 int cus_per_xcd(int dev) {

@@ -176,9 +176,10 @@ __device__ inline T* sor_plane(const SorArgs<T>& a, int idx) {
 }
 
 // A tile's LDS: the waves' first and last rows, and one column per thread of per-lane sums.
-template <typename T, int NW, int SE, bool kNorm>
+template <typename T, int NW, int SE, bool kNorm, int FL = 0>
 struct SorShared {
     T xch[2][NW][2][64];  // [half-sweep parity][wave][first/last row][lane]
+    T fcl[FL > 0 ? FL * 2 * NW * 64 : 1];  // the source term of the rows that registers do not hold
     double lred[SE][NW * 64];  // this launch's per-lane L1 update sums, one row per summed sweep
     double lnrm[kNorm ? NW * 64 : 1];  // the per-lane iterate norm after the last sweep
 };
@@ -208,14 +209,23 @@ struct SorTile {
     typedef typename std::conditional<sizeof(T) == 4, float, double>::type Acc;
     typedef typename PairOf<T>::type Pair;
 
-    typedef SorShared<T, NW, SE, kNorm> Shared;
+    // Thick FP64 tiles (resident solves of large grids) have no registers for a relaxation factor per
+    // point: the rows' share of it, and of the norms' weights, is a bit mask, from which every row's
+    // factor comes as a scalar; the columns' share, 0 on the domain boundary, is in the lane's
+    // reciprocal.  The thickest keep the source term of only RF rows of a wave, the others' in LDS.
+    static constexpr bool kMasks = sizeof(T) == 8 && NW * RB >= 96;
+    static constexpr int RF = kMasks && RB > 10 ? 5 : RB;
+
+    typedef SorShared<T, NW, SE, kNorm, RB - RF> Shared;
 
     T v[2][RB];   // v[q][r]: value at (row0 + r, 2*lane + q)
-    T fc[2][RB];  // FP64: c3*f (the hoisted c3*f product of the update); FP32: -be*c3*f
-    T be[2][RB];  // FP64: bcoef at interior points, 0 on the domain boundary and outside it
+    T fc[2][RF];  // FP64: c3*f (the hoisted c3*f product of the update); FP32: -be*c3*f
+    T be[2][kMasks ? 1 : RB];  // FP64: bcoef at interior points, 0 on the domain boundary and outside it
     T cn[2][RB];  // FP32: be*c1 and be*c2, the relaxation folded into the stencil coefficients
     T ce[2][ISO ? 1 : RB];
-    Acc w[RB];    // 1 for owned rows inside the domain, else 0 (wave-uniform)
+    Acc w[kMasks ? 1 : RB];  // 1 for owned rows inside the domain, else 0 (wave-uniform)
+    unsigned inner, owned;   // kMasks: bit r for an interior, an owned row r
+    T bcoef, rBc[2];         // kMasks: the relaxation factor; rB, 0 on the domain boundary's columns
     T c1, c2, B, rB, omb;
     int gi0, gj0, gj, lane, wv, row0, nr, nc;
     unsigned bld;
@@ -249,18 +259,19 @@ struct SorTile {
     }
 
     // the tile's values from plane src, its source term and its coefficients
-    __device__ __forceinline__ void load(const SorArgs<T>& a, const T* __restrict__ src) {
+    __device__ __forceinline__ void load(const SorArgs<T>& a, const T* __restrict__ src, Shared& sh) {
 #pragma clang fp contract(off)
         // relaxation factor of an updated point: FP64 beta (1 for Gauss-Seidel), applied before the
         // division; FP32 beta/B (1/B), which folds the division in.  Per column, 0 off the interior
         // columns; per point, also 0 on the boundary rows and outside the domain.
-        T bcoef;
         if constexpr (sizeof(T) == 8) bcoef = GS ? T(1) : a.beta;
         else bcoef = GS ? a.rB : a.beta * a.rB;
         const T c3s = a.negate ? -a.c3 : a.c3;  // f = -src folded in: c3*(-x) == (-c3)*x exactly
         T bcol[2], cncol[2], cecol[2];
+        inner = owned = 0;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
+            rBc[q] = colin[q] ? a.rB : T(0);
             bcol[q] = colin[q] ? bcoef : T(0);
             cncol[q] = colin[q] ? bcoef * a.c1 : T(0);
             cecol[q] = colin[q] ? bcoef * a.c2 : T(0);
@@ -270,7 +281,13 @@ struct SorTile {
             const int li = row0 + r;
             const int gi = gi0 + li;
             const bool rint = gi >= 1 && gi <= nr - 2;
-            w[r] = (li >= H && li < H + TI && gi < nr) ? Acc(1) : Acc(0);
+            const bool own = li >= H && li < H + TI && gi < nr;
+            if constexpr (kMasks) {
+                inner |= (unsigned)rint << r;
+                owned |= (unsigned)own << r;
+            } else {
+                w[r] = own ? Acc(1) : Acc(0);
+            }
             const Pair d = load_pair(row_of(a, src, gi), bld);
             const Pair f = load_pair(row_of(a, a.src_f, gi), bld);
             v[0][r] = d.x;
@@ -281,10 +298,12 @@ struct SorTile {
                 const bool inter = rint && colin[q];
                 const T fq = q ? f.y : f.x;
                 if constexpr (sizeof(T) == 8) {
-                    fc[q][r] = inter ? c3s * fq : T(0);
-                    be[q][r] = rint ? bcol[q] : T(0);
+                    const T fr = inter ? c3s * fq : T(0);
+                    if (r < RF) fc[q][r < RF ? r : 0] = fr;
+                    else sh.fcl[(r < RF ? 0 : (r - RF) * 2 + q) * NW * 64 + threadIdx.x] = fr;
+                    if constexpr (!kMasks) be[q][r] = rint ? bcol[q] : T(0);
                 } else {
-                    fc[q][r] = inter ? bcoef * -(c3s * fq) : T(0);
+                    fc[q][r < RF ? r : 0] = inter ? bcoef * -(c3s * fq) : T(0);
                     cn[q][r] = rint ? cncol[q] : T(0);
                     if constexpr (!ISO) ce[q][r] = rint ? cecol[q] : T(0);
                 }
@@ -313,9 +332,11 @@ struct SorTile {
         }
     }
     __device__ __forceinline__ bool owns_rows() const {  // wave-uniform: the wave holds an owned row
-        bool owns = false;
+        bool owns = kMasks && owned != 0;
+        if constexpr (!kMasks) {
 #pragma unroll
-        for (int r = 0; r < RB; ++r) owns = owns || w[r] != Acc(0);
+            for (int r = 0; r < RB; ++r) owns = owns || w[r] != Acc(0);
+        }
         return owns;
     }
 
@@ -337,6 +358,12 @@ struct SorTile {
         Acc acc[2] = {Acc(0), Acc(0)}, nrm[2] = {Acc(0), Acc(0)};
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
+            // LDS offsets reach 64 KB: the source terms beyond have a base of their own
+            constexpr int kNear = 65536 / (NW * 64 * (int)sizeof(T)) - 1;
+            unsigned at0 = tid, at1 = tid + kNear * NW * 64;
+            if constexpr (RF < RB) asm volatile("" : "+v"(at0), "+v"(at1));
+            unsigned in_now = kMasks ? inner : 0, own_now = kMasks ? owned : 0;
+            if constexpr (kMasks) asm volatile("" : "+s"(in_now), "+s"(own_now));  // the rows' scalars are not kept
             // boundary rows of the neighbouring waves (colour 1-c, written by half-sweep h-1)
             const T sb = sh.xch[c ^ 1][wv > 0 ? wv - 1 : 0][1][lane];
             const T nb = sh.xch[c ^ 1][wv < NW - 1 ? wv + 1 : NW - 1][0][lane];
@@ -355,18 +382,26 @@ struct SorTile {
                 if constexpr (sizeof(T) == 8) {
                     // the reference's association: ((c1*(N+S) + c2*(E+W)) - c3*f), times beta,
                     // divided by B, plus (1-beta)*u0; + is commutative, so E/W order is free
-                    const T x = c1 * (up + dn) + c2 * (own + far) - fc[q][r];
-                    const T y = be[q][r] * x;
-                    const T qt = XR ? y * rB : sor_div(y, B, rB);
+                    const int j2 = r < RF ? 0 : (r - RF) * 2 + q;  // compile-time
+                    const bool far_f = j2 >= kNear;
+                    const T x = c1 * (up + dn) + c2 * (own + far) - (r < RF ? fc[q][r < RF ? r : 0] : sh.fcl[far_f ? at1 + (j2 - kNear) * NW * 64 : at0 + j2 * NW * 64]);
+                    const T y = (kMasks ? (in_now >> r & 1 ? bcoef : T(0)) : be[q][kMasks ? 0 : r]) * x;
+                    const T rq = kMasks ? rBc[q] : rB;
+                    const T qt = XR ? y * rq : sor_div(y, B, rq);
                     cand = GS ? qt : qt + omb * old;
-                    v[q][r] = cand;
+                    if constexpr (!kMasks) v[q][r] = cand;
                     if constexpr (kL1) {
-                        acc[q] = __fma_rn(w[r], fabs(cand - old), acc[q]);
-                        if (kNorm && with_norm) nrm[q] = __fma_rn(w[r], fabs(cand), nrm[q]);
+                        const T wr = kMasks ? (own_now >> r & 1 ? T(1) : T(0)) : w[kMasks ? 0 : r];
+                        acc[q] = __fma_rn(wr, fabs(cand - old), acc[q]);
+                        if (kNorm && with_norm) nrm[q] = __fma_rn(wr, fabs(cand), nrm[q]);
                     }
+                    // into the old value's register, once the sum is done with that: the compiler
+                    // otherwise holds every row twice and moves all of them at the end of a sweep
+                    // (no lane exchange of this value follows before the next barrier)
+                    if constexpr (kMasks) asm volatile("v_mov_b64 %0, %2" : "+v"(v[q][r]), "+v"(acc[q]) : "v"(cand));
                 } else {
                     // relaxation and 1/B folded into cn, ce and fc (0 where the point is fixed)
-                    const T x = __fmaf_rn(cn[q][r], up + dn, __fmaf_rn(ISO ? cn[q][r] : ce[q][ISO ? 0 : r], own + far, fc[q][r]));
+                    const T x = __fmaf_rn(cn[q][r], up + dn, __fmaf_rn(ISO ? cn[q][r] : ce[q][ISO ? 0 : r], own + far, fc[q][r < RF ? r : 0]));
                     cand = GS ? x : __fmaf_rn(omb, old, x);
                     v[q][r] = cand;
                     if (kL1 && with_norm) {
@@ -420,6 +455,12 @@ struct SorTile {
     }
     // the owned tile to plane dst; domain-boundary points hold +-0: store +0
     __device__ __forceinline__ void store(const SorArgs<T>& a, T* __restrict__ dst) const {
+        int gj = this->gj;
+        if constexpr (kMasks) {  // not kept from the loads on
+            int m = threadIdx.x & 63;
+            asm volatile("" : "+v"(m));
+            gj = gj0 + 2 * m;
+        }
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
             const int li = row0 + r;
@@ -474,7 +515,7 @@ __device__ __forceinline__ void sor_rb_sweeper(const SorArgs<T>& a, const int L,
     t.place(a, ti, tj);
     // Speculative tile load for the common case (sweep on from the previous launch's output),
     // issued before the state slot is read so that both are in flight together.
-    t.load(a, sor_plane(a, L % NB));
+    t.load(a, sor_plane(a, L % NB), sh);
 
     // what this launch does: the state after launch L-2 and the sweeps launch L-1 performed
     const int pstatus = prev->status;

@@ -17,7 +17,8 @@
 // L2 holds for it and what other XCDs have written through.  Tile rows are dealt to the XCDs in
 // contiguous bands, and each workgroup takes the next free tile of the band of the XCD it finds
 // itself on (workgroups are dealt to the XCDs round-robin, so every band gets as many as it has
-// tiles; if one did not, its neighbours' waits would run out), so most cells are read on the XCD that
+// tiles; if one did not, its neighbours' waits would run out; where whole tile rows leave too many
+// CUs empty, an eighth of all tiles takes the place of a band), so most cells are read on the XCD that
 // wrote them: these are stored plainly, into that L2; only the rows another band reads are
 // written through (agent-scope stores).  Writing every cell through measured 5.9 us per exchange
 // at 1024^2 with (5, 16, 4) tiles, this split 3.0; polling flags instead of the data 10.8.
@@ -107,11 +108,26 @@ typedef double SnapPair __attribute__((ext_vector_type(2)));
 template <typename T, int NW, int RB>
 constexpr int kSnapPairs = sizeof(T) == 8 && resident_snap_lds(NW, RB) ? 2 * RB * NW * 64 : 1;
 
-// One tile's workgroup: tile (ti, tj), in the band of tile rows [row_lo, row_hi) that one XCD holds;
+// the largest share of rb rows that has at most `most`
+constexpr int chunk_rows(int rb, int most) {
+    int rows = rb < most ? rb : most;
+    while (rb % rows) --rows;
+    return rows;
+}
+
+// The rows of a band [row_lo, row_hi) of tile rows that other bands read: below lo or from hi on.
+template <typename Tile, typename T>
+__device__ __forceinline__ int band_lo(const SorArgs<T>& a, int row_lo) { return row_lo > 0 ? row_lo * Tile::TI + Tile::H : 0; }
+template <typename Tile, typename T>
+__device__ __forceinline__ int band_hi(const SorArgs<T>& a, int row_hi) {
+    return row_hi < a.tiles_i ? row_hi * Tile::TI - Tile::H : a.nr;
+}
+
+// One tile's workgroup: tile (ti, tj); grid rows below lo or from hi on are read on other XCDs;
 // snap_part: which part of r.snap is its own.
 template <typename T, int S, int NW, int RB, bool GS, bool XR, bool NORM, bool ISO = false>
 __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const SorResident& r, const int ti, const int tj,
-                                                  const int row_lo, const int row_hi, const int snap_part,
+                                                  const int lo, const int hi, const int snap_part,
                                                   typename SorTile<T, S, NW, RB, GS, XR, NORM>::Shared& sh,
                                                   SnapPair* const snap_lds) {
     typedef SorTile<T, S, NW, RB, GS, XR, NORM, ISO> Tile;
@@ -119,6 +135,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     constexpr bool kSnap = sizeof(T) == 8;
     constexpr bool kSnapLds = kSnap && resident_snap_lds(NW, RB);
     typedef SnapPair Two;
+    constexpr bool kThick = NW * RB >= 96 && H <= RB;
 
     const int tile = ti * a.tiles_j + tj;
     const SorCtl* P = a.ctl + r.rslot;
@@ -127,7 +144,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     int k = P->k;
     Tile t;
     t.place(a, ti, tj);
-    t.load(a, sor_plane(a, r.src));
+    t.load(a, sor_plane(a, r.src), sh);
     t.fix_odd_edge();
     const bool owns = t.owns_rows();
 
@@ -138,20 +155,27 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     const int pitch = r.ldx * (int)sizeof(T);
     const int plane = (int)(r.xplane * (long long)sizeof(T));
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(r.exch, 0, 3 * plane, 0x00027000);
-    auto own_row = [&](int rr) {
-        const int li = t.row0 + rr;
+    // The rows' masks and addresses are held through the sweeps (worked out anew at every exchange they
+    // cost 10% of a sweep at 64^2); where the source term is in LDS their registers are needed, and those of
+    // what a tile gives and what it does with what it took are worked out when it does.
+    auto row_now = [&]() -> int {
+        if constexpr (Tile::RF == RB) return t.row0;
+        int row0 = __builtin_amdgcn_readfirstlane(t.row0);
+        asm volatile("" : "+s"(row0));
+        return row0;
+    };
+    auto own_row = [&](int row0, int rr) {
+        const int li = row0 + rr;
         return li >= H && li < H + TI && t.gi0 + li < t.nr;
     };
-    auto takes = [&](int rr) {
-        const int gi = t.gi0 + t.row0 + rr;
-        return gi >= 0 && gi < t.nr && inside && !(own_row(rr) && owncol);
+    auto takes = [&](int row0, int rr) {
+        const int gi = t.gi0 + row0 + rr;
+        return gi >= 0 && gi < t.nr && inside && !(own_row(row0, rr) && owncol);
     };
-    auto gives = [&](int rr) {
-        const int li = t.row0 + rr;
-        return own_row(rr) && (li < 2 * H || li >= TI ? owncol : ringcol);
+    auto gives = [&](int row0, int rr) {
+        const int li = row0 + rr;
+        return own_row(row0, rr) && (li < 2 * H || li >= TI ? owncol : ringcol);
     };
-    const int lo = row_lo > 0 ? row_lo * TI + H : 0;  // rows another band reads: below lo or from hi on
-    const int hi = row_hi < a.tiles_i ? row_hi * TI - H : t.nr;
     // Columns.  A wave whose rows are all owned takes only S pairs at each end of a row, and gives only
     // the S next to them unless its rows are read from above or below: 10 of 64 lanes.  A memory
     // instruction costs its 16 cycles whatever its lanes do, so such a wave handles kRows rows with
@@ -161,7 +185,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     // 1.46 -> 1.45; with two rows a wave the detour costs more than the one instruction saved (3% at
     // 64^2), and so it does on 12 waves in FP64 (2% at 600^2).
     constexpr int kPairs = 2 * S;
-    constexpr int kRows = RB * kPairs <= 64 ? RB : RB / 2;
+    constexpr int kRows = chunk_rows(RB, 64 / kPairs);
     static_assert(kRows * kPairs <= 64 && RB % kRows == 0, "a chunk of rows is one pair a lane");
     typedef T Pair2 __attribute__((ext_vector_type(2)));
     Pair2* const stage = reinterpret_cast<Pair2*>(sh.xch[1][t.wv][0]);  // 64 pairs
@@ -172,7 +196,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     // (offsets are worked out when they are used: held through the sweeps they cost registers those need)
     auto lane_now = [&]() -> int {
         int m = threadIdx.x & 63;
-        asm volatile("" : "+v"(m));
+        if constexpr (RB > 2) asm volatile("" : "+v"(m));
         return m;
     };
     auto row_offset = [&]() -> int { return (t.gj0 + 2 * lane_now()) * (int)sizeof(T); };
@@ -183,19 +207,20 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
         const int gj = t.gj0 + 2 * at;
         return Column{mr < kRows && gj >= 0 && gj < t.nc, mr * pitch + gj * (int)sizeof(T)};
     };
-    constexpr bool kColumns = RB >= 4 && (sizeof(T) == 4 || NW >= 16);
+    constexpr bool kColumns = RB >= 4 && (sizeof(T) == 4 || NW != 12 || RB > 4);
     bool all_own = kColumns, no_ring = kColumns;  // wave-uniform
 #pragma unroll
     for (int rr = 0; rr < RB; ++rr) {
         const int li = t.row0 + rr;
-        all_own = all_own && own_row(rr);
-        no_ring = no_ring && own_row(rr) && li >= 2 * H && li < TI;
+        all_own = all_own && own_row(t.row0, rr);
+        no_ring = no_ring && own_row(t.row0, rr) && li >= 2 * H && li < TI;
     }
-    auto give = [&](int slot, bool marks) {
+    auto give = [&](int slot, bool marks) __attribute__((always_inline)) {
         T mk = Marked<T>::mark();
-        asm volatile("" : "+v"(mk));
+        if constexpr (RB > 2) asm volatile("" : "+v"(mk));
+        const int row0 = row_now();
         if (no_ring) {
-            const bool through = t.gi0 + t.row0 < lo || t.gi0 + t.row0 + RB > hi;
+            const bool through = t.gi0 + row0 < lo || t.gi0 + row0 + RB > hi;
             const Column col = column(false);
 #pragma unroll
             for (int c = 0; c < RB; c += kRows) {
@@ -211,7 +236,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
                     }
                     d = stage[lane_now()];
                 }
-                const int soff = slot * plane + (t.gi0 + t.row0 + c) * pitch;
+                const int soff = slot * plane + (t.gi0 + row0 + c) * pitch;
                 if (col.has) {
                     if (through) exch_store<T, kAgent>(rs, col.voff, soff, d.x, d.y);
                     else exch_store<T, 0>(rs, col.voff, soff, d.x, d.y);
@@ -222,8 +247,8 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
         const int voff = row_offset();
 #pragma unroll
         for (int rr = 0; rr < RB; ++rr) {
-            const int gi = t.gi0 + t.row0 + rr;
-            if (!gives(rr)) continue;
+            const int gi = t.gi0 + row0 + rr;
+            if (!gives(row0, rr)) continue;
             const T x0 = marks ? mk : t.v[0][rr], x1 = marks ? mk : t.v[1][rr];
             if (gi < lo || gi >= hi) exch_store<T, kAgent>(rs, voff, slot * plane + gi * pitch, x0, x1);
             else exch_store<T, 0>(rs, voff, slot * plane + gi * pitch, x0, x1);
@@ -232,8 +257,88 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
 
     bool dead = gave_up(r);  // a batch's kernel goes on to other tiles after a wave has given up
     const u64* dec = r.dec + (size_t)tile * 8;
+    // Thick tiles (H <= RB): halo rows are the first H of wave 0 and the last H of wave NW - 1; every
+    // wave takes the columns of its owned rows by chunks.  What is under way then needs registers for
+    // H rows, and not for all RB beside the values they replace.
+    auto take_thick = [&](int slot, int decided) __attribute__((always_inline)) -> u64 {
+        u64 word = 0;
+        struct {
+            T x, y;
+        } got[RB / kRows], row[H];
+        const bool edge = t.wv == 0 || t.wv == NW - 1;
+        for (int spins = 0;; ++spins) {
+            bool ok = true;
+            if (decided) word = agent_load(dec);
+            if (slot >= 0) {
+                const Column col = column(true);
+                const int m = lane_now() / kPairs;
+                const int first = t.gi0 + t.row0;
+                if (edge && inside) {
+                    const int voff = row_offset();
+                    const int at = first + (t.wv == 0 ? 0 : RB - H);
+#pragma unroll
+                    for (int j = 0; j < H; ++j)
+                        if (at + j >= 0 && at + j < t.nr) exch_load<T>(rs, voff, slot * plane + (at + j) * pitch, row[j].x, row[j].y);
+                }
+#pragma unroll
+                for (int c = 0; c < RB / kRows; ++c)
+                    if (col.has && own_row(t.row0, c * kRows + m)) exch_load<T>(rs, col.voff, slot * plane + (first + c * kRows) * pitch, got[c].x, got[c].y);
+                if (edge && inside) {
+                    const int at = t.gi0 + t.row0 + (t.wv == 0 ? 0 : RB - H);
+#pragma unroll
+                    for (int j = 0; j < H; ++j)
+                        if (at + j >= 0 && at + j < t.nr) ok = ok && Marked<T>::ready(row[j].x) && Marked<T>::ready(row[j].y);
+                }
+#pragma unroll
+                for (int c = 0; c < RB / kRows; ++c)
+                    if (col.has && own_row(t.row0, c * kRows + m)) ok = ok && Marked<T>::ready(got[c].x) && Marked<T>::ready(got[c].y);
+            }
+            if (decided) ok = ok && (int)(word >> 32) >= decided;
+            if (__all(ok) || dead) break;
+            if (spins >= r.spins) {
+                dead = true;
+                report_abort(r);
+            }
+        }
+        if (slot >= 0) {
+            const int row0 = row_now();
+            const int first = t.gi0 + row0;
+#pragma unroll
+            for (int rr = 0; rr < RB; ++rr) {
+                const bool in = inside && first + rr >= 0 && first + rr < t.nr;
+                if (rr < H) {
+                    const bool top = in && t.wv == 0;
+                    t.v[0][rr] = top ? row[rr < H ? rr : 0].x : t.v[0][rr];
+                    t.v[1][rr] = top ? row[rr < H ? rr : 0].y : t.v[1][rr];
+                }
+                if (rr >= RB - H) {
+                    const bool bottom = in && t.wv == NW - 1;
+                    t.v[0][rr] = bottom ? row[rr >= RB - H ? rr - (RB - H) : 0].x : t.v[0][rr];
+                    t.v[1][rr] = bottom ? row[rr >= RB - H ? rr - (RB - H) : 0].y : t.v[1][rr];
+                }
+            }
+            const int m = lane_now();
+            const int j = m < S ? m : m - 64 + kPairs;
+#pragma unroll
+            for (int c = 0; c < RB / kRows; ++c) {
+                stage[m] = Pair2{got[c].x, got[c].y};
+                if (inside && !owncol && j >= 0) {
+#pragma unroll
+                    for (int rr = 0; rr < kRows; ++rr) {
+                        if (!own_row(row0, c * kRows + rr)) continue;
+                        const Pair2 d = stage[rr * kPairs + j];
+                        t.v[0][c * kRows + rr] = d.x;
+                        t.v[1][c * kRows + rr] = d.y;
+                    }
+                }
+            }
+        }
+        const unsigned hi32 = __builtin_amdgcn_readfirstlane((unsigned)(word >> 32));
+        const unsigned lo32 = __builtin_amdgcn_readfirstlane((unsigned)word);
+        return ((u64)hi32 << 32) | lo32;
+    };
     // the halo cells of plane `slot` (slot < 0: none) and a decision on `decided` epochs (0: none)
-    auto take = [&](int slot, int decided) -> u64 {
+    auto take_thin = [&](int slot, int decided) __attribute__((always_inline)) -> u64 {
         u64 word = 0;
         struct {
             T x, y;
@@ -255,10 +360,10 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
             } else if (slot >= 0) {
 #pragma unroll
                 for (int rr = 0; rr < RB; ++rr)
-                    if (takes(rr)) exch_load<T>(rs, voff, slot * plane + (t.gi0 + t.row0 + rr) * pitch, t.v[0][rr], t.v[1][rr]);
+                    if (takes(t.row0, rr)) exch_load<T>(rs, voff, slot * plane + (t.gi0 + t.row0 + rr) * pitch, t.v[0][rr], t.v[1][rr]);
 #pragma unroll
                 for (int rr = 0; rr < RB; ++rr)
-                    if (takes(rr)) ok = ok && Marked<T>::ready(t.v[0][rr]) && Marked<T>::ready(t.v[1][rr]);
+                    if (takes(t.row0, rr)) ok = ok && Marked<T>::ready(t.v[0][rr]) && Marked<T>::ready(t.v[1][rr]);
             }
             if (decided) ok = ok && (int)(word >> 32) >= decided;
             if (__all(ok) || dead) break;
@@ -286,6 +391,11 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
         const unsigned hi32 = __builtin_amdgcn_readfirstlane((unsigned)(word >> 32));
         const unsigned lo32 = __builtin_amdgcn_readfirstlane((unsigned)word);
         return ((u64)hi32 << 32) | lo32;
+    };
+
+    auto take = [&](int slot, int decided) __attribute__((always_inline)) -> u64 {
+        if constexpr (kThick) return take_thick(slot, decided);
+        else return take_thin(slot, decided);
     };
 
     // the values at an epoch's start, in two turns (FP64)
@@ -612,19 +722,32 @@ __global__ void __launch_bounds__(NW * 64) sor_resident_kernel(SorArgs<T> a, Sor
     __shared__ SnapPair snap_lds[kSnapPairs<T, NW, RB>];
     __shared__ int place;
     const int band = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & (kBands - 1);  // hwreg XCC_ID
-    const int row_lo = band_start(band, a.tiles_i), row_hi = band_start(band + 1, a.tiles_i);
-    const int tiles = (row_hi - row_lo) * a.tiles_j;
+    // its tiles: those of a band of tile rows, or (runs) an eighth of all tiles, row after row
+    int first = band_start(band, r.runs ? r.ntiles : a.tiles_i), end = band_start(band + 1, r.runs ? r.ntiles : a.tiles_i);
+    int lo = band_lo<Tile>(a, first), hi = band_hi<Tile>(a, end);
+    if (!r.runs) {
+        first *= a.tiles_j;
+        end *= a.tiles_j;
+    }
     if (threadIdx.x == 0) {
         int at = atomicAdd(r.claim + band * kClaimStride, 1);
-        if (at >= tiles) at = atomicAdd(r.claim + kBands * kClaimStride, 1) == 0 ? -1 : -2;
+        if (at >= end - first) at = atomicAdd(r.claim + kBands * kClaimStride, 1) == 0 ? -1 : -2;
         place = at;
     }
     __syncthreads();
     const int at = __builtin_amdgcn_readfirstlane(place);
     if (at >= 0) {
-        const int ti = row_lo + at / a.tiles_j, tj = at % a.tiles_j;
-        sor_resident_tile<T, S, NW, RB, GS, XR, NORM>(a, r, ti, tj, row_lo, row_hi, ti * a.tiles_j + tj, sh,
-                                                        snap_lds);
+        const int tile = first + at;
+        const int ti = tile / a.tiles_j, tj = tile - ti * a.tiles_j;
+        if (r.runs) {  // TI and TJ >= H: only the 8 tiles around it read its cells
+            const int l = tj > 0, g = tj < a.tiles_j - 1;
+            const bool beside = (l && tile == first) || (g && tile + 1 == end);
+            const bool above = ti > 0 && tile - a.tiles_j - l < first;
+            const bool below = ti < a.tiles_i - 1 && tile + a.tiles_j + g >= end;
+            lo = beside ? a.nr : (above ? ti * Tile::TI + Tile::H : 0);
+            hi = below ? (ti + 1) * Tile::TI - Tile::H : a.nr;
+        }
+        sor_resident_tile<T, S, NW, RB, GS, XR, NORM>(a, r, ti, tj, lo, hi, tile, sh, snap_lds);
     } else if (at == -1) {
         sor_resident_decider<T, S, NW, RB, NORM>(a, r);
     }
@@ -666,14 +789,15 @@ __global__ void __launch_bounds__(NW * 64) sor_resident_batch_kernel(const SorAr
         const ResidentJob j = q.jobs[at];
         const SorArgs<T>& a = args[j.inst];
         const int ti = j.tile / a.tiles_j, tj = j.tile % a.tiles_j;
+        const int lo = band_lo<Tile>(a, j.row_lo), hi = band_hi<Tile>(a, j.row_hi);
         if constexpr (sizeof(T) == 8) {
             if (!a.exact_rcp) {
-                sor_resident_tile<T, S, NW, RB, GS, false, false>(a, res[j.inst], ti, tj, j.row_lo, j.row_hi, blockIdx.x, sh,
+                sor_resident_tile<T, S, NW, RB, GS, false, false>(a, res[j.inst], ti, tj, lo, hi, blockIdx.x, sh,
                                                                   snap_lds);
                 continue;
             }
         }
-        sor_resident_tile<T, S, NW, RB, GS, true, false, RB == 8>(a, res[j.inst], ti, tj, j.row_lo, j.row_hi, blockIdx.x,
+        sor_resident_tile<T, S, NW, RB, GS, true, false, RB == 8>(a, res[j.inst], ti, tj, lo, hi, blockIdx.x,
                                                                   sh, snap_lds);
     }
 }
@@ -698,20 +822,27 @@ inline int sor_resident_launch_shape(const SorArgs<T>& a, const SorResident& r, 
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
-// The shapes compiled as resident kernels.
+// The shapes compiled as resident kernels, and those for FP64 only.
 #define CNV_RESIDENT_SHAPES(X) \
     X(6, 16, 2)                \
     X(5, 16, 2)                \
     X(4, 16, 2)                \
     X(6, 12, 4)                \
     X(6, 16, 4)                \
-    X(5, 16, 4)
+    X(5, 16, 4)                \
+    X(5, 12, 8)                \
+    X(5, 12, 10)
+#define CNV_RESIDENT_SHAPES_FP64(X) \
+    X(3, 12, 14)
 
 template <typename T>
 inline int sor_resident_dispatch(const SorArgs<T>& a, const SorResident& r, TileShape sh, bool gs, hipStream_t st) {
 #define CNV_RESIDENT_CASE(s_, nw_, rb_) \
     if (sh.s == s_ && sh.nw == nw_ && sh.rb == rb_) return sor_resident_launch_shape<T, s_, nw_, rb_>(a, r, gs, st);
     CNV_RESIDENT_SHAPES(CNV_RESIDENT_CASE)
+    if constexpr (sizeof(T) == 8) {
+        CNV_RESIDENT_SHAPES_FP64(CNV_RESIDENT_CASE)
+    }
 #undef CNV_RESIDENT_CASE
     return 2;
 }

@@ -33,9 +33,11 @@ def check(n, f, beta, tol, itmax, ptype=2):
 
 
 # sides around the largest grid of each tile shape (8 x 104, 12 x 108, 16 x 112, 24 x 104, 40 x 104,
-# 44 x 108 owned points, at most 32 tiles on each of 8 XCDs), the smallest grid, and beyond the last
+# 44 x 108 owned points, at most 32 tiles on each of 8 XCDs; 76 x 108, 100 x 108, and 156 x 116,
+# at most 255 in all), the smallest grid, and beyond the last
 @pytest.mark.parametrize("n", [8, 9, 64, 97, 104, 105, 416, 417, 432, 512, 540, 541, 560, 672, 673, 728, 960, 1000,
-                               1001, 1055, 1056, 1057])
+                               1001, 1055, 1056, 1057, 1080, 1081, 1300, 1404, 1405, 1620, 1621, 1800, 2048, 2088,
+                               2089])
 def test_solves_equal_the_oracle(n):
     f = field(n)
     e = [orc.poisson(orc.make_params(n, tol=-1.0, itmax=s, ordering=orc.REDBLACK, beta_=0.9, threads=8), f)[1].e
@@ -46,7 +48,7 @@ def test_solves_equal_the_oracle(n):
     assert check(n, f, 1.0, e[1], 1000, ptype=1)[0] == cnv.OK
 
 
-@pytest.mark.parametrize("n", [300, 600, 1024])
+@pytest.mark.parametrize("n", [300, 600, 1024, 1250, 1501, 1700, 2048])
 def test_solve_that_ends_from_far_out(n):
     # a short-wave source under weak relaxation: its update falls about twofold a sweep, so when it
     # crosses the tolerance the tiles held in device memory have kept no epoch's start
@@ -60,7 +62,7 @@ def test_solve_that_ends_from_far_out(n):
 
 
 @pytest.mark.parametrize("n,launches", [(64, (5, 8, 8)), (257, (5, 8, 8)), (600, (6, 8, 8)), (900, (6, 8, 8)),
-                                        (1030, (5, 8, 8))])
+                                        (1030, (5, 8, 8)), (1211, (5, 8, 8)), (1444, (5, 8, 8))])
 def test_refined_equals_launches(n, launches):
     # the named shape is compiled for launches only; the sweeps and their order are the same
     kw = dict(precision=cnv.PREC_FP32_DC, Re=400.0, dt=1e-5, tol=1e-8, itmax=100000)
