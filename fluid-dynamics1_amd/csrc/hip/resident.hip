@@ -112,6 +112,7 @@ bool resident_plan(int n, bool fp64, int dev, TileShape base, bool named, Reside
     if (!slots) return false;
     p->units = std::min(slots, per_xcd);
     resident_layout(n, fp64, p->shape, p);
+    r.launch_s = base.s;
     return true;
 }
 
@@ -124,6 +125,7 @@ void resident_layout(int n, bool fp64, TileShape sh, ResidentPlan* p) {
     // exchange rows start on 128-byte lines: rows of two bands share none
     r.ldx = (n + 1 + 31) / 32 * 32;
     r.xplane = (long long)r.ldx * n;
+    r.launch_s = sh.s;
     r.epochs = kEpochs;
     r.spins = kSpins;
     ResidentReset& rr = p->reset;

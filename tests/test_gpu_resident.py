@@ -182,3 +182,17 @@ def test_batch_solves_that_end_from_far_out():
     ps = [cnv.default_params(n, Re=1e6, dt=1e-12, tol=e[s] * (1 + 1e-6), itmax=1000, beta=0.6) for s in ends]
     st = batch_equals_alone(ps, 1, [dict(w=f, psi=np.zeros((n, n))) for _ in ends])
     assert {s.k for s in st} == {s - 1 for s in ends}
+
+
+@pytest.mark.parametrize("n", [64, 1024])
+def test_diverging_solve_reports_as_launches(n):
+    f = 1e200 * field(n)
+    for beta in (3.5, 12.0):
+        sums = []
+        with cnv.Cavity(cnv.default_params(n, tol=-1.0, itmax=400, beta=beta)) as cav, \
+                cnv.Cavity(cnv.default_params(n, tol=-1.0, itmax=400, beta=beta, sweeps_per_launch=5, tile_waves=8,
+                                              wave_rows=8)) as launches:
+            for c in (cav, launches):
+                rc, _, k, _ = c.poisson(f)
+                sums.append((rc, k))
+        assert sums[0] == sums[1] and sums[0][0] == cnv.DIVERGED
