@@ -109,6 +109,7 @@ struct SorArgs {
     T c1, c2, c3, B, beta, omb;  // dy*dy, dx*dx, dx*dx*dy*dy, 2*(dx*dx+dy*dy), beta, 1-beta
     T rB;                // RN(1/B)
     int exact_rcp;       // 1: 1/B is exact (B a power of two), so x*rB == RN(x/B)
+    int scaled;          // FP64: c1 = c2 = B/4 a power of two, relaxation factors of ordinary size (SorTile)
     int norm;            // FP64: also sum the iterate's L1 norm (needed when rtol > 0)
     int test_mask;       // FP32: the stopping rule is tested on the last sweep of the launches
                          // with (launch & test_mask) == test_mask only (test_mask + 1, a power

@@ -137,6 +137,9 @@ inline cnv::SorArgs<T> sor_args_for(int n, int ld, double dx, double dy, double 
     a.rB = (T)(1.0 / (2 * (dx * dx + dy * dy)));
     int e2 = 0;
     const double Bd = 2 * (dx * dx + dy * dy);
+    // for the update's short form (SorTile): its proof needs these ranges
+    a.scaled = a.c1 == a.c2 && std::frexp((double)a.c1, &e2) == 0.5 && e2 >= -60 && e2 <= 1 && Bd == 4 * (double)a.c1 &&
+               std::fabs((double)a.beta) >= 0.0625 && std::fabs((double)a.beta) <= 16 && std::fabs((double)a.omb) >= 0.015625;
     a.exact_rcp = std::frexp(Bd, &e2) == 0.5 && std::isnormal(1.0 / Bd) && (1.0 / Bd) * Bd == 1.0;
     a.test_mask = 0;
     return a;

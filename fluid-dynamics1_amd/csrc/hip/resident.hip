@@ -39,6 +39,7 @@ std::atomic<int> g_units[kMaxDevices];  // CUs per XCD in use by resident solves
 //   6,12,4  1.142  1.294  1.314  1.306  1.350  -
 //   6,16,4  1.202  1.372  1.388  1.405  1.445  1.471  -
 //   5,16,4  1.272  1.479  1.475  1.493  1.486  1.526  1.459
+// and with the short update (powers of two) 0.728 at 64^2, 1.323 at 1024^2;
 // so thin tiles first: an epoch's sweeps cost as much as the rows of its tile.  As launches of
 // sor_rb.h the default shapes took 1.27 us at 64^2, 1.34 at 257^2 and 2.0 at 1024^2.  Larger grids
 // (us per FP64 sweep; "launches" the (5, 16, 4) ones, all that these grids had before; an FP32

@@ -175,6 +175,10 @@ __device__ inline T* sor_plane(const SorArgs<T>& a, int idx) {
     else return idx == 0 ? a.psi0 : (idx == 1 ? a.psi1 : a.psi2);
 }
 
+// Values at which a scaled tile's arithmetic is exact (SorTile): 0 or of a magnitude in [2^-200, 2^900).
+constexpr unsigned kSmallHi = (1023u - 200) << 21, kRangeHi = 1100u << 21;  // of the high word, its sign shifted out
+__device__ __forceinline__ bool in_range(double x) { return ((unsigned)__double2hiint(x) << 1) - kSmallHi < kRangeHi; }
+
 // A tile's LDS: the waves' first and last rows, and one column per thread of per-lane sums.
 template <typename T, int NW, int SE, bool kNorm, int FL = 0>
 struct SorShared {
@@ -182,11 +186,24 @@ struct SorShared {
     T fcl[FL > 0 ? FL * 2 * NW * 64 : 1];  // the source term of the rows that registers do not hold
     double lred[SE][NW * 64];  // this launch's per-lane L1 update sums, one row per summed sweep
     double lnrm[kNorm ? NW * 64 : 1];  // the per-lane iterate norm after the last sweep
+    int exact[NW];             // scaled tiles: the wave's values are in range
 };
 
 // A workgroup's tile in registers (NW waves of 64 lanes): wave w holds rows [w*RB, w*RB + RB) of the
 // extended tile, lane m columns 2m and 2m+1.
-// ISO (FP32): dx = dy, the two stencil coefficients of a point are one number and held once.
+// ISO: dx = dy.  FP32: the two stencil coefficients of a point are one number and held once.  FP64 (a
+// "scaled" tile): c1 = c2 = B/4 is a power of two 2^-m, so that factor can be taken out of the update:
+//   ((c1*(N+S) + c1*(E+W)) - c3*f) * beta / B  ==  (((N+S) + (E+W)) - (c3*f)/c1) * beta / 4
+// with every rounding in the same place of a number 2^m times as large: the same bits in 7
+// operations a point instead of 10, as long as no result is subnormal or infinite on either side.
+// That holds for a pass of up to 12 half-sweeps from values that are 0 or in [2^-200, 2^900) in
+// magnitude (in_range): they are multiples of 2^-252; sums of multiples are multiples; a product with
+// beta or 1-beta (1/64 to 16) is rounded to a multiple of a number at most 2^58 times smaller.  So
+// what is not 0 stays above 2^-948, 2^-m (at least 2^-61) times that is a normal number, and
+// nothing grows by more than 2^6 in a half-sweep.  Where a tile has other values (the front of a
+// first iterate, whose cells fall off twofold from one to the next), it takes the general form.
+// Resident, us per sweep: 64^2 0.765 -> 0.728, 256^2 0.860 -> 0.832, 1024^2 1.445 -> 1.323; the check is
+// about 20 of an epoch's 600 instructions.
 template <typename T, int S, int NW, int RB, bool GS, bool XR, bool NORM, bool ISO = false>
 struct SorTile {
     static constexpr int H = 2 * S;
@@ -215,6 +232,7 @@ struct SorTile {
     // reciprocal.  The thickest keep the source term of only RF rows of a wave, the others' in LDS.
     static constexpr bool kMasks = sizeof(T) == 8 && NW * RB >= 96;
     static constexpr int RF = kMasks && RB > 10 ? 5 : RB;
+    static_assert(!(ISO && kMasks), "no scaled thick tiles: both forms of their update do not fit the registers");
 
     typedef SorShared<T, NW, SE, kNorm, RB - RF> Shared;
 
@@ -226,6 +244,7 @@ struct SorTile {
     Acc w[kMasks ? 1 : RB];  // 1 for owned rows inside the domain, else 0 (wave-uniform)
     unsigned inner, owned;   // kMasks: bit r for an interior, an owned row r
     T bcoef, rBc[2];         // kMasks: the relaxation factor; rB, 0 on the domain boundary's columns
+    bool f_exact;            // scaled: this lane's source terms are in range
     T c1, c2, B, rB, omb;
     int gi0, gj0, gj, lane, wv, row0, nr, nc;
     unsigned bld;
@@ -269,6 +288,7 @@ struct SorTile {
         const T c3s = a.negate ? -a.c3 : a.c3;  // f = -src folded in: c3*(-x) == (-c3)*x exactly
         T bcol[2], cncol[2], cecol[2];
         inner = owned = 0;
+        f_exact = true;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             rBc[q] = colin[q] ? a.rB : T(0);
@@ -298,7 +318,9 @@ struct SorTile {
                 const bool inter = rint && colin[q];
                 const T fq = q ? f.y : f.x;
                 if constexpr (sizeof(T) == 8) {
-                    const T fr = inter ? c3s * fq : T(0);
+                    // scaled: (c3*f)/c1
+                    const T fr = inter ? (ISO ? (c3s * fq) * (T(1) / a.c1) : c3s * fq) : T(0);
+                    if constexpr (ISO) f_exact = f_exact && (in_range(fr) || fr == T(0));
                     if (r < RF) fc[q][r < RF ? r : 0] = fr;
                     else sh.fcl[(r < RF ? 0 : (r - RF) * 2 + q) * NW * 64 + threadIdx.x] = fr;
                     if constexpr (!kMasks) be[q][r] = rint ? bcol[q] : T(0);
@@ -351,7 +373,8 @@ struct SorTile {
     // (FP32: and the update, which only the last sweep sums); kL1: sum the L1 norms at all, which
     // a wave holding no owned row skips (its sums are 0); more: another sweep follows, which needs
     // the other waves' boundary rows
-    template <bool kL1>
+    // kScaled: the short form of a scaled tile's update
+    template <bool kL1, bool kScaled = false>
     __device__ __forceinline__ void sweep(Shared& sh, const int s, const bool with_norm, const bool more) {
 #pragma clang fp contract(off)
         const int tid = threadIdx.x;
@@ -384,11 +407,18 @@ struct SorTile {
                     // divided by B, plus (1-beta)*u0; + is commutative, so E/W order is free
                     const int j2 = r < RF ? 0 : (r - RF) * 2 + q;  // compile-time
                     const bool far_f = j2 >= kNear;
-                    const T x = c1 * (up + dn) + c2 * (own + far) - (r < RF ? fc[q][r < RF ? r : 0] : sh.fcl[far_f ? at1 + (j2 - kNear) * NW * 64 : at0 + j2 * NW * 64]);
-                    const T y = (kMasks ? (in_now >> r & 1 ? bcoef : T(0)) : be[q][kMasks ? 0 : r]) * x;
-                    const T rq = kMasks ? rBc[q] : rB;
-                    const T qt = XR ? y * rq : sor_div(y, B, rq);
-                    cand = GS ? qt : qt + omb * old;
+                    if constexpr (kScaled) {
+                        const T z = be[q][kMasks ? 0 : r] * (((up + dn) + (own + far)) - fc[q][r]);
+                        cand = __fma_rn(z, T(0.25), omb * old);
+                    } else {
+                        const T x = c1 * (up + dn) + c2 * (own + far) -
+                                    (r < RF ? (ISO ? c1 : T(1)) * fc[q][r < RF ? r : 0]
+                                            : sh.fcl[far_f ? at1 + (j2 - kNear) * NW * 64 : at0 + j2 * NW * 64]);
+                        const T y = (kMasks ? (in_now >> r & 1 ? bcoef : T(0)) : be[q][kMasks ? 0 : r]) * x;
+                        const T rq = kMasks ? rBc[q] : rB;
+                        const T qt = XR ? y * rq : sor_div(y, B, rq);
+                        cand = GS ? qt : qt + omb * old;
+                    }
                     if constexpr (!kMasks) v[q][r] = cand;
                     if constexpr (kL1) {
                         const T wr = kMasks ? (own_now >> r & 1 ? T(1) : T(0)) : w[kMasks ? 0 : r];
@@ -422,8 +452,29 @@ struct SorTile {
         if (kNorm && with_norm)
             sh.lnrm[tid] = (double)((ownc[0] ? nrm[0] : Acc(0)) + (ownc[1] ? nrm[1] : Acc(0)));
     }
+    // scaled tiles, before begin() and after it: whether the short form gives the same bits, the same
+    // for every wave of the workgroup (they read one another's rows)
+    __device__ __forceinline__ void check(Shared& sh) const {
+        bool ok = f_exact;
+#pragma unroll
+        for (int r = 0; r < RB; ++r)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) ok = ok && in_range(v[q][r]);
+        if (!__all(ok)) {  // some are 0: in boundary tiles, and in a first iterate
+            ok = f_exact;
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) ok = ok && (in_range(v[q][r]) || v[q][r] == T(0));
+        }
+        const bool all = __all(ok);
+        if (lane == 0) sh.exact[wv] = all;
+    }
+    __device__ __forceinline__ bool checked(const Shared& sh) const { return __all(sh.exact[lane < NW ? lane : 0] != 0); }
     // s_run sweeps of a launch or epoch, with the L1 sums its stopping test needs (tested)
     __device__ __forceinline__ void sweeps(Shared& sh, const int s_run, const bool tested, const bool owns) {
+        constexpr bool kShort = ISO && sizeof(T) == 8;
+        const bool general = kShort && !checked(sh);
         // the common full pass, unrolled: the values stay in their registers from sweep to sweep (a
         // rolled loop makes the compiler rotate them through copies at every iteration); not for the
         // FP64 shapes whose unrolled pass no longer fits the register budget of their wave count.
@@ -432,7 +483,7 @@ struct SorTile {
         // The waves that hold only halo rows (a quarter of them at 1024^2) run it without the FP64
         // L1 sums, two of the point update's 14 instructions.
         constexpr bool kUnroll = sizeof(T) == 4 || (S * RB <= 40 && NW != 12 && !(kNorm && S * RB > 20));
-        if (kUnroll && s_run == S) {
+        if (kUnroll && s_run == S && !general) {
             // FP32: an untested launch skips the last sweep's sums.  Small shapes get a pass of their
             // own without them (6.10 against 6.29 us per launch at 1024^2 with (5, 16, 4)); large ones
             // branch on the uniform flag in the last sweep, since a second unrolled pass of their
@@ -440,14 +491,16 @@ struct SorTile {
             constexpr bool kSplit = sizeof(T) == 4 && S * RB <= 24;
             if (kSplit && !tested) {
 #pragma unroll
-                for (int s = 0; s < S; ++s) sweep<false>(sh, s, false, s < S - 1);
+                for (int s = 0; s < S; ++s) sweep<false, kShort>(sh, s, false, s < S - 1);
             } else if (owns || sizeof(T) == 4) {
 #pragma unroll
-                for (int s = 0; s < S; ++s) sweep<true>(sh, s, s == S - 1 && (kSplit || tested), s < S - 1);
+                for (int s = 0; s < S; ++s) sweep<true, kShort>(sh, s, s == S - 1 && (kSplit || tested), s < S - 1);
             } else {
 #pragma unroll
-                for (int s = 0; s < S; ++s) sweep<false>(sh, s, s == S - 1, s < S - 1);
+                for (int s = 0; s < S; ++s) sweep<false, kShort>(sh, s, s == S - 1, s < S - 1);
             }
+        } else if (!kUnroll && kShort && !general) {
+            for (int s = 0; s < s_run; ++s) sweep<true, kShort>(sh, s, kNorm, s < s_run - 1);
         } else {
             for (int s = 0; s < s_run; ++s)
                 sweep<true>(sh, s, kLastOnly ? tested && s == s_run - 1 : kNorm, s < s_run - 1);

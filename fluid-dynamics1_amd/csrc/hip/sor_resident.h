@@ -444,6 +444,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
         const bool tested = r.stop == 0 && (sizeof(T) == 8 || ((r.launch0 + e) & a.test_mask) == a.test_mask);
         if (kSnapLds || near) keep(e & 1);
         if (!kSnap && tested_prev) t.store(a, dst);  // FP32: what a decision on the last epoch would end with
+        if constexpr (ISO && sizeof(T) == 8) t.check(sh);
         t.begin(sh);
         t.sweeps(sh, s_run, tested, owns);
         k += s_run;
@@ -719,7 +720,7 @@ __device__ __forceinline__ void sor_resident_wave_decider(const SorArgs<T>& a, c
     if (lane == 0) d.end(a.ctl, r);
 }
 
-template <typename T, int S, int NW, int RB, bool GS, bool XR, bool NORM>
+template <typename T, int S, int NW, int RB, bool GS, bool XR, bool NORM, bool ISO>
 __global__ void __launch_bounds__(NW * 64) sor_resident_kernel(SorArgs<T> a, SorResident r) {
     // the next free tile of this XCD's band; the first workgroup that finds none decides
     typedef SorTile<T, S, NW, RB, GS, XR, NORM> Tile;
@@ -752,7 +753,7 @@ __global__ void __launch_bounds__(NW * 64) sor_resident_kernel(SorArgs<T> a, Sor
             lo = beside ? a.nr : (above ? ti * Tile::TI + Tile::H : 0);
             hi = below ? (ti + 1) * Tile::TI - Tile::H : a.nr;
         }
-        sor_resident_tile<T, S, NW, RB, GS, XR, NORM>(a, r, ti, tj, lo, hi, tile, sh, snap_lds);
+        sor_resident_tile<T, S, NW, RB, GS, XR, NORM, ISO>(a, r, ti, tj, lo, hi, tile, sh, snap_lds);
     } else if (at == -1) {
         sor_resident_decider<T, S, NW, RB, NORM>(a, r);
     }
@@ -812,17 +813,25 @@ inline int sor_resident_launch_shape(const SorArgs<T>& a, const SorResident& r, 
     const dim3 grid(r.blocks), block(NW * 64);
     const bool xr = sizeof(T) == 4 || a.exact_rcp;
     if constexpr (sizeof(T) == 8) {
-        if (a.norm && !gs) {
-            if (xr) hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, false, true, true>), grid, block, 0, st, a, r);
-            else hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, false, false, true>), grid, block, 0, st, a, r);
-            return hipGetLastError() == hipSuccess ? 0 : 1;
+        if (!gs) {
+            constexpr bool kScaled = NW * RB < 96;  // the short form beside the general one: not in thick tiles
+            if (kScaled && a.scaled) {
+                if (a.norm) hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, false, true, true, kScaled>), grid, block, 0, st, a, r);
+                else hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, false, true, false, kScaled>), grid, block, 0, st, a, r);
+                return hipGetLastError() == hipSuccess ? 0 : 1;
+            }
+            if (a.norm) {
+                if (xr) hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, false, true, true, false>), grid, block, 0, st, a, r);
+                else hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, false, false, true, false>), grid, block, 0, st, a, r);
+                return hipGetLastError() == hipSuccess ? 0 : 1;
+            }
         }
     }
-    if (gs && xr) hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, true, true, false>), grid, block, 0, st, a, r);
-    else if (xr) hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, false, true, false>), grid, block, 0, st, a, r);
+    if (gs && xr) hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, true, true, false, false>), grid, block, 0, st, a, r);
+    else if (xr) hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, false, true, false, false>), grid, block, 0, st, a, r);
     else if constexpr (sizeof(T) == 8) {
-        if (gs) hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, true, false, false>), grid, block, 0, st, a, r);
-        else hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, false, false, false>), grid, block, 0, st, a, r);
+        if (gs) hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, true, false, false, false>), grid, block, 0, st, a, r);
+        else hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, false, false, false, false>), grid, block, 0, st, a, r);
     }
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }

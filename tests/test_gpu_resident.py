@@ -184,6 +184,20 @@ def test_batch_solves_that_end_from_far_out():
     assert {s.k for s in st} == {s - 1 for s in ends}
 
 
+# dx = dy a power of two: the update's short form, and values for which it does not hold
+@pytest.mark.parametrize("n", [8, 64, 256, 512, 1024])
+@pytest.mark.parametrize("scale", [1.0, 1e-40, 1e-70, 1e-250, 1e-290, 1e260, 1e285])
+def test_scaled_update_equals_the_oracle(n, scale):
+    f = scale * field(n, seed=n)
+    for beta in (1.0 + 1 / 64, 1.9, 0.3, 1.001):  # the last one has a factor 1 - beta too small for it
+        check(n, f, beta, -1.0, 29)
+    f[:, n // 2:] = 0.0
+    check(n, f, 1.7, -1.0, 29)
+    spot = np.zeros((n, n))  # the front of a first iterate: subnormal numbers at its edge
+    spot[n // 3, n // 2] = scale
+    check(n, spot, 1.5, -1.0, min(n, 300))
+
+
 @pytest.mark.parametrize("n", [64, 1024])
 def test_diverging_solve_reports_as_launches(n):
     f = 1e200 * field(n)
