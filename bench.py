@@ -8,7 +8,9 @@ continuity diagnostic).  The same steps are then run in the FP32 + FP64 defect-c
 and compared with the FP64 run.
 
 Prints one JSON line.  value = cells * steps / wall time of the timed steps (HIP events on the
-solver stream), inputs resident in HBM.  roofline: the SOR kernel (the dominant one).  Its
+solver stream), inputs resident in HBM.  roofline: the SOR kernel as launches of S sweeps, the
+form a solve takes when the GPU cannot hold it (the timed steps run theirs as one resident
+kernel, whose time per sweep is ms_per_step / sweeps_per_step).  Its
 achieved bandwidth is the bytes one launch must move -- read psi and omega, write psi, once per
 launch: 24 B per cell in FP64, 12 B in FP32 (the S sweeps of a launch run from registers) --
 over its mean launch duration, measured with HIP events on the stream it runs on; frac is that

@@ -62,7 +62,8 @@ typedef struct {
                               5 or 6 with the tile shape, both chosen by grid size)          */
     int tile_waves;        /* wave64s per SOR workgroup (compiled shapes only)               */
     int wave_rows;         /* grid rows held in registers per wave (compiled shapes only)    */
-    int launches_per_poll; /* SOR launches queued between host polls of the convergence flag
+    int launches_per_poll; /* solves that run as launches (cnv_time_sor below says which):
+                              SOR launches queued between host polls of the convergence flag
                               (0: per solve from the previous solve's length, 66 per captured
                               chunk with use_graph (72 for FP32_DC: chunks hold multiples of 6,
                               12 for FP32_DC), 2 for a batch)                               */
@@ -71,7 +72,8 @@ typedef struct {
                               launches, chunks of launches_per_poll SOR launches and tail
                               chunks of 6 (12 for FP32_DC), the post-solve launches; FP32_DC also the residual
                               and correction of each outer iteration, with the sweep budget
-                              kept on the device); results identical to the eager launches   */
+                              kept on the device); results identical to the eager launches.
+                              A resident solve is one kernel launch either way               */
     double inner_beta;     /* FP32_DC: relaxation of the inner FP32 SOR solves (0 = beta)     */
     int warm_start;        /* 1 = each Poisson solve starts from the previous step's psi
                               instead of 0 (src/poisson.c:229 starts from 0): fewer sweeps,
@@ -196,7 +198,9 @@ int cnv_sub_host(int m, int n, const double *a, const double *b, double *out);
  * current f with convergence disabled and returns the mean launch duration in ms, measured with
  * HIP events on the stream the kernel runs on, after 1000 untimed launches (the steady state of
  * a solve); the timed launches are captured in a graph and replayed, as a solve's chunks are.
- * Restores nothing: call on a scratch context. */
+ * Restores nothing: call on a scratch context.  (A solve runs as such launches where it cannot run
+ * as one resident kernel: grids of more than about 2080^2 points, launch shapes named in
+ * cnv_params that are not among the resident ones, a GPU whose CUs other resident solves hold.) */
 int cnv_time_sor(cnv_ctx *ctx, int launches, double *mean_ms);
 int cnv_sweeps_per_launch(const cnv_ctx *ctx);
 /* Counter calibration: copies nbytes between two scratch device buffers with a plain copy kernel
