@@ -4,10 +4,11 @@
 // stream-ordered launches; only the Poisson solve has a data-dependent length:
 //   wall vorticity (edges of w, in place)           src/main.c:283-320
 //   transport: derivatives + explicit Euler, w -> w' (ping-pong)   src/main.c:323-344
-//   Poisson: init (psi = 0, control block reset), then SOR launches queued in chunks; each
-//            launch checks the device control block and turns into a no-op once the solve
-//            has converged, so the host only polls a pinned copy of that block between chunks
-//            and stops queueing                   src/main.c:347-363, src/poisson.c:224-285
+//   Poisson: init (psi = 0, control block reset) in the transport launch, then one resident
+//            kernel for the solve (resident.hip), with what follows it queued behind; or, where
+//            that cannot run, SOR launches queued in chunks: each checks the device control block
+//            and turns into a no-op once the solve has converged, so the host only polls a
+//            pinned copy of that block between chunks     src/main.c:347-363, src/poisson.c:224-285
 //   velocity: u = DY psi, v = -(DX psi)            src/main.c:366-383
 //   continuity max/min (optional diagnostic)       src/main.c:387-408
 #include <hip/hip_runtime.h>

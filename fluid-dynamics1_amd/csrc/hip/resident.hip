@@ -164,6 +164,7 @@ int resident_setup(cnv_ctx* c) {
 }
 
 bool resident_enter(int dev, int units) {
+    if (dev < 0 || dev >= kMaxDevices) return false;
     std::atomic<int>& used = g_units[dev];
     if (used.fetch_add(units) + units <= cus_per_xcd(dev)) return true;
     used.fetch_sub(units);
