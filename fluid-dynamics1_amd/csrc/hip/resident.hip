@@ -35,7 +35,7 @@ std::atomic<int> g_units[kMaxDevices];  // CUs per XCD in use by resident solves
 //   n       64     257    384    513    700    900    1024
 //   6,16,2  0.755  0.917  0.938  -
 //   5,16,2  0.817  0.972  1.012  1.037  -
-//   4,16,2  0.866  1.019  1.028  1.044  -
+//   4,16,2  0.866  1.019  1.028  1.044  -      (600^2 1.14, 660^2 1.22 as eighths of all tiles)
 //   6,12,4  1.142  1.294  1.314  1.306  1.350  -
 //   6,16,4  1.202  1.372  1.388  1.405  1.445  1.471  -
 //   5,16,4  1.272  1.479  1.475  1.493  1.486  1.526  1.459

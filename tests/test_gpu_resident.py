@@ -35,7 +35,7 @@ def check(n, f, beta, tol, itmax, ptype=2):
 # sides around the largest grid of each tile shape (8 x 104, 12 x 108, 16 x 112, 24 x 104, 40 x 104,
 # 44 x 108 owned points, at most 32 tiles on each of 8 XCDs; 76 x 108, 100 x 108, and 156 x 116,
 # at most 255 in all), the smallest grid, and beyond the last
-@pytest.mark.parametrize("n", [8, 9, 64, 97, 104, 105, 416, 417, 432, 512, 540, 541, 560, 672, 673, 728, 960, 1000,
+@pytest.mark.parametrize("n", [8, 9, 64, 97, 104, 105, 416, 417, 432, 512, 540, 541, 560, 672, 673, 728, 744, 745, 960, 1000,
                                1001, 1055, 1056, 1057, 1080, 1081, 1300, 1404, 1405, 1620, 1621, 1800, 2048, 2088,
                                2089])
 def test_solves_equal_the_oracle(n):
