@@ -396,7 +396,7 @@ static int poisson_fp64(cnv_ctx* c, const double* f_src, int negate, SorCtl* fin
     if (c->p.warm_start)
         LAUNCH(c, warm_start_launch(c->psi[0], planes_of(c), c->ctl + c->fin_slot, c->n, c->ld, c->stream));
     LAUNCH(c, poisson_init_launch(c->psi[0], c->ctl, c->diag, c->n, c->ld, c->p.tol, c->p.itmax, c->stream,
-                                  !c->p.warm_start, resident_reset_of(c)));
+                                  !c->p.warm_start, c->res.fp64 ? resident_reset_of(c) : ResidentReset{}));
     SorArgs<double> a = sor_args64(c, f_src, negate);
     int rc = run_sor<double>(c, a, fin);
     if (rc) return rc;

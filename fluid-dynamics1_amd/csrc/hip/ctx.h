@@ -15,6 +15,7 @@ constexpr int kSlots = 4;  // pinned copies of the control block in flight
 // How a grid's solves run resident: tile shape, launch arguments, memory (resident.hip).
 struct ResidentPlan {
     cnv::TileShape shape{5, 16, 4};
+    bool fp64 = true;          // the solves it is for: planes, marks and kept values differ
     int tiles_i = 0, tiles_j = 0;
     int units = 0;             // CUs per XCD it holds while it runs
     long long words = 0;       // 64-bit words of exchange planes, partial sums, decision words, counters
@@ -55,6 +56,7 @@ struct cnv_ctx {
     float* r32 = nullptr;
     // launch shape
     cnv::TileShape shape{5, 16, 4};
+    bool fp64 = true;          // the solves it is for: planes, marks and kept values differ
     int tiles_i = 0, tiles_j = 0;
     int launches_per_poll = 66;  // SOR launches per captured chunk (graph path), a multiple of tail_chunk
     int poll_fixed = 0;   // launches per poll as requested; 0: chosen per solve (eager path)
@@ -289,7 +291,8 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, cnv::SorArgs<T> a, bool g
 int resident_setup(cnv_ctx* c);
 // What the init kernels reset for a solve that may run resident.
 inline cnv::ResidentReset resident_reset_of(const cnv_ctx* c) { return c->res_on ? c->res.reset : cnv::ResidentReset{}; }
-// The solve as resident kernels when they can run now (*ran = false: nothing was done).
+// The solve as resident kernels when they can run now (*ran = false: nothing was done).  A refined
+// context's plan is for its inner solves; its FP64 solves (cnv_poisson_host) run as launches.
 template <typename T>
 int run_sor_resident(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* final_ctl, bool* ran, Behind* behind = nullptr);
 

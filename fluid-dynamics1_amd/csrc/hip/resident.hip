@@ -120,6 +120,7 @@ bool resident_plan(int n, bool fp64, int dev, TileShape base, bool named, Reside
 void resident_layout(int n, bool fp64, TileShape sh, ResidentPlan* p) {
     SorResident& r = p->r;
     p->shape = sh;
+    p->fp64 = fp64;
     p->tiles_i = (n + tile_rows(sh) - 1) / tile_rows(sh);
     p->tiles_j = (n + tile_cols(sh) - 1) / tile_cols(sh);
     r.ntiles = p->tiles_i * p->tiles_j;
@@ -235,7 +236,7 @@ template <typename T>
 int run_sor_resident(cnv_ctx* c, const SorArgs<T>& a, SorCtl* final_ctl, bool* ran, Behind* behind) {
     const int dev = c->p.device;
     // with other resident solves running that leave too few CUs, this one runs as launches
-    *ran = c->res_on && resident_enter(dev, c->res.units);
+    *ran = c->res_on && c->res.fp64 == (sizeof(T) == 8) && resident_enter(dev, c->res.units);
     if (!*ran) return CNV_OK;
     int resume = -1;
     const int rc = resident_chunks<T>(c, c->res, a, c->p.poisson_type == 1, c->p.itmax, c->stream, c->h_ctl, final_ctl,

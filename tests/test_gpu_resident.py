@@ -90,6 +90,26 @@ def test_noalloc_equals_context(n):
         assert (k, e) == (k2.value, e2.value) and np.array_equal(cav.get_state()["u"], psi)
 
 
+@pytest.mark.parametrize("n", [8, 65, 257, 600, 1024, 1444])
+def test_fp64_solve_of_a_refined_context(n):
+    # the context's resident memory is laid out for its FP32 inner solves
+    f = field(n)
+    kw = dict(Re=400.0, dt=1e-5, tol=1e-3, itmax=2000, beta=1.5)
+    with cnv.Cavity(cnv.default_params(n, **kw)) as cav:
+        want = cav.poisson(f)
+    with cnv.Cavity(cnv.default_params(n, precision=cnv.PREC_FP32_DC, **kw)) as cav, \
+            cnv.Cavity(cnv.default_params(n, precision=cnv.PREC_FP32_DC, **kw)) as plain:
+        for _ in range(2):  # between steps of the refined form, which it leaves as they were
+            rc, psi, k, e = cav.poisson(f)
+            assert (rc, k) == (want[0], want[2]) and abs(e - want[3]) <= 1e-12 * want[3]
+            assert np.array_equal(psi, want[1])
+            assert [(s.status, s.sweeps, s.outer) for s in cav.step(1)] == \
+                   [(s.status, s.sweeps, s.outer) for s in plain.step(1)]
+        a, b = cav.get_state(), plain.get_state()
+        for name in ("w", "psi", "u", "v"):
+            assert np.array_equal(a[name], b[name]), name
+
+
 def test_two_solves_at_once():
     n, f = 1024, field(1024)
     kw = dict(tol=1e-4, itmax=100000, beta=1.9)
