@@ -8,10 +8,14 @@
 // Exchange.  The cells go through three planes in device memory (epoch e's through plane e % 3)
 // whose cells hold a mark -- a signalling NaN, which no arithmetic result is -- until they are
 // written: a reader loads its halo cells again until none is marked, so data and "ready" travel
-// together, in one trip.  After a tile has taken epoch e+1's cells, its own cells of epoch e have
-// been read by everyone (the tiles that published e+1 had taken e before), and it marks them
-// again; the plane's next use is two epochs later, so the marks are in place before a reader can
-// look for it (the wait before a publication orders the tile's own marks before it).
+// together, in one trip.  Once all waves of a tile have taken epoch e+1's cells, the tile's own cells
+// of epoch e have been read by everyone: each tile that reads them is one whose cells it reads, and
+// that one published e+1 after all its waves had taken e.  A wave by itself knows less -- one whose
+// rows are all owned takes nothing from above and below, where its rows may be read -- so the cells
+// are marked again behind the first barrier of the next epoch's sweeps, which every wave reaches
+// after its take.  The plane is used next by the publication at the end of the epoch after that one,
+// so the marks are in place before a reader can look for it (the wait before a publication orders
+// the tile's own marks before it, and a reader takes that one before it looks for the next).
 //
 // Coherence.  The 8 XCDs have an L2 each.  Reads are agent-scope loads, which see what the XCD's own
 // L2 holds for it and what other XCDs have written through.  Tile rows are dealt to the XCDs in
@@ -436,7 +440,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     T* const dst = sor_plane(a, r.dst);
     bool tested_prev = false;
     bool near = true;  // the decision on the epoch before the last: keep this epoch's start
-    int give_to = 1, mark_in = 0;  // planes (e + 1) % 3 and e % 3
+    int give_to = 1;  // plane (e + 1) % 3
     for (int e = 0;; ++e) {
         const int budget = itmax - k;
         const int s_run = budget < S ? budget : S;
@@ -446,6 +450,8 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
         if (!kSnap && tested_prev) t.store(a, dst);  // FP32: what a decision on the last epoch would end with
         if constexpr (ISO && sizeof(T) == 8) t.check(sh);
         t.begin(sh);
+        // every wave has taken what epoch e - 1 left: what epoch e - 2 left has been read (plane (e - 1) % 3)
+        if (e > 1) give(give_to == 2 ? 0 : give_to + 1, true);
         t.sweeps(sh, s_run, tested, owns);
         k += s_run;
         if (e == 0) {  // a first iterate's wall values (kept +0 by every store) end with the first epoch
@@ -491,8 +497,6 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
             return;
         }
         if (code != RES_CONTINUE || last) break;
-        if (e > 0) give(mark_in, true);
-        mark_in = give_to;
         give_to = give_to == 2 ? 0 : give_to + 1;
         tested_prev = tested;
     }
