@@ -99,6 +99,12 @@ __device__ __forceinline__ void wait_memory() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
+// LDS that lanes of one wave hand to one another: what was written before is read after, and not overwritten sooner
+__device__ __forceinline__ void wave_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // a decision word: the number of decided epochs, whether the end is near after the last of them and
 // after the one before, what to do, sweeps to redo
 enum ResidentCode : unsigned { RES_CONTINUE = 0, RES_END = 1, RES_REDO = 2, RES_RERUN = 3 };
@@ -238,7 +244,9 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
 #pragma unroll
                         for (int rr = 0; rr < kRows; ++rr) stage[rr * kPairs + j] = Pair2{t.v[0][c + rr], t.v[1][c + rr]};
                     }
+                    wave_lds();
                     d = stage[lane_now()];
+                    wave_lds();
                 }
                 const int soff = slot * plane + (t.gi0 + row0 + c) * pitch;
                 if (col.has) {
@@ -326,6 +334,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
 #pragma unroll
             for (int c = 0; c < RB / kRows; ++c) {
                 stage[m] = Pair2{got[c].x, got[c].y};
+                wave_lds();
                 if (inside && !owncol && j >= 0) {
 #pragma unroll
                     for (int rr = 0; rr < kRows; ++rr) {
@@ -335,6 +344,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
                         t.v[1][c * kRows + rr] = d.y;
                     }
                 }
+                wave_lds();
             }
         }
         const unsigned hi32 = __builtin_amdgcn_readfirstlane((unsigned)(word >> 32));
@@ -382,6 +392,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
 #pragma unroll
             for (int c = 0; c < RB / kRows; ++c) {
                 stage[m] = Pair2{got[c].x, got[c].y};
+                wave_lds();
                 if (inside && !owncol && j >= 0) {
 #pragma unroll
                     for (int rr = 0; rr < kRows; ++rr) {
@@ -390,6 +401,7 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
                         t.v[1][c * kRows + rr] = d.y;
                     }
                 }
+                wave_lds();
             }
         }
         const unsigned hi32 = __builtin_amdgcn_readfirstlane((unsigned)(word >> 32));
