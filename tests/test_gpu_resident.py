@@ -94,7 +94,7 @@ def test_noalloc_equals_context(n):
 def test_fp64_solve_of_a_refined_context(n):
     # the context's resident memory is laid out for its FP32 inner solves
     f = field(n)
-    kw = dict(Re=400.0, dt=1e-5, tol=1e-3, itmax=2000, beta=1.5)
+    kw = dict(Re=400.0, dt=1e-5, tol=1e-3, itmax=20000)
     with cnv.Cavity(cnv.default_params(n, **kw)) as cav:
         want = cav.poisson(f)
     with cnv.Cavity(cnv.default_params(n, precision=cnv.PREC_FP32_DC, **kw)) as cav, \
