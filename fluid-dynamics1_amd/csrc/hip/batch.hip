@@ -495,7 +495,8 @@ static int run_sor_batch(cnv_batch* b, bool fp32, std::vector<SorCtl>& snaps) {
 
 // ---- resident solves of a batch ---------------------------------------------------------------
 constexpr int kPerXcd = 32;           // workgroups of one launch on each XCD, one a CU
-constexpr int kBatchSpins = 1 << 24;  // polls of a wait: a solve also waits for the ones before it
+// polls of a wait (0.25 to 1.5 us each): a solve also waits for the ones before it, which may run for seconds
+constexpr int kBatchSpins = 1 << 24;
 
 // Which tiles run where and in which order: the longest solves first, each as soon as its tiles have
 // room, in bands of whole tile rows on as few XCDs as that takes; a shorter one goes ahead where a
@@ -606,7 +607,7 @@ static int resident_batch_setup(cnv_batch* b) {
         ResidentPlan& p = b->plan[i];
         resident_bind(&p, b->d_rwords + words, b->d_rsnap, b->d_ctl + 2 * i);
         p.r.abort = p.reset.abort = b->d_rcount + kQueueCounters;
-        p.r.spins = kBatchSpins;
+        p.r.spins = resident_polls(kBatchSpins);
         words += (p.words + 15) / 16 * 16;
         rr.push_back(p.reset);
         cnv_ctx* c = b->ctx[i];

@@ -699,7 +699,7 @@ static int one_step(cnv_ctx* c, cnv_step_stats* stats) {
         rc = solve<double>(c, sor_args64(c, c->w[c->wcur], 1), c->wcur, c->k_prev, &fin, &behind);
         c->k_prev = fin.k;
         posted = behind.counts;
-        early = !posted && c->res_on;  // the diagnostic was taken before the solve's end
+        early = behind.queued && !posted;  // the diagnostic was taken before the solve's end
     }
     if (rc) return rc;
     if (!posted) {

@@ -265,6 +265,8 @@ inline int run_sor_launches(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* f
 bool resident_plan(int n, bool fp64, int dev, cnv::TileShape base, bool named, ResidentPlan* p);
 // The part of a plan that follows from the tile shape alone: tiles, memory, launch arguments.
 void resident_layout(int n, bool fp64, cnv::TileShape sh, ResidentPlan* p);
+// Polls of a wait before it is given up: dflt, or the environment's CNV_RESIDENT_POLLS.
+int resident_polls(int dflt);
 // Gives a plan its memory: words and snap as it says, the solve's slots (the abort flag after them).
 void resident_bind(ResidentPlan* p, unsigned long long* words, double* snap, cnv::SorCtl* ctl);
 // Takes a plan's share of the device for the time of a solve (false: not now).
@@ -279,6 +281,7 @@ struct Behind {
     // the slots are read back before them (they change the slots), and the host waits for this
     // event; else after them, with the diagnostic
     hipEvent_t read = nullptr;
+    bool queued = false;  // set: the launches were queued
     bool counts = false;  // set: the first kernel did end the solve, what was queued counts
 };
 // The kernels of one solve, between the two calls above, on fresh slots and reset memory.  h: four

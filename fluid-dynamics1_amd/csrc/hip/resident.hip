@@ -8,6 +8,8 @@
 // process's resident kernel -- is left to the bounded waits: the solve goes on as launches and the
 // context uses those from then on.
 #include <hip/hip_runtime.h>
+#include <limits.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
@@ -26,7 +28,9 @@ constexpr int kMaxDevices = 64;
 // of 64, the longest test cadence of FP32 inner solves.
 constexpr int kEpochs = 1984;
 
-constexpr int kSpins = 1 << 20;  // polls of a wait: about 0.1 s
+// Polls of a wait.  A poll of a tile's halo takes 0.24 us at 256^2, 0.9 at 1024^2, 1.65 at 2048^2 (FP32 0.84 to 1.5):
+// a wait is given up after 0.25 to 1.7 s.
+constexpr int kSpins = 1 << 20;
 
 std::atomic<int> g_units[kMaxDevices];  // CUs per XCD in use by resident solves
 
@@ -117,6 +121,13 @@ bool resident_plan(int n, bool fp64, int dev, TileShape base, bool named, Reside
     return true;
 }
 
+int resident_polls(int dflt) {
+    const char* s = getenv("CNV_RESIDENT_POLLS");
+    char* end = nullptr;
+    const long v = s ? strtol(s, &end, 10) : -1;
+    return s && end != s && !*end && v >= 0 && v <= INT_MAX ? (int)v : dflt;
+}
+
 void resident_layout(int n, bool fp64, TileShape sh, ResidentPlan* p) {
     SorResident& r = p->r;
     p->shape = sh;
@@ -129,7 +140,7 @@ void resident_layout(int n, bool fp64, TileShape sh, ResidentPlan* p) {
     r.xplane = (long long)r.ldx * n;
     r.launch_s = sh.s;
     r.epochs = kEpochs;
-    r.spins = kSpins;
+    r.spins = resident_polls(kSpins);
     ResidentReset& rr = p->reset;
     rr.exch = 3 * r.xplane / (fp64 ? 1 : 2);
     rr.part = 4LL * r.ntiles * kResidentRows;
@@ -191,6 +202,7 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, in
         r.wslot = r.rslot ^ 1;
         LAUNCH(c, launch_resident(a, r, p.shape, gs, st));
         const bool first = r.launch0 == 0 && r.stop == 0 && behind && behind->queue;
+        if (first) behind->queued = true;
         int rc = first && !behind->read ? behind->queue(c, behind->arg) : CNV_OK;
         if (rc) return rc;
         HIPC(c, hipMemcpyAsync(h, a.ctl, 4 * sizeof(SorCtl), hipMemcpyDeviceToHost, st));

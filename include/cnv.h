@@ -118,6 +118,12 @@ void cnv_default_params(cnv_params *p, int n);
 size_t cnv_params_size(void);
 double cnv_reference_beta(int nx, int ny);
 
+/* A solve that runs as one resident kernel needs all its workgroups on the GPU together.  The process's
+ * own solves see to that; where another process's kernels keep some of them out for too long, the solve
+ * gives up waiting, is repeated as launches (same results), and the context or batch runs its solves
+ * as launches from then on.  The environment's CNV_RESIDENT_POLLS, read when a context or batch
+ * is created and by each cnv_poisson_device_noalloc, says how many polls of a wait are too many (default
+ * 2^20, 0.25 s at 256^2 to 1.7 s at 2048^2, for a batch 2^24; 0: the first one that finds nothing). */
 int cnv_create(const cnv_params *p, cnv_ctx **out);
 void cnv_destroy(cnv_ctx *ctx);
 const char *cnv_last_error(const cnv_ctx *ctx);   /* ctx may be NULL: this thread's last error */
