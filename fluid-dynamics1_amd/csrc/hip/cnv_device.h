@@ -134,7 +134,6 @@ struct SorResident {
     int ldx, ntiles;
     int blocks;                // workgroups of a launch
     int runs;                  // an XCD's tiles are an eighth of all, row after row (0: a band of whole tile rows)
-    int launch_s;              // a solve that diverges reports the sweeps of launches of so many (as run_sor_launches)
     int epochs, launch0;       // epochs at most; index of the first one within the solve
     int stop;                  // > 0: run to exactly this many sweeps of the solve, without tests
     int spins;                 // polls of one wait before it is given up

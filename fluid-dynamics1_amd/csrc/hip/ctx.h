@@ -16,6 +16,7 @@ constexpr int kSlots = 4;  // pinned copies of the control block in flight
 struct ResidentPlan {
     cnv::TileShape shape{5, 16, 4};
     bool fp64 = true;          // the solves it is for: planes, marks and kept values differ
+    int launch_s = 0;          // sweeps of one launch, where the solve runs as launches
     int tiles_i = 0, tiles_j = 0;
     int units = 0;             // CUs per XCD it holds while it runs
     long long words = 0;       // 64-bit words of exchange planes, partial sums, decision words, counters
@@ -286,10 +287,12 @@ struct Behind {
 };
 // The kernels of one solve, between the two calls above, on fresh slots and reset memory.  h: four
 // slots of host memory.  *resume < 0: it has ended (*fin, in slot *fin_slot), else the launch index
-// to go on from as launches (a wave gave up waiting).
+// to go on from as launches: a wave gave up waiting (*gave_up), or the solve has diverged, whose end
+// -- the launch in which its update became non-finite -- the epochs of another length do not have.
 template <typename T>
 int resident_chunks(cnv_ctx* c, const ResidentPlan& p, cnv::SorArgs<T> a, bool gs, int itmax, hipStream_t st,
-                    cnv::SorCtl* h, cnv::SorCtl* fin, int* fin_slot, int* resume, Behind* behind = nullptr);
+                    cnv::SorCtl* h, cnv::SorCtl* fin, int* fin_slot, int* resume, bool* gave_up,
+                    Behind* behind = nullptr);
 // Sets up the context's resident solves where its grid and the device allow them.
 int resident_setup(cnv_ctx* c);
 // What the init kernels reset for a solve that may run resident.

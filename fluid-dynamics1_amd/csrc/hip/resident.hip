@@ -25,8 +25,9 @@ namespace {
 
 constexpr int kMaxDevices = 64;
 // epochs of one launch: at 1024^2 about 16 ms, after which other work gets its turn.  A multiple
-// of 64, the longest test cadence of FP32 inner solves.
-constexpr int kEpochs = 1984;
+// of 64, the longest test cadence of FP32 inner solves, and of 30, so that launches of 5 or 6 sweeps
+// that take over between two kernels go on in step with those from the solve's start.
+constexpr int kEpochs = 1920;
 
 // Polls of a wait.  A poll of a tile's halo takes 0.24 us at 256^2, 0.9 at 1024^2, 1.65 at 2048^2 (FP32 0.84 to 1.5):
 // a wait is given up after 0.25 to 1.7 s.
@@ -117,7 +118,7 @@ bool resident_plan(int n, bool fp64, int dev, TileShape base, bool named, Reside
     if (!slots) return false;
     p->units = std::min(slots, per_xcd);
     resident_layout(n, fp64, p->shape, p);
-    r.launch_s = base.s;
+    p->launch_s = base.s;
     return true;
 }
 
@@ -138,7 +139,7 @@ void resident_layout(int n, bool fp64, TileShape sh, ResidentPlan* p) {
     // exchange rows start on 128-byte lines: rows of two bands share none
     r.ldx = (n + 1 + 31) / 32 * 32;
     r.xplane = (long long)r.ldx * n;
-    r.launch_s = sh.s;
+    p->launch_s = sh.s;
     r.epochs = kEpochs;
     r.spins = resident_polls(kSpins);
     ResidentReset& rr = p->reset;
@@ -186,7 +187,7 @@ void resident_leave(int dev, int units) { g_units[dev].fetch_sub(units); }
 
 template <typename T>
 int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, int itmax, hipStream_t st, SorCtl* h,
-                    SorCtl* fin, int* fin_slot, int* resume, Behind* behind) {
+                    SorCtl* fin, int* fin_slot, int* resume, bool* gave_up, Behind* behind) {
     constexpr int NB = SorPlanes<T>::value;
     SorResident r = p.r;
     a.tiles_i = p.tiles_i;
@@ -196,6 +197,7 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, in
     r.src = 0;
     r.rslot = 0;
     *resume = -1;
+    *gave_up = false;
     const long long most = (long long)itmax / p.shape.s + 2LL * kEpochs;  // epochs of a whole budget
     while (r.launch0 <= most) {
         r.dst = (r.src + 1) % NB;
@@ -215,7 +217,9 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, in
         }
         int aborted = 0;
         memcpy(&aborted, h + 2, sizeof(aborted));
-        if (aborted) {
+        const SorCtl s = h[r.wslot];
+        if (aborted || (s.status == SOR_DIVERGED && p.shape.s != p.launch_s)) {
+            *gave_up = aborted;
             // both slots as the chunk found them; FP32 planes: into plane 0, where launch 0 reads
             HIPC(c, hipMemcpyAsync(a.ctl + r.wslot, a.ctl + r.rslot, sizeof(SorCtl), hipMemcpyDeviceToDevice, st));
             if (NB == 2 && r.src == 1)
@@ -223,7 +227,6 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, in
             *resume = NB == 2 ? 0 : r.src;
             return CNV_OK;
         }
-        const SorCtl s = h[r.wslot];
         if (sor_done(s.status)) {
             if (s.rb_n != kNotStored || r.stop > 0) {
                 *fin = s;
@@ -242,7 +245,7 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, in
     return cnv_fail(c, CNV_ERR_HIP, "SOR state did not terminate after %d epochs", r.launch0);
 }
 template int resident_chunks<double>(cnv_ctx*, const ResidentPlan&, SorArgs<double>, bool, int, hipStream_t, SorCtl*,
-                                     SorCtl*, int*, int*, Behind*);
+                                     SorCtl*, int*, int*, bool*, Behind*);
 
 template <typename T>
 int run_sor_resident(cnv_ctx* c, const SorArgs<T>& a, SorCtl* final_ctl, bool* ran, Behind* behind) {
@@ -251,13 +254,14 @@ int run_sor_resident(cnv_ctx* c, const SorArgs<T>& a, SorCtl* final_ctl, bool* r
     *ran = c->res_on && c->res.fp64 == (sizeof(T) == 8) && resident_enter(dev, c->res.units);
     if (!*ran) return CNV_OK;
     int resume = -1;
+    bool gave_up = false;
     const int rc = resident_chunks<T>(c, c->res, a, c->p.poisson_type == 1, c->p.itmax, c->stream, c->h_ctl, final_ctl,
-                                      &c->fin_slot, &resume, behind);
+                                      &c->fin_slot, &resume, &gave_up, behind);
     // a failed call may leave its kernel running, which holds its place until it has ended
     if (rc) (void)hipStreamSynchronize(c->stream);
     resident_leave(dev, c->res.units);
     if (rc || resume < 0) return rc;
-    c->res_on = false;
+    if (gave_up) c->res_on = false;
     return run_sor_launches<T>(c, a, final_ctl, resume);
 }
 template int run_sor_resident<double>(cnv_ctx*, const SorArgs<double>&, SorCtl*, bool*, Behind*);

@@ -526,7 +526,7 @@ struct ResidentDecider {
     // this epoch and the next (what the decisions on the epochs two and one before said)
     static constexpr bool kAlways = sizeof(T) == 4 || resident_snap_lds(NW, RB);
     bool kept = true, kept_next = true;
-    int itmax, k, status, launches, launch_s, rb_n = 0;
+    int itmax, k, status, launches, rb_n = 0;
     double tol, rtol, e_last, n_last;
     int e = 0, k_prev, sd;
     bool last, tested;
@@ -539,7 +539,6 @@ struct ResidentDecider {
         k = p->k;
         status = p->status;
         launches = p->launches;
-        launch_s = r.launch_s;
         tol = p->tol;
         rtol = p->rtol;
         e_last = p->e_last;
@@ -624,10 +623,6 @@ struct ResidentDecider {
         } else if (s_conv >= 0 || s_fold >= 0 || s_bad >= 0) {
             code = RES_END;
             status = s_conv >= 0 ? SOR_CONVERGED : (s_fold >= 0 ? SOR_FOLD : SOR_DIVERGED);
-            if (status == SOR_DIVERGED) {
-                const int n = (k_prev + s_bad + launch_s) / launch_s * launch_s;
-                k = n < itmax ? n : itmax;
-            }
         }
         if (!kAlways && code != RES_CONTINUE) {
             // the end of this epoch is the next one's start (the tile's own values, if last)

@@ -230,3 +230,20 @@ def test_diverging_solve_reports_as_launches(n):
                 rc, _, k, _ = c.poisson(f)
                 sums.append((rc, k))
         assert sums[0] == sums[1] and sums[0][0] == cnv.DIVERGED
+
+
+# sides whose resident epochs are of 6, 4, 6, 5 and 3 sweeps, where a launch has 5 or 6; the slowest overflows in the
+# second kernel of its solve
+@pytest.mark.parametrize("n,beta", [(64, 3.5), (64, 2.05), (500, 3.5), (700, 12.0), (1024, 3.5), (2048, 12.0)])
+def test_diverging_solve_ends_as_launches(n, beta):
+    f = 1e200 * field(n) if beta > 3 else field(n)
+    kw = dict(tol=-1.0, itmax=30000, beta=beta)
+    with cnv.Cavity(cnv.default_params(n, **kw)) as cav:
+        got = [cav.poisson(f), cav.poisson(f)]
+        s = cav.sweeps_per_launch
+    with cnv.Cavity(cnv.default_params(n, sweeps_per_launch=s, tile_waves=8, wave_rows=8, **kw)) as cav:
+        rc, psi, k, e = cav.poisson(f)
+    assert rc == cnv.DIVERGED and (beta > 3 or k > 1920 * 6)
+    for g in got:
+        assert (g[0], g[2]) == (rc, k)
+        assert np.array_equal(g[1], psi, equal_nan=True) and np.array_equal(g[3], e, equal_nan=True)
