@@ -452,8 +452,8 @@ int cnv_adj_create(const cnv_params* p, int checkpoint_every, double rtol_forwar
     auto setup = [&]() -> int {
         cnv_params q = *p;
         q.diagnostics = 0;
-        int rc = cnv_create(&q, &a->c);
-        if (!rc) rc = cnv_create(&q, &a->cz);
+        int rc = cnv_create_ctx(&q, &a->c, Resident::in_step);
+        if (!rc) rc = cnv_create_ctx(&q, &a->cz, Resident::in_step);
         if (rc) return afail(a, rc, "%s", cnv_last_error(nullptr));
         a->cells = a->c->cells;
         const size_t bytes = sizeof(double) * a->cells;

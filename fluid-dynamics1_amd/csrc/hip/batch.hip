@@ -967,7 +967,7 @@ int cnv_batch_create(const cnv_params* items, int count, cnv_batch** out) {
     auto setup = [&]() -> int {
         for (int i = 0; i < count; ++i) {
             cnv_ctx* c = nullptr;
-            const int rc = cnv_create_ctx(&items[i], &c, false);  // a batch runs its solves as batched launches
+            const int rc = cnv_create_ctx(&items[i], &c, Resident::none);  // a batch runs its solves as batched launches
             if (rc) return bfail(b, rc, "batch item %d: %s", i, cnv_last_error(nullptr));
             b->ctx.push_back(c);
         }

@@ -299,9 +299,9 @@ void cnv_destroy(cnv_ctx* c) {
     delete c;
 }
 
-int cnv_create(const cnv_params* p, cnv_ctx** out) { return cnv_create_ctx(p, out, true); }
+int cnv_create(const cnv_params* p, cnv_ctx** out) { return cnv_create_ctx(p, out, Resident::any); }
 
-int cnv_create_ctx(const cnv_params* p, cnv_ctx** out, bool resident) {
+int cnv_create_ctx(const cnv_params* p, cnv_ctx** out, Resident use) {
     if (!out) return cnv_fail(nullptr, CNV_ERR_ARG, "null output pointer");
     *out = nullptr;
     if (!p) return cnv_fail(nullptr, CNV_ERR_ARG, "null params");
@@ -373,7 +373,7 @@ int cnv_create_ctx(const cnv_params* p, cnv_ctx** out, bool resident) {
             HIPC(c, hipMalloc(&c->d_budget, 2 * sizeof(int)));
         }
         int rc = upload_tables(c);
-        if (!rc && resident) rc = resident_setup(c);
+        if (!rc) rc = resident_setup(c, use);
         if (rc) return rc;
         return initial_state(c);
     };

@@ -261,9 +261,13 @@ inline int run_sor_launches(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* f
 }
 
 // ---- resident solves (resident.hip) -----------------------------------------------------------
+// Which of a context's solves run resident: none, all, or those with the launches' sweeps an epoch.
+enum class Resident { none, any, in_step };
 // The plan for n x n grids on a device; base: the launches' shape, named: the caller chose it (then
-// that one or none; else an FP32 solve keeps its sweeps per launch).  false: they run as launches.
-bool resident_plan(int n, bool fp64, int dev, cnv::TileShape base, bool named, ResidentPlan* p);
+// that one or none).  in_step: epochs of the launches' sweeps, for solves that may end with the
+// last sweep of one -- FP32 solves, and FP64 ones with the relative rule, whose norm is taken
+// there.  false: they run as launches.
+bool resident_plan(int n, bool fp64, int dev, cnv::TileShape base, bool named, bool in_step, ResidentPlan* p);
 // The part of a plan that follows from the tile shape alone: tiles, memory, launch arguments.
 void resident_layout(int n, bool fp64, cnv::TileShape sh, ResidentPlan* p);
 // Polls of a wait before it is given up: dflt, or the environment's CNV_RESIDENT_POLLS.
@@ -294,7 +298,7 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, cnv::SorArgs<T> a, bool g
                     cnv::SorCtl* h, cnv::SorCtl* fin, int* fin_slot, int* resume, bool* gave_up,
                     Behind* behind = nullptr);
 // Sets up the context's resident solves where its grid and the device allow them.
-int resident_setup(cnv_ctx* c);
+int resident_setup(cnv_ctx* c, Resident use);
 // What the init kernels reset for a solve that may run resident.
 inline cnv::ResidentReset resident_reset_of(const cnv_ctx* c) { return c->res_on ? c->res.reset : cnv::ResidentReset{}; }
 // The solve as resident kernels when they can run now (*ran = false: nothing was done).  A refined
@@ -308,5 +312,5 @@ inline int run_sor(cnv_ctx* c, const cnv::SorArgs<T>& a, cnv::SorCtl* final_ctl)
     const int rc = run_sor_resident<T>(c, a, final_ctl, &ran);
     return ran ? rc : run_sor_launches<T>(c, a, final_ctl);
 }
-// cnv_create without (resident = false) the memory of resident solves, which a batch does not use.
-int cnv_create_ctx(const cnv_params* p, cnv_ctx** out, bool resident);
+// cnv_create with a say in the resident solves: a batch has its own, the adjoint's end by the relative rule.
+int cnv_create_ctx(const cnv_params* p, cnv_ctx** out, Resident use);

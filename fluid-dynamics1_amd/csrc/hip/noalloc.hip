@@ -97,7 +97,7 @@ int cnv_poisson_device_noalloc(int n, double dx, double dy, double beta, double 
     SorCtl* ctl = reinterpret_cast<SorCtl*>(base + kIterDoubles + kPartialDoubles);
     hipStream_t st = nullptr;  // the null stream
     ResidentPlan plan;
-    bool resident = resident_plan(n, true, dev, sh, false, &plan) && plan.words <= (long long)kResidentWords &&
+    bool resident = resident_plan(n, true, dev, sh, false, false, &plan) && plan.words <= (long long)kResidentWords &&
                     plan.snap <= (long long)kSnapDoubles && resident_enter(dev, plan.units);
     if (resident) {
         double* const words = base + kIterDoubles + kPartialDoubles + kCtlDoubles;

@@ -35,8 +35,8 @@ constexpr int kSpins = 1 << 20;
 
 std::atomic<int> g_units[kMaxDevices];  // CUs per XCD in use by resident solves
 
-// The shapes in order of speed; a solve takes the first whose tiles fit on the GPU together (an FP32
-// inner solve among those with the launches' sweeps, its test cadence).  us per FP64 sweep:
+// The shapes in order of speed; a solve takes the first whose tiles fit on the GPU together (FP32 inner
+// solves and the adjoint's among those with the launches' sweeps an epoch).  us per FP64 sweep:
 //   n       64     257    384    513    700    900    1024
 //   6,16,2  0.755  0.917  0.938  -
 //   5,16,2  0.817  0.972  1.012  1.037  -
@@ -98,7 +98,7 @@ int launch_resident(const SorArgs<float>& a, const SorResident& r, TileShape sh,
 
 }  // namespace
 
-bool resident_plan(int n, bool fp64, int dev, TileShape base, bool named, ResidentPlan* p) {
+bool resident_plan(int n, bool fp64, int dev, TileShape base, bool named, bool in_step, ResidentPlan* p) {
     const int per_xcd = dev < kMaxDevices ? cus_per_xcd(dev) : 0;
     if (per_xcd < 8) return false;
     *p = ResidentPlan{};
@@ -109,7 +109,7 @@ bool resident_plan(int n, bool fp64, int dev, TileShape base, bool named, Reside
         if (sor_resident_supported(base)) slots = resident_slots(n, base, per_xcd, &r);
     } else {
         for (const TileShape& sh : kShapes) {
-            if (!fp64 && sh.s != base.s) continue;
+            if (in_step && sh.s != base.s) continue;
             p->shape = sh;
             slots = resident_slots(n, sh, per_xcd, &r);
             if (slots) break;
@@ -164,10 +164,13 @@ void resident_bind(ResidentPlan* p, unsigned long long* words, double* snap, Sor
     r.abort = rr.abort;
 }
 
-int resident_setup(cnv_ctx* c) {
+int resident_setup(cnv_ctx* c, Resident use) {
     const bool named = c->p.sweeps_per_launch > 0 || c->p.tile_waves > 0 || c->p.wave_rows > 0;
     ResidentPlan p;
-    if (!resident_plan(c->n, c->p.precision == CNV_PREC_FP64, c->p.device, c->shape, named, &p)) return CNV_OK;
+    const bool fp64 = c->p.precision == CNV_PREC_FP64;
+    if (use == Resident::none ||
+        !resident_plan(c->n, fp64, c->p.device, c->shape, named, !fp64 || use == Resident::in_step, &p))
+        return CNV_OK;
     HIPC(c, hipMalloc(&c->d_res, sizeof(*c->d_res) * p.words));
     if (p.snap) HIPC(c, hipMalloc(&c->d_res_snap, sizeof(double) * p.snap));
     resident_bind(&p, c->d_res, c->d_res_snap, c->ctl);

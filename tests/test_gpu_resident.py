@@ -247,3 +247,18 @@ def test_diverging_solve_ends_as_launches(n, beta):
     for g in got:
         assert (g[0], g[2]) == (rc, k)
         assert np.array_equal(g[1], psi, equal_nan=True) and np.array_equal(g[3], e, equal_nan=True)
+
+
+@pytest.mark.parametrize("n", [64, 97, 256, 500, 700])
+def test_adjoint_equals_launches(n):
+    # its solves end with the last sweep of the epoch, or launch, in which the relative rule is met
+    w0, out = cnv.gaussian_vorticity(n, count=12, seed=4), []
+    with cnv.Cavity(cnv.default_params(n)) as cav:
+        s = cav.sweeps_per_launch
+    for shape in ({}, dict(sweeps_per_launch=s, tile_waves=8, wave_rows=8)):
+        p = cnv.default_params(n, Re=400.0, dt=0.05 / n ** 2 * 400, tol=1e-8, itmax=200000, **shape)
+        with cnv.Adjoint(p, checkpoint_every=2) as adj:
+            E = adj.forward(w0, 1.0, 5)
+            out.append((adj.backward(), E, adj.sweeps()))
+    (g, dU), E, sweeps = out[0]
+    assert (dU, E, sweeps) == (out[1][0][1],) + out[1][1:] and np.array_equal(g, out[1][0][0])
