@@ -622,18 +622,11 @@ static int behind_next(cnv_ctx* c, int src) {
 }
 
 // One solve with whatever form it takes; *behind says whether what was queued behind it counts.
-// With use_graph its end is in slot 1, where the captured launches read it.
 template <typename T>
 static int solve(cnv_ctx* c, const SorArgs<T>& a, int src, int predicted, SorCtl* fin, Behind* behind) {
     bool ran = false;
-    int rc = run_sor_resident<T>(c, a, fin, &ran, behind);
-    if (ran) {
-        if (!rc && c->p.use_graph && c->fin_slot != 1) {
-            HIPC(c, hipMemcpyAsync(c->ctl + 1, c->ctl, sizeof(SorCtl), hipMemcpyDeviceToDevice, c->stream));
-            c->fin_slot = 1;
-        }
-        return rc;
-    }
+    const int rc = run_sor_resident<T>(c, a, fin, &ran, behind);
+    if (ran) return rc;
     if (c->p.use_graph) return replay_solve(c, src, predicted, fin);
     c->k_prev = predicted;
     return run_sor_launches<T>(c, a, fin);

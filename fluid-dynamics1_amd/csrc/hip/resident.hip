@@ -258,14 +258,20 @@ int run_sor_resident(cnv_ctx* c, const SorArgs<T>& a, SorCtl* final_ctl, bool* r
     if (!*ran) return CNV_OK;
     int resume = -1;
     bool gave_up = false;
-    const int rc = resident_chunks<T>(c, c->res, a, c->p.poisson_type == 1, c->p.itmax, c->stream, c->h_ctl, final_ctl,
+    int rc = resident_chunks<T>(c, c->res, a, c->p.poisson_type == 1, c->p.itmax, c->stream, c->h_ctl, final_ctl,
                                       &c->fin_slot, &resume, &gave_up, behind);
     // a failed call may leave its kernel running, which holds its place until it has ended
     if (rc) (void)hipStreamSynchronize(c->stream);
     resident_leave(dev, c->res.units);
-    if (rc || resume < 0) return rc;
+    if (rc) return rc;
     if (gave_up) c->res_on = false;
-    return run_sor_launches<T>(c, a, final_ctl, resume);
+    if (resume >= 0 && (rc = run_sor_launches<T>(c, a, final_ctl, resume))) return rc;
+    // captured launches read a solve's end from slot 1, whichever call made it
+    if (c->p.use_graph && c->fin_slot != 1) {
+        HIPC(c, hipMemcpyAsync(c->ctl + 1, c->ctl, sizeof(SorCtl), hipMemcpyDeviceToDevice, c->stream));
+        c->fin_slot = 1;
+    }
+    return CNV_OK;
 }
 template int run_sor_resident<double>(cnv_ctx*, const SorArgs<double>&, SorCtl*, bool*, Behind*);
 template int run_sor_resident<float>(cnv_ctx*, const SorArgs<float>&, SorCtl*, bool*, Behind*);

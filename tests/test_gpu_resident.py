@@ -262,3 +262,19 @@ def test_adjoint_equals_launches(n):
             out.append((adj.backward(), E, adj.sweeps()))
     (g, dU), E, sweeps = out[0]
     assert (dU, E, sweeps) == (out[1][0][1],) + out[1][1:] and np.array_equal(g, out[1][0][0])
+
+
+def test_warm_start_after_a_solve_of_two_kernels():
+    # 12000 sweeps are more than one resident kernel runs; the next step starts from where they got to
+    n, out = 256, []
+    for graph in (0, 1):
+        p = cnv.default_params(n, Re=400.0, dt=1e-5, tol=1e-3, itmax=12000, beta=1.0, warm_start=1, use_graph=graph)
+        with cnv.Cavity(p) as cav:
+            first = cav.step(1, check=False)
+            rc, _, k, _ = cav.poisson(field(n))
+            assert (rc, k) == (cnv.NOT_CONVERGED, 11999)
+            st = first + cav.step(2, check=False)
+            out.append(([(s.status, s.k, s.e) for s in st], cav.get_state()))
+    assert out[0][0] == out[1][0]
+    for name in ("w", "psi", "u", "v"):
+        assert np.array_equal(out[0][1][name], out[1][1][name]), name
