@@ -560,8 +560,33 @@ static bool resident_schedule(cnv_batch* b, const std::vector<int>& todo, Reside
     return true;
 }
 
-// Plans and memory; res_on stays false where a cavity's solve cannot run resident.
-static int resident_batch_setup(cnv_batch* b) {
+// Tables of a size known from the start, written anew (no kernel that reads them is running).
+template <typename V>
+static int put(cnv_batch* b, V* dst, const std::vector<V>& src) {
+    if (!src.empty()) BHIP(b, hipMemcpy(dst, src.data(), sizeof(V) * src.size(), hipMemcpyHostToDevice));
+    return CNV_OK;
+}
+
+static void resident_batch_drop(cnv_batch* b) {
+    auto drop = [](auto** p) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+    };
+    drop(&b->d_rwords);
+    drop(&b->d_rsnap);
+    drop(&b->d_rcount);
+    drop(&b->d_res);
+    drop(&b->d_rreset);
+    drop(&b->d_rargs64[0]);
+    drop(&b->d_rargs64[1]);
+    drop(&b->d_rargs32);
+    drop(&b->d_jobs);
+    drop(&b->d_order);
+}
+
+// Plans and memory; res_on stays false where a cavity's solve cannot run resident, or where there is no
+// memory for that (then the batch runs as launches).
+static void resident_batch_setup(cnv_batch* b) {
     const cnv_params& p0 = b->ctx[0]->p;
     const bool named = p0.sweeps_per_launch > 0 || p0.tile_waves > 0 || p0.wave_rows > 0;
     std::vector<int> all(b->count);
@@ -587,18 +612,26 @@ static int resident_batch_setup(cnv_batch* b) {
             sh = c.shape;
         }
     }
-    if (sh.s == 0) return CNV_OK;
-    long long words = 0;
+    if (sh.s == 0) return;
+    long long words = 0, tiles = 0;
     for (int i = 0; i < b->count; ++i) {
         b->plan[i] = ResidentPlan{};
         resident_layout(b->ctx[i]->n, !b->dc, sh, &b->plan[i]);
         words += (b->plan[i].words + 15) / 16 * 16;
+        tiles += b->plan[i].r.ntiles;
     }
     const int blocks = kBands * kPerXcd;
-    BHIP(b, hipMalloc(&b->d_rwords, sizeof(*b->d_rwords) * words));
-    if (!b->dc && !resident_snap_lds(sh.nw, sh.rb))
-        BHIP(b, hipMalloc(&b->d_rsnap, sizeof(double) * 2 * (size_t)blocks * sh.nw * sh.rb * 128));
-    BHIP(b, hipMalloc(&b->d_rcount, sizeof(int) * (kQueueCounters + kClaimStride)));
+    const auto memory = [&]() -> int {
+        BHIP(b, hipMalloc(&b->d_rwords, sizeof(*b->d_rwords) * words));
+        if (!b->dc && !resident_snap_lds(sh.nw, sh.rb))
+            BHIP(b, hipMalloc(&b->d_rsnap, sizeof(double) * 2 * (size_t)blocks * sh.nw * sh.rb * 128));
+        BHIP(b, hipMalloc(&b->d_rcount, sizeof(int) * (kQueueCounters + kClaimStride)));
+        BHIP(b, hipMalloc(&b->d_jobs, sizeof(ResidentJob) * tiles));
+        BHIP(b, hipMalloc(&b->d_order, sizeof(int) * b->count));
+        BHIP(b, hipMalloc(&b->d_res, sizeof(SorResident) * b->count));
+        return CNV_OK;
+    };
+    int rc = memory();
     words = 0;
     std::vector<ResidentReset> rr;
     std::vector<SorArgs<double>> a64[2];
@@ -623,12 +656,15 @@ static int resident_batch_setup(cnv_batch* b) {
             a32.back().test_mask = inner_test_every(c->p, 1) - 1;
         }
     }
-    int rc = upload(b, &b->d_rreset, rr);
+    if (!rc) rc = upload(b, &b->d_rreset, rr);
     for (int w = 0; w < 2 && !rc && !b->dc; ++w) rc = upload(b, &b->d_rargs64[w], a64[w]);
     if (!rc && b->dc) rc = upload(b, &b->d_rargs32, a32);
     b->res_shape = sh;
     b->res_on = rc == CNV_OK;
-    return rc;
+    if (rc) {
+        (void)hipGetLastError();
+        resident_batch_drop(b);
+    }
 }
 
 // The queues of the cavities in `todo`.
@@ -645,8 +681,8 @@ static int resident_queues(cnv_batch* b, const std::vector<int>& todo) {
         all.insert(all.end(), jobs[x].begin(), jobs[x].end());
     }
     b->queues.start[kBands] = (int)all.size();
-    int rc = upload(b, &b->d_jobs, all);
-    if (!rc) rc = upload(b, &b->d_order, order);
+    int rc = put(b, b->d_jobs, all);
+    if (!rc) rc = put(b, b->d_order, order);
     b->queues.jobs = b->d_jobs;
     b->queues.order = b->d_order;
     b->queues.count = (int)order.size();
@@ -675,12 +711,11 @@ static int run_batch_resident(cnv_batch* b, bool fp32, std::vector<SorCtl>& snap
         int rc = CNV_OK;
         if (b->res_dirty) {
             rc = resident_queues(b, todo);
-            if (!rc) rc = upload(b, &b->d_res, res);
+            if (!rc) rc = put(b, b->d_res, res);
             if (rc) return rc;
             b->res_dirty = false;
         }
         snaps.resize(b->count);
-        bool again = false;
         while (true) {
             const int e = fp32 ? sor_resident_batch_launch<float>(b->d_rargs32, b->d_res, b->queues, b->res_shape,
                                                                   kBands * kPerXcd, b->gs, b->stream)
@@ -720,7 +755,7 @@ static int run_batch_resident(cnv_batch* b, bool fp32, std::vector<SorCtl>& snap
                     return bfail(b, CNV_ERR_HIP, "resident reset failed: %s", hipGetErrorString(hipGetLastError()));
             }
             if (left.empty()) break;
-            again = true;
+            b->res_dirty = true;
             todo = left;
             ResidentReset counters{};
             counters.base = reinterpret_cast<unsigned long long*>(b->d_rcount);
@@ -730,10 +765,9 @@ static int run_batch_resident(cnv_batch* b, bool fp32, std::vector<SorCtl>& snap
                 return bfail(b, CNV_ERR_HIP, "resident reset failed: %s", hipGetErrorString(hipGetLastError()));
             BHIP(b, hipStreamSynchronize(b->stream));
             rc = resident_queues(b, todo);
-            if (!rc) rc = upload(b, &b->d_res, res);
+            if (!rc) rc = put(b, b->d_res, res);
             if (rc) return rc;
         }
-        if (again) b->res_dirty = true;
         b->fin_slot = 1;
         *ran = true;
         return CNV_OK;
@@ -915,11 +949,10 @@ void cnv_batch_destroy(cnv_batch* b) {
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     for (cnv_ctx* c : b->ctx) cnv_destroy(c);
     void* dev[] = {b->d_items, b->d_ctl, b->d_diag, b->d_partial, b->d_args64[0], b->d_args64[1], b->d_args32,
-                   b->d_dc, b->d_map_edge, b->d_map_cell, b->d_map_lin, b->d_map_sor,
-                   b->d_rwords, b->d_rsnap, b->d_rcount, b->d_res, b->d_rreset, b->d_rargs64[0], b->d_rargs64[1],
-                   b->d_rargs32, b->d_jobs, b->d_order};
+                   b->d_dc, b->d_map_edge, b->d_map_cell, b->d_map_lin, b->d_map_sor};
     for (void* p : dev)
         if (p) (void)hipFree(p);
+    resident_batch_drop(b);
     if (b->h_ctl) (void)hipHostFree(b->h_ctl);
     if (b->h_diag) (void)hipHostFree(b->h_diag);
     if (b->h_dc) (void)hipHostFree(b->h_dc);
@@ -1021,7 +1054,7 @@ int cnv_batch_create(const cnv_params* items, int count, cnv_batch** out) {
         // a one-cavity default follows that cavity's size, a batch's spans its cavities
         const bool named = p0.sweeps_per_launch > 0 || p0.tile_waves > 0 || p0.wave_rows > 0;
         if (!rc) rc = build_sor(b, named ? b->ctx[0]->shape : TileShape{5, 16, 4});
-        if (!rc) rc = resident_batch_setup(b);
+        if (!rc) resident_batch_setup(b);
         if (!rc) BHIP(b, hipDeviceSynchronize());
         return rc;
     };

@@ -171,8 +171,14 @@ int resident_setup(cnv_ctx* c, Resident use) {
     if (use == Resident::none ||
         !resident_plan(c->n, fp64, c->p.device, c->shape, named, !fp64 || use == Resident::in_step, &p))
         return CNV_OK;
-    HIPC(c, hipMalloc(&c->d_res, sizeof(*c->d_res) * p.words));
-    if (p.snap) HIPC(c, hipMalloc(&c->d_res_snap, sizeof(double) * p.snap));
+    if (hipMalloc(&c->d_res, sizeof(*c->d_res) * p.words) != hipSuccess ||
+        (p.snap && hipMalloc(&c->d_res_snap, sizeof(double) * p.snap) != hipSuccess)) {
+        (void)hipGetLastError();  // no room for them: the solves run as launches
+        if (c->d_res) (void)hipFree(c->d_res);
+        c->d_res = nullptr;
+        c->d_res_snap = nullptr;
+        return CNV_OK;
+    }
     resident_bind(&p, c->d_res, c->d_res_snap, c->ctl);
     c->res = p;
     c->res_on = true;
