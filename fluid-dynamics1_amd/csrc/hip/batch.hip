@@ -366,6 +366,7 @@ static int build_maps(cnv_batch* b) {
     b->nb_edge = (int)edge.size();
     b->nb_cell = (int)cell.size();
     b->nb_lin = (int)lin.size();
+    b->res_dirty = true;  // the queues hold the live cavities too
     int rc = upload(b, &b->d_map_edge, edge);
     if (!rc) rc = upload(b, &b->d_map_cell, cell);
     if (!rc) rc = upload(b, &b->d_map_lin, lin);
@@ -787,7 +788,6 @@ static int batch_one_step(cnv_batch* b, cnv_step_stats* stats) {
         if (!rc) rc = build_sor(b, b->shape);
         if (rc) return rc;
         b->maps_dirty = false;
-        b->res_dirty = true;
     }
     int nalive = 0;
     for (int i = 0; i < cnt; ++i) nalive += b->alive[i];

@@ -278,3 +278,40 @@ def test_warm_start_after_a_solve_of_two_kernels():
     assert out[0][0] == out[1][0]
     for name in ("w", "psi", "u", "v"):
         assert np.array_equal(out[0][1][name], out[1][1][name]), name
+
+
+@pytest.mark.parametrize("precision", [cnv.PREC_FP64, cnv.PREC_FP32_DC], ids=["fp64", "refined"])
+@pytest.mark.parametrize("when", ["dropped", "back"])
+def test_autotuned_batch_follows_its_live_cavities(precision, when):
+    # the autotuner makes the workgroup maps anew after a cavity has been dropped or come back; the next
+    # step's queues have to follow
+    sides = (48, 64, 97)
+    ps = [cnv.default_params(n, Re=100.0 + 50 * i, dt=1e-4, tol=1e-6, itmax=200000, precision=precision,
+                             inner_test_every=1, beta=cnv.reference_beta(n)) for i, n in enumerate(sides)]
+    ps[1].blowup_speed = 5.0
+    good = {k: 1e-3 * field(64, seed) for seed, k in enumerate(("w", "u", "v"))}
+    out = []
+    for tune in (False, True):
+        with cnv.Batch(ps) as b:
+            b.step(4)
+            b.set_state(1, w=1e5 * field(64))
+            assert b.step(1, check=False)[0][1].status == cnv.DIVERGED
+            dropped = b.get_state(1)
+            if tune and when == "dropped":
+                b.autotune(8)
+            b.step(2, check=False)
+            now = b.get_state(1)
+            assert all(np.isfinite(now[k]).all() and np.array_equal(now[k], dropped[k]) for k in ("w", "u", "v"))
+            b.set_state(1, psi=np.zeros((64, 64)), **good)
+            if tune and when == "back":
+                b.autotune(8)
+            st = b.step(2)
+            out.append(([(s.status, s.sweeps, s.outer) for row in st for s in row],
+                        [b.get_state(i) for i in range(len(sides))], now["psi"]))
+    if precision == cnv.PREC_FP64:  # the refined form's tests follow the launches' sweeps, which the tuner may choose anew
+        assert out[0][0] == out[1][0]
+        assert all(np.array_equal(x[k], y[k]) for x, y in zip(out[0][1], out[1][1]) for k in x)
+    else:
+        assert all(np.max(np.abs(x[k] - y[k])) <= 1e-6 * np.max(np.abs(x[k])) for x, y in zip(out[0][1], out[1][1]) for k in x)
+    # (the tuner zeroes the live cavities' iterates only)
+    assert np.array_equal(out[0][2], out[1][2])
