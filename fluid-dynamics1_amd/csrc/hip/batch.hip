@@ -290,10 +290,13 @@ struct cnv_batch {
     // resident solves: plans and memory of each cavity, the queues, tables of this batch's arguments
     // with the resident shape's tiles (res_on: usable)
     bool res_on = false, res_dirty = true;  // res_dirty: the queues are to be made again
+    bool res_use = false;                   // and whether the solves in them are faster so than as launches
+    double tuned_us = 0.0;                  // a sweep of the launches in `shape`, all cavities live, as the autotuner timed it (0: not)
     std::vector<ResidentPlan> plan;
     std::vector<int> last_k;                // sweeps of each cavity's first steps, what orders the queues
     int order_steps = 0;
     TileShape res_shape{5, 16, 4};
+    double res_us = 0.0;                    // a sweep of it, on a full GPU
     unsigned long long* d_rwords = nullptr;
     double* d_rsnap = nullptr;
     int* d_rcount = nullptr;                // the queues' counters, then the abort flag
@@ -508,8 +511,10 @@ struct ResidentSchedule {
     std::vector<int> order;
     std::vector<ResidentJob> jobs[kBands];
     double length = 0.0;  // sweeps from the first solve's start to the last one's end
+    int most = 0;         // solves that run at once
+    int deciders = 0;     // deciding workgroups
 };
-static bool resident_schedule(cnv_batch* b, const std::vector<int>& todo, ResidentSchedule* sc) {
+static bool resident_schedule(cnv_batch* b, const std::vector<int>& todo, int per_xcd, ResidentSchedule* sc) {
     struct Running {
         double end;
         int rows[kBands], tiles_j;
@@ -518,7 +523,7 @@ static bool resident_schedule(cnv_batch* b, const std::vector<int>& todo, Reside
     std::stable_sort(waiting.begin(), waiting.end(), [&](int x, int y) { return b->last_k[x] > b->last_k[y]; });
     std::vector<Running> running;
     int room[kBands];
-    for (int& r : room) r = kPerXcd - 1;  // an XCD's workgroups less a deciding one
+    for (int& r : room) r = kPerXcd - per_xcd;  // an XCD's workgroups less its deciding ones
     double now = 0.0;
     while (!waiting.empty()) {
         for (size_t w = 0; w < waiting.size();) {
@@ -546,6 +551,7 @@ static bool resident_schedule(cnv_batch* b, const std::vector<int>& todo, Reside
                 lo = hi;
             }
             running.push_back(r);
+            sc->most = std::max(sc->most, (int)running.size());
             sc->order.push_back(i);
             waiting.erase(waiting.begin() + w);
         }
@@ -558,7 +564,54 @@ static bool resident_schedule(cnv_batch* b, const std::vector<int>& todo, Reside
         running.erase(next);
     }
     for (const Running& r : running) sc->length = std::max(sc->length, r.end);
+    // a deciding wave for each of the solves that run at once; later ones take the earlier ones' waves
+    sc->deciders = std::min(per_xcd * kBands, ((int)sc->order.size() + 15) / 16);
     return true;
+}
+// With a place for one deciding workgroup of 16 waves on each XCD, or for two where more than 128 solves run
+// at once (up to 240 of one tile).
+static bool resident_schedule(cnv_batch* b, const std::vector<int>& todo, ResidentSchedule* sc) {
+    for (int per_xcd = 1; per_xcd <= 2; ++per_xcd) {
+        *sc = ResidentSchedule{};
+        if (!resident_schedule(b, todo, per_xcd, sc)) return false;
+        if (sc->most <= 16 * per_xcd * kBands) break;
+    }
+    return true;
+}
+
+// us of one launch of (5, 16, 4) tiles whose workgroups are `rounds` times the 256 CUs.  FP64 workgroups
+// fill a CU, and a launch takes as many rounds of them as it has to (measured 10.8 at 0.6, 19.9 at
+// 1.04, 31.6 at 2.4, 51.4 at 4.75, 101 at 9.5, 170 at 15.25); two FP32 workgroups share one.
+static double launch_us(double rounds, bool fp32) {
+    if (!fp32) return 10.7 * std::max(1.0, std::ceil(rounds - 0.02));
+    static const double at[][2] = {{0, 7.3}, {1, 7.5}, {1, 9.6}, {2, 10.4}, {2, 12.8}, {3, 15.5}, {4, 20.5},
+                                   {5, 25},  {7, 32.5}, {10, 42.5}, {15, 62}};
+    constexpr int last = sizeof(at) / sizeof(at[0]) - 1;
+    if (rounds >= at[last][0]) return at[last][1] * rounds / at[last][0];
+    int i = 1;
+    while (rounds > at[i][0] || at[i][0] == at[i - 1][0]) ++i;
+    return at[i - 1][1] + (at[i][1] - at[i - 1][1]) * (rounds - at[i - 1][0]) / (at[i][0] - at[i - 1][0]);
+}
+
+// us that the solves of `todo` take as launches: all advance together, and a workgroup whose solve
+// has ended costs about two fifths of one that sweeps.
+static double launches_us(cnv_batch* b, const std::vector<int>& todo) {
+    std::vector<int> by(todo);
+    std::sort(by.begin(), by.end(), [&](int x, int y) { return b->last_k[x] < b->last_k[y]; });
+    const TileShape sh{5, 16, 4};
+    double working = 0.0, ended = 0.0, us = 0.0;
+    int ti, tj, k = 0;
+    for (int i : by) working += tiles_of(b->ctx[i]->n, sh, &ti, &tj) + 1;
+    const int cus = kBands * kPerXcd;
+    const double scale = b->tuned_us > 0 ? b->tuned_us * sh.s / launch_us(working / cus, b->dc) : 1.0;
+    for (int i : by) {
+        us += (b->last_k[i] - k) * launch_us((working + 0.4 * ended) / cus, b->dc) / sh.s;
+        k = b->last_k[i];
+        const int nt = tiles_of(b->ctx[i]->n, sh, &ti, &tj) + 1;
+        working -= nt;
+        ended += nt;
+    }
+    return us * scale;
 }
 
 // Tables of a size known from the start, written anew (no kernel that reads them is running).
@@ -611,6 +664,7 @@ static void resident_batch_setup(cnv_batch* b) {
         if (sh.s == 0 || sc.length * c.us < best) {
             best = sc.length * c.us;
             sh = c.shape;
+            b->res_us = c.us;
         }
     }
     if (sh.s == 0) return;
@@ -668,27 +722,55 @@ static void resident_batch_setup(cnv_batch* b) {
     }
 }
 
-// The queues of the cavities in `todo`.
-static int resident_queues(cnv_batch* b, const std::vector<int>& todo) {
-    ResidentSchedule sc;
-    if (!resident_schedule(b, todo, &sc)) return bfail(b, CNV_ERR_ARG, "a cavity does not fit the GPU");
-    const std::vector<int>& order = sc.order;
-    const std::vector<ResidentJob>* jobs = sc.jobs;
-    // a deciding wave for each of the solves that run at once; later ones take the earlier ones' waves
-    const int deciders = std::min(kBands, ((int)order.size() + 15) / 16);
+// The queues of the cavities in `todo`, in *sc.
+static int resident_queues(cnv_batch* b, const ResidentSchedule& sc) {
     std::vector<ResidentJob> all;
     for (int x = 0; x < kBands; ++x) {
         b->queues.start[x] = (int)all.size();
-        all.insert(all.end(), jobs[x].begin(), jobs[x].end());
+        all.insert(all.end(), sc.jobs[x].begin(), sc.jobs[x].end());
     }
     b->queues.start[kBands] = (int)all.size();
     int rc = put(b, b->d_jobs, all);
-    if (!rc) rc = put(b, b->d_order, order);
+    if (!rc) rc = put(b, b->d_order, sc.order);
     b->queues.jobs = b->d_jobs;
     b->queues.order = b->d_order;
-    b->queues.count = (int)order.size();
-    b->queues.deciders = deciders;
+    b->queues.count = (int)sc.order.size();
+    b->queues.deciders = sc.deciders;
     b->queues.counters = b->d_rcount;
+    return rc;
+}
+
+static bool resident_used(const cnv_batch* b) { return b->res_on && b->res_use; }
+
+// A solve's arguments at its start.
+static SorResident resident_start(const cnv_batch* b, int i) {
+    SorResident r = b->plan[i].r;
+    r.dst = 1;
+    r.wslot = 1;
+    return r;
+}
+
+// Before a step: the queues of the live cavities, and whether they are to be used.  Resident solves keep the
+// GPU full while cavities of different lengths end one by one; launches fill it better where all are
+// alike and their tiles just miss a round of workgroups.  Both forms' times are worked out from the
+// expected lengths; of 300 uniform and mixed batches, sides 48 to 800, the faster form is taken in all
+// but one, and without this rule 40 were slower than as launches (32 cavities of 256^2, refined: 2.45
+// against 1.95 ms a step; 8 of 800^2, FP64: 30.6 against 25.6).
+static int resident_prepare(cnv_batch* b) {
+    if (!b->res_on || !b->res_dirty) return CNV_OK;
+    std::vector<int> live;
+    for (int i = 0; i < b->count; ++i)
+        if (b->alive[i]) live.push_back(i);
+    ResidentSchedule sc;
+    b->res_use = resident_schedule(b, live, &sc) && sc.length * b->res_us <= launches_us(b, live);
+    int rc = CNV_OK;
+    if (b->res_use) {
+        std::vector<SorResident> res(b->count);
+        for (int i = 0; i < b->count; ++i) res[i] = resident_start(b, i);
+        rc = resident_queues(b, sc);
+        if (!rc) rc = put(b, b->d_res, res);
+    }
+    b->res_dirty = rc != CNV_OK;
     return rc;
 }
 
@@ -697,25 +779,14 @@ static int resident_queues(cnv_batch* b, const std::vector<int>& todo) {
 // slot 1, snaps); else they are as before, and the init kernel is to be repeated if *spoilt.
 static int run_batch_resident(cnv_batch* b, bool fp32, std::vector<SorCtl>& snaps, bool* ran, bool* spoilt) {
     *ran = *spoilt = false;
-    if (!b->res_on || !resident_enter(b->device, kPerXcd)) return CNV_OK;
+    if (!resident_used(b) || !resident_enter(b->device, kPerXcd)) return CNV_OK;
     const size_t per = (size_t)2 * b->count;
     auto body = [&]() -> int {
         std::vector<int> todo;
         for (int i = 0; i < b->count; ++i)
             if (b->alive[i]) todo.push_back(i);
         std::vector<SorResident> res(b->count);
-        for (int i = 0; i < b->count; ++i) {
-            res[i] = b->plan[i].r;
-            res[i].dst = 1;
-            res[i].wslot = 1;
-        }
-        int rc = CNV_OK;
-        if (b->res_dirty) {
-            rc = resident_queues(b, todo);
-            if (!rc) rc = put(b, b->d_res, res);
-            if (rc) return rc;
-            b->res_dirty = false;
-        }
+        for (int i = 0; i < b->count; ++i) res[i] = resident_start(b, i);
         snaps.resize(b->count);
         while (true) {
             const int e = fp32 ? sor_resident_batch_launch<float>(b->d_rargs32, b->d_res, b->queues, b->res_shape,
@@ -765,7 +836,9 @@ static int run_batch_resident(cnv_batch* b, bool fp32, std::vector<SorCtl>& snap
             if (resident_reset_launch(counters, b->stream))
                 return bfail(b, CNV_ERR_HIP, "resident reset failed: %s", hipGetErrorString(hipGetLastError()));
             BHIP(b, hipStreamSynchronize(b->stream));
-            rc = resident_queues(b, todo);
+            ResidentSchedule sc;
+            if (!resident_schedule(b, todo, &sc)) return bfail(b, CNV_ERR_ARG, "a cavity does not fit the GPU");
+            int rc = resident_queues(b, sc);
             if (!rc) rc = put(b, b->d_res, res);
             if (rc) return rc;
         }
@@ -813,11 +886,12 @@ static int batch_one_step(cnv_batch* b, cnv_step_stats* stats) {
         if (b->alive[i]) b->ctx[i]->wcur = b->wcur;
     const auto init = [&]() -> int {
         hipLaunchKernelGGL(batch_poisson_init_kernel, dim3(b->nb_lin), dim3(kBlock), 0, b->stream, b->d_items,
-                           b->d_map_lin, !b->dc && b->res_on ? b->d_rreset : nullptr, b->d_rcount);
+                           b->d_map_lin, !b->dc && resident_used(b) ? b->d_rreset : nullptr, b->d_rcount);
         BLAUNCH(b);
         return CNV_OK;
     };
-    int rci = init();
+    int rci = b->dc ? CNV_OK : resident_prepare(b);
+    if (!rci) rci = init();
     if (rci) return rci;
 
     std::vector<SorCtl> fin(cnt), snaps;
@@ -849,11 +923,12 @@ static int batch_one_step(cnv_batch* b, cnv_step_stats* stats) {
             BLAUNCH(b);
             const auto inner_init = [&]() -> int {
                 hipLaunchKernelGGL(batch_dc_inner_init_kernel, dim3(b->nb_lin), dim3(kBlock), 0, b->stream, b->d_items,
-                                   b->d_map_lin, b->d_dc, b->rtol, b->res_on ? b->d_rreset : nullptr, b->d_rcount);
+                                   b->d_map_lin, b->d_dc, b->rtol, resident_used(b) ? b->d_rreset : nullptr, b->d_rcount);
                 BLAUNCH(b);
                 return CNV_OK;
             };
-            int rc = inner_init();
+            int rc = resident_prepare(b);
+            if (!rc) rc = inner_init();
             if (rc) return rc;
             b->k_prev = o < cnv_batch::kDcPred ? b->k_dc[o] : 0;  // this outer iteration's last length
             rc = run_batch_resident(b, true, snaps, &ran, &spoilt);
@@ -1225,6 +1300,8 @@ int cnv_batch_autotune(cnv_batch* b, int launches, int* sweeps_per_launch, int* 
         BHIP(b, hipStreamSynchronize(b->stream));
     }
     b->k_prev = 0;
+    if (!rc_tune) b->tuned_us = 1e3 * best_ms;
+    b->res_dirty = true;  // launches of the tuned shape may now be the faster form
     if (rc_tune) return bfail(b, rc_tune, "%s", msg);
     if (rc) return rc;
     if (sweeps_per_launch) *sweeps_per_launch = best.s;

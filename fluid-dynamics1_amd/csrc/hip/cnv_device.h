@@ -155,7 +155,7 @@ struct ResidentQueues {
     int start[kBands + 1];     // XCD x takes jobs [start[x], start[x + 1])
     const int* order;
     int count;                 // solves
-    int deciders;              // workgroups that decide, on XCDs 0 .. deciders - 1
+    int deciders;              // workgroups that decide: the first on each of XCDs 0, 1, ..., then the second
     int* counters;             // [2 * kBands + 1][kClaimStride], zeroed: workgroups arrived and jobs taken on
                                // each XCD, solves taken by the deciders
 };

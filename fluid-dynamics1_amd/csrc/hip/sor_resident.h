@@ -787,7 +787,7 @@ __global__ void __launch_bounds__(NW * 64) sor_resident_batch_kernel(const SorAr
     const int xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & (kBands - 1);  // hwreg XCC_ID
     if (threadIdx.x == 0) place = atomicAdd(q.counters + xcc * kClaimStride, 1);
     __syncthreads();
-    if (__builtin_amdgcn_readfirstlane(place) == 0 && xcc < q.deciders) {
+    if (__builtin_amdgcn_readfirstlane(place) * kBands + xcc < q.deciders) {
         while (true) {
             int c = 0;
             if ((threadIdx.x & 63) == 0) c = atomicAdd(q.counters + 2 * kBands * kClaimStride, 1);
@@ -881,7 +881,7 @@ struct ResidentBatchShape {
 template <typename T>
 inline const std::vector<ResidentBatchShape>& resident_batch_shapes() {
     static const std::vector<ResidentBatchShape> f64 = {{{5, 16, 2}, 1.10}, {{5, 16, 4}, 1.56}};
-    static const std::vector<ResidentBatchShape> f32 = {{{5, 16, 2}, 0.76}, {{5, 16, 4}, 1.08}, {{5, 16, 8}, 1.70}};
+    static const std::vector<ResidentBatchShape> f32 = {{{5, 16, 2}, 0.86}, {{5, 16, 4}, 1.17}, {{5, 16, 8}, 1.73}};
     return sizeof(T) == 8 ? f64 : f32;
 }
 

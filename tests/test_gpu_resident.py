@@ -315,3 +315,20 @@ def test_autotuned_batch_follows_its_live_cavities(precision, when):
         assert all(np.max(np.abs(x[k] - y[k])) <= 1e-6 * np.max(np.abs(x[k])) for x, y in zip(out[0][1], out[1][1]) for k in x)
     # (the tuner zeroes the live cavities' iterates only)
     assert np.array_equal(out[0][2], out[1][2])
+
+
+@pytest.mark.parametrize("precision", [cnv.PREC_FP64, cnv.PREC_FP32_DC], ids=["fp64", "refined"])
+def test_batch_of_more_solves_at_once_than_128(precision):
+    # one tile each (two deciding workgroups on an XCD): those of unlike lengths take one another's places
+    ps = [cnv.default_params(n, Re=100.0 + i, dt=1e-5, tol=1e-6 * 10.0 ** -(i % 4), itmax=200000, precision=precision,
+                             inner_test_every=1, beta=cnv.reference_beta(n)) for i, n in enumerate([40, 33, 44] * 84)]
+    assert all(s.status == cnv.OK for s in batch_equals_alone(ps, 2))
+
+
+# uniform batches on either side of the line between resident solves and launches
+@pytest.mark.parametrize("n,count,precision", [(256, 27, cnv.PREC_FP32_DC), (256, 28, cnv.PREC_FP32_DC),
+                                               (800, 3, cnv.PREC_FP64), (800, 8, cnv.PREC_FP64)])
+def test_batch_of_like_cavities(n, count, precision):
+    ps = [cnv.default_params(n, Re=400.0, dt=1e-5, tol=1e-5, itmax=200000, precision=precision, inner_test_every=1,
+                             beta=cnv.reference_beta(n), u=[0.0, 0.0, 0.0, 1.0 + 0.01 * i]) for i in range(count)]
+    assert all(s.status == cnv.OK for s in batch_equals_alone(ps, 3))
