@@ -109,7 +109,8 @@ struct SorArgs {
     T c1, c2, c3, B, beta, omb;  // dy*dy, dx*dx, dx*dx*dy*dy, 2*(dx*dx+dy*dy), beta, 1-beta
     T rB;                // RN(1/B)
     int exact_rcp;       // 1: 1/B is exact (B a power of two), so x*rB == RN(x/B)
-    int scaled;          // FP64: c1 = c2 = B/4 a power of two, relaxation factors of ordinary size (SorTile)
+    int scaled;          // FP64: c1 = c2 = B/4 a power of two, relaxation factors of ordinary size (SorTile); 2: and
+                         // the general form all the same
     int norm;            // FP64: also sum the iterate's L1 norm (needed when rtol > 0)
     int test_mask;       // FP32: the stopping rule is tested on the last sweep of the launches
                          // with (launch & test_mask) == test_mask only (test_mask + 1, a power
@@ -130,7 +131,8 @@ struct SorResident {
     double* part;              // [4][ntiles][kResidentRows], marked
     unsigned long long* dec;   // [ntiles][8]: each tile's decision word
     double* snap;              // FP64 tiles too large for LDS: two copies of each extended tile
-    int* abort;                // set by a wave that gave up waiting
+    int* abort;                // set by a wave that gave up waiting; [1]: by a tile of a scaled grid whose source
+                               // term is out of the short form's range
     int ldx, ntiles;
     int blocks;                // workgroups of a launch
     int runs;                  // an XCD's tiles are an eighth of all, row after row (0: a band of whole tile rows)
@@ -161,7 +163,7 @@ struct ResidentQueues {
 };
 constexpr int kQueueCounters = (2 * kBands + 1) * kClaimStride;
 // What one reset writes before a resident launch: marks over the exchange planes, marks over the
-// partial sums, zeros over the decision words and tile counters (in that order from base) and in the abort flag.
+// partial sums, zeros over the decision words and tile counters (in that order from base) and in the two flags at abort.
 struct ResidentReset {
     unsigned long long* base;    // nullptr: nothing to reset
     long long exch, part, zero;  // 64-bit words

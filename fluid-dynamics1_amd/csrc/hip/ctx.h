@@ -80,6 +80,7 @@ struct cnv_ctx {
     hipGraphExec_t g_post = nullptr;
     // resident solves (sor_resident.h, resident.hip): usable, their plan and memory
     bool res_on = false;
+    bool src_out = false;      // the last one's source was out of the short update's range (SorTile)
     ResidentPlan res;
     unsigned long long* d_res = nullptr;
     double* d_res_snap = nullptr;
@@ -293,10 +294,12 @@ struct Behind {
 // slots of host memory.  *resume < 0: it has ended (*fin, in slot *fin_slot), else the launch index
 // to go on from as launches: a wave gave up waiting (*gave_up), or the solve has diverged, whose end
 // -- the launch in which its update became non-finite -- the epochs of another length do not have.
+// *src_out: on a scaled grid, whether the general update is to be used (only speed depends on it); set to
+// what the solve's source calls for.
 template <typename T>
 int resident_chunks(cnv_ctx* c, const ResidentPlan& p, cnv::SorArgs<T> a, bool gs, int itmax, hipStream_t st,
                     cnv::SorCtl* h, cnv::SorCtl* fin, int* fin_slot, int* resume, bool* gave_up,
-                    Behind* behind = nullptr);
+                    bool* src_out, Behind* behind = nullptr);
 // Sets up the context's resident solves where its grid and the device allow them.
 int resident_setup(cnv_ctx* c, Resident use);
 // What the init kernels reset for a solve that may run resident.

@@ -116,8 +116,8 @@ int cnv_poisson_device_noalloc(int n, double dx, double dy, double beta, double 
     if (resident) {
         SorCtl h[4];
         int slot = 0;
-        bool gave_up = false;
-        rc = resident_chunks<double>(nullptr, plan, a, gs, itmax, st, h, &fin, &slot, &resume, &gave_up);
+        bool gave_up = false, src_out = false;
+        rc = resident_chunks<double>(nullptr, plan, a, gs, itmax, st, h, &fin, &slot, &resume, &gave_up, &src_out);
         if (rc) (void)hipStreamSynchronize(st);
         resident_leave(dev, plan.units);
         if (rc) return rc;

@@ -196,7 +196,7 @@ void resident_leave(int dev, int units) { g_units[dev].fetch_sub(units); }
 
 template <typename T>
 int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, int itmax, hipStream_t st, SorCtl* h,
-                    SorCtl* fin, int* fin_slot, int* resume, bool* gave_up, Behind* behind) {
+                    SorCtl* fin, int* fin_slot, int* resume, bool* gave_up, bool* src_out, Behind* behind) {
     constexpr int NB = SorPlanes<T>::value;
     SorResident r = p.r;
     a.tiles_i = p.tiles_i;
@@ -211,6 +211,7 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, in
     while (r.launch0 <= most) {
         r.dst = (r.src + 1) % NB;
         r.wslot = r.rslot ^ 1;
+        if (a.scaled) a.scaled = *src_out ? 2 : 1;
         LAUNCH(c, launch_resident(a, r, p.shape, gs, st));
         const bool first = r.launch0 == 0 && r.stop == 0 && behind && behind->queue;
         if (first) behind->queued = true;
@@ -224,8 +225,10 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, in
         } else {
             HIPC(c, hipStreamSynchronize(st));
         }
-        int aborted = 0;
-        memcpy(&aborted, h + 2, sizeof(aborted));
+        int flags[2];
+        memcpy(flags, h + 2, sizeof(flags));
+        const bool aborted = flags[0];
+        *src_out = flags[1];
         const SorCtl s = h[r.wslot];
         if (aborted || (s.status == SOR_DIVERGED && p.shape.s != p.launch_s)) {
             *gave_up = aborted;
@@ -254,7 +257,7 @@ int resident_chunks(cnv_ctx* c, const ResidentPlan& p, SorArgs<T> a, bool gs, in
     return cnv_fail(c, CNV_ERR_HIP, "SOR state did not terminate after %d epochs", r.launch0);
 }
 template int resident_chunks<double>(cnv_ctx*, const ResidentPlan&, SorArgs<double>, bool, int, hipStream_t, SorCtl*,
-                                     SorCtl*, int*, int*, bool*, Behind*);
+                                     SorCtl*, int*, int*, bool*, bool*, Behind*);
 
 template <typename T>
 int run_sor_resident(cnv_ctx* c, const SorArgs<T>& a, SorCtl* final_ctl, bool* ran, Behind* behind) {
@@ -265,7 +268,7 @@ int run_sor_resident(cnv_ctx* c, const SorArgs<T>& a, SorCtl* final_ctl, bool* r
     int resume = -1;
     bool gave_up = false;
     int rc = resident_chunks<T>(c, c->res, a, c->p.poisson_type == 1, c->p.itmax, c->stream, c->h_ctl, final_ctl,
-                                      &c->fin_slot, &resume, &gave_up, behind);
+                                      &c->fin_slot, &resume, &gave_up, &c->src_out, behind);
     // a failed call may leave its kernel running, which holds its place until it has ended
     if (rc) (void)hipStreamSynchronize(c->stream);
     resident_leave(dev, c->res.units);

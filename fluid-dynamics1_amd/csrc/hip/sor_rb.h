@@ -201,7 +201,11 @@ struct SorShared {
 // beta or 1-beta (1/64 to 16) is rounded to a multiple of a number at most 2^58 times smaller.  So
 // what is not 0 stays above 2^-948, 2^-m (at least 2^-61) times that is a normal number, and
 // nothing grows by more than 2^6 in a half-sweep.  Where a tile has other values (the front of a
-// first iterate, whose cells fall off twofold from one to the next), it takes the general form.
+// first iterate, whose cells fall off twofold from one to the next), it takes the general form, in a
+// rolled loop.  A tile whose source term has other values (the front of a vorticity that spreads from
+// the walls: below 2^-200 from step 16 on at 1024^2) would do so at every epoch, and all tiles wait for
+// it: it says so, and the solve's next kernels, and the next solve's, are the general form's, until
+// the source is in range again (1024^2 from rest, steps from 17 on: 1.62 -> 1.45 us a sweep).
 // Resident, us per sweep: 64^2 0.765 -> 0.728, 256^2 0.860 -> 0.832, 1024^2 1.445 -> 1.323; the check is
 // about 20 of an epoch's 600 instructions.
 template <typename T, int S, int NW, int RB, bool GS, bool XR, bool NORM, bool ISO = false>
@@ -244,7 +248,7 @@ struct SorTile {
     Acc w[kMasks ? 1 : RB];  // 1 for owned rows inside the domain, else 0 (wave-uniform)
     unsigned inner, owned;   // kMasks: bit r for an interior, an owned row r
     T bcoef, rBc[2];         // kMasks: the relaxation factor; rB, 0 on the domain boundary's columns
-    bool f_exact;            // scaled: this lane's source terms are in range
+    bool f_exact;            // this lane's source terms are in range (a scaled tile's, or one that could be)
     T c1, c2, B, rB, omb;
     int gi0, gj0, gj, lane, wv, row0, nr, nc;
     unsigned bld;
@@ -321,6 +325,10 @@ struct SorTile {
                     // scaled: (c3*f)/c1
                     const T fr = inter ? (ISO ? (c3s * fq) * (T(1) / a.c1) : c3s * fq) : T(0);
                     if constexpr (ISO) f_exact = f_exact && (in_range(fr) || fr == T(0));
+                    else if (XR && !GS && !kMasks && a.scaled == 2) {
+                        const T fs = fr * (T(1) / a.c1);
+                        f_exact = f_exact && (in_range(fs) || fs == T(0));
+                    }
                     if (r < RF) fc[q][r < RF ? r : 0] = fr;
                     else sh.fcl[(r < RF ? 0 : (r - RF) * 2 + q) * NW * 64 + threadIdx.x] = fr;
                     if constexpr (!kMasks) be[q][r] = rint ? bcol[q] : T(0);

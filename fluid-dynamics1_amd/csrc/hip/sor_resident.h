@@ -89,6 +89,9 @@ __device__ __forceinline__ void agent_store(u64* p, u64 x) { __hip_atomic_store(
 __device__ __forceinline__ void report_abort(const SorResident& r) {
     __hip_atomic_store(r.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void report_source(const SorResident& r) {
+    __hip_atomic_store(r.abort + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ bool gave_up(const SorResident& r) {
     return __builtin_amdgcn_readfirstlane(__hip_atomic_load(r.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
 }
@@ -156,6 +159,9 @@ __device__ __forceinline__ void sor_resident_tile(const SorArgs<T>& a, const Sor
     t.place(a, ti, tj);
     t.load(a, sor_plane(a, r.src), sh);
     t.fix_odd_edge();
+    if constexpr (sizeof(T) == 8) {
+        if (!__all(t.f_exact)) report_source(r);
+    }
     const bool owns = t.owns_rows();
 
     // pairs of this lane's columns, and which rows' pairs it takes from or gives to other tiles
@@ -826,7 +832,7 @@ inline int sor_resident_launch_shape(const SorArgs<T>& a, const SorResident& r, 
     if constexpr (sizeof(T) == 8) {
         if (!gs) {
             constexpr bool kScaled = NW * RB < 96;  // the short form beside the general one: not in thick tiles
-            if (kScaled && a.scaled) {
+            if (kScaled && a.scaled == 1) {
                 if (a.norm) hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, false, true, true, kScaled>), grid, block, 0, st, a, r);
                 else hipLaunchKernelGGL((sor_resident_kernel<T, S, NW, RB, false, true, false, kScaled>), grid, block, 0, st, a, r);
                 return hipGetLastError() == hipSuccess ? 0 : 1;

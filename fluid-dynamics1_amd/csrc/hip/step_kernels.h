@@ -111,7 +111,7 @@ __device__ inline void transport_fp64_at(const double* __restrict__ w, double* _
 // ---- what a resident solve finds at its start, thread q of `threads` in the grid -------------
 __device__ inline void resident_reset_at(const ResidentReset& rr, long long q, long long threads) {
     if (!rr.base) return;
-    if (q == 0) *rr.abort = 0;
+    if (q == 0) rr.abort[0] = rr.abort[1] = 0;
     const long long total = rr.exch + rr.part + rr.zero;
     for (; q < total; q += threads) rr.base[q] = q < rr.exch ? rr.mark : (q < rr.exch + rr.part ? kMark64 : 0ull);
 }

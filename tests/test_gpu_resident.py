@@ -4,6 +4,7 @@ epoch, inside an epoch, on its last sweep, on a spent budget, and from so far ou
 nothing to go back to; the refined form's inner solves; two solves at once from two threads."""
 import ctypes as C
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -332,3 +333,36 @@ def test_batch_of_like_cavities(n, count, precision):
     ps = [cnv.default_params(n, Re=400.0, dt=1e-5, tol=1e-5, itmax=200000, precision=precision, inner_test_every=1,
                              beta=cnv.reference_beta(n), u=[0.0, 0.0, 0.0, 1.0 + 0.01 * i]) for i in range(count)]
     assert all(s.status == cnv.OK for s in batch_equals_alone(ps, 3))
+
+
+@pytest.mark.parametrize("n", [64, 256, 1024])
+def test_source_in_and_out_of_the_short_updates_range(n):
+    # one context, sources of either kind in turn, solves of one kernel and of two: the form follows the source
+    near, far = field(n), field(n, 5)
+    far[:, : n // 3] *= 1e-80
+    for itmax in (31, 11600 if n < 1000 else 43):
+        want = {i: orc.poisson(orc.make_params(n, tol=-1.0, itmax=itmax, ordering=orc.REDBLACK, beta_=1.5, threads=8), f)
+                for i, f in enumerate((near, far))}
+        with cnv.Cavity(cnv.default_params(n, tol=-1.0, itmax=itmax, beta=1.5)) as cav:
+            for i in (0, 1, 1, 0, 0, 1):
+                rc, psi, k, e = cav.poisson((near, far)[i])
+                assert rc == cnv.NOT_CONVERGED and np.array_equal(psi, want[i][0])
+                assert abs(e - want[i][1].e) <= 1e-12 * want[i][1].e
+
+
+@pytest.mark.parametrize("n,most", [(256, 1.12), (1024, 1.16)])
+def test_far_front_costs_no_more_than_the_general_update(n, most):
+    # a sweep of the general form against the short one: 1.03 at 256^2, 1.10 at 1024^2 by the kernels' own times;
+    # the general form as an epoch of the short one's kernel: 1.22 and 1.23
+    near, far = field(n), field(n)
+    far[:, : n // 3] *= 1e-80
+    dt = {0: [], 1: []}
+    with cnv.Cavity(cnv.default_params(n, tol=-1.0, itmax=9000, beta=1.5)) as cav:
+        for _ in range(6):
+            for i, f in enumerate((near, far)):
+                cav.poisson(f)
+                t = time.perf_counter()
+                cav.poisson(f)
+                dt[i].append(time.perf_counter() - t)
+    print(n, min(dt[1]) / min(dt[0]), flush=True)
+    assert min(dt[1]) <= most * min(dt[0])
