@@ -63,8 +63,6 @@ constexpr TileShape kShapes[] = {{6, 16, 2}, {5, 16, 2}, {4, 16, 2}, {6, 12, 4},
 // Workgroups per XCD of a resident solve with tiles of shape sh (0: they do not fit together).
 int resident_slots(int n, TileShape sh, int per_xcd, SorResident* r) {
     const int ti = (n + tile_rows(sh) - 1) / tile_rows(sh), tj = (n + tile_cols(sh) - 1) / tile_cols(sh);
-    // a workgroup of 16 waves (or of 8 with twice the registers each) fills a CU; two of 4 waves fit
-    const int room = sh.nw > 4 ? per_xcd : 2 * per_xcd;
     r->ntiles = ti * tj;
     // An XCD's tiles are whole tile rows where they fit so; else an eighth of all tiles, whose cells are
     // written through more often: up to 2 more neighbours' tiles are on other XCDs.
@@ -78,7 +76,7 @@ int resident_slots(int n, TileShape sh, int per_xcd, SorResident* r) {
                                           : (band_start(b + 1, ti) - band_start(b, ti)) * tj);
         r->blocks = kBands * most + (r->ntiles == kBands * most);
         const int slots = (r->blocks + kBands - 1) / kBands;
-        if (slots <= room) return slots;
+        if (slots <= per_xcd) return slots;  // a workgroup, of 12 or 16 waves, a CU
     }
     return 0;
 }
@@ -116,7 +114,7 @@ bool resident_plan(int n, bool fp64, int dev, TileShape base, bool named, bool i
         }
     }
     if (!slots) return false;
-    p->units = std::min(slots, per_xcd);
+    p->units = slots;
     resident_layout(n, fp64, p->shape, p);
     p->launch_s = base.s;
     return true;
