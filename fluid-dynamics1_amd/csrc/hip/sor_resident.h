@@ -886,7 +886,7 @@ struct ResidentBatchShape {
 };
 template <typename T>
 inline const std::vector<ResidentBatchShape>& resident_batch_shapes() {
-    static const std::vector<ResidentBatchShape> f64 = {{{5, 16, 2}, 1.10}, {{5, 16, 4}, 1.56}};
+    static const std::vector<ResidentBatchShape> f64 = {{{5, 16, 2}, 1.12}, {{5, 16, 4}, 1.60}};
     static const std::vector<ResidentBatchShape> f32 = {{{5, 16, 2}, 0.86}, {{5, 16, 4}, 1.17}, {{5, 16, 8}, 1.73}};
     return sizeof(T) == 8 ? f64 : f32;
 }
