@@ -244,7 +244,8 @@ int cnv_batch_status(const cnv_batch *b, int *status);
 /* Launch-shape autotuner: times `launches` batched SOR launches of every compiled shape on a
  * synthetic source over the whole batch, keeps the fastest per sweep and reports it.  Leaves w,
  * u, v as they were; the Poisson iterates are zeroed (every step recomputes psi from zero).  The shape is
- * that of solves that run as launches; resident solves of the batch keep theirs. */
+ * that of solves that run as launches, and its time counts when the batch chooses between those and
+ * resident solves, which keep their own. */
 int cnv_batch_autotune(cnv_batch *b, int launches, int *sweeps_per_launch, int *tile_waves,
                        int *wave_rows, double *ms_per_sweep);
 
