@@ -101,3 +101,21 @@ def test_speed_limit_is_held_against_the_end_of_the_solve(n, graph, no_polls):
         for name in NAMES:
             kw.pop(name, None)
     assert out[1][0] == out[0][0] and same_fields(out[1][1], out[0][1])
+
+
+@pytest.mark.parametrize("polls", [1, 2, 4, 8, 16])
+@pytest.mark.parametrize("precision", [cnv.PREC_FP64, cnv.PREC_FP32_DC], ids=["fp64", "refined"])
+def test_whenever_a_wait_is_too_long(precision, polls, monkeypatch):
+    # a few polls may or may not be enough, in the first kernel of a solve or a later one: solves of 12 000 sweeps and
+    # more (plain relaxation), of which a kernel runs 9600 to 11 520
+    n = 200
+    kw = dict(precision=precision, Re=400.0, dt=1e-5, tol=1e-7, itmax=200000, beta=1.0, inner_test_every=1)
+    with cnv.Cavity(cnv.default_params(n, **kw, **dict(zip(NAMES, (5, 8, 8))))) as cav:
+        want, fields = cav.step(2), cav.get_state()
+    assert want[0].sweeps > 12000
+    monkeypatch.setenv("CNV_RESIDENT_POLLS", str(polls))
+    for _ in range(3):
+        with cnv.Cavity(cnv.default_params(n, **kw)) as cav:
+            got = cav.step(2)
+            assert [(s.status, s.sweeps, s.outer) for s in got] == [(s.status, s.sweeps, s.outer) for s in want]
+            assert same_fields(cav.get_state(), fields)
